@@ -344,7 +344,7 @@ size_t batch_workspace_bytes(int fmt, const size_t* rows, size_t count, size_t t
 // once (the reference batches exactly this sharing, src/quant.cpp:1521-1554).
 int enqueue_gemm_batch(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
                        const float* X, size_t tokens, size_t cols, int act, void* ws, size_t ws_bytes, hipStream_t s,
-                       uint64_t* dispatches) {
+                       uint64_t* dispatches, bool own_ws = false) {
     if (ws_bytes < batch_workspace_bytes(fmt, rows, count, tokens, cols, act)) return ZQ_ERR_ARG;
     if (act == ZQ_ACT_INT8) {
         if (!ws) return ZQ_ERR_ARG;
@@ -368,7 +368,7 @@ int enqueue_gemm_batch(int fmt, const uint8_t* const* w, float* const* Y, const 
     for (size_t i = 0; i < count; ++i) {
         uint32_t n = 0;
         if (const int ls = launch_status(
-                zq::launch_gemm_f32(fmt, w[i], X, Y[i], ws, ws ? ws_bytes : 0, tokens, rows[i], cols, s, &n));
+                zq::launch_gemm_f32(fmt, w[i], X, Y[i], ws, ws ? ws_bytes : 0, tokens, rows[i], cols, s, &n, own_ws));
             ls != ZQ_OK)
             return ls;
         *dispatches += n;
@@ -687,7 +687,9 @@ int gemm_batch_locked(Backend& b, int fmt, const float* X, const zq_gemm_task* t
         ybytes += align_up(tokens * rows[i] * sizeof(float), 256);
         ymax = std::max(ymax, tokens * rows[i] * sizeof(float));
     }
-    const size_t wsbytes = batch_workspace_bytes(fmt, rows, count, tokens, cols, act);
+    size_t wsbytes = batch_workspace_bytes(fmt, rows, count, tokens, cols, act);
+    if (act != ZQ_ACT_INT8)
+        for (size_t i = 0; i < count; ++i) wsbytes = std::max(wsbytes, zq::gemm_f32_best_bytes(fmt, tokens, rows[i], cols));
     st = ensure_scratch(b, xbytes + ybytes + wsbytes, std::max(xbytes, ymax));
     if (st != ZQ_OK) return st;
     uint8_t* base = static_cast<uint8_t*>(b.dev_scratch);
@@ -703,7 +705,7 @@ int gemm_batch_locked(Backend& b, int fmt, const float* X, const zq_gemm_task* t
     if ((st = c.put(dx, X, tokens * cols * sizeof(float))) != ZQ_OK) return st;
     c.begin();
     uint64_t n = 0;
-    st = enqueue_gemm_batch(fmt, dw, dy, rows, count, dx, tokens, cols, act, ws, wsbytes, b.stream, &n);
+    st = enqueue_gemm_batch(fmt, dw, dy, rows, count, dx, tokens, cols, act, ws, wsbytes, b.stream, &n, true);
     if (st != ZQ_OK) {
         ++b.stats.errors;
         return st;

@@ -12,7 +12,8 @@
 //    arithmetic of gemv_q8_0_avx2_int8_prequant (kernels/avx2.cpp:562-585) and
 //    of the D3D12 int8 GEMM (shaders/q8_0_gemm_i8.hlsl:249-257).
 //
-//  * fp32 activations (all formats; the reference CPU arithmetic).  Weights
+//  * fp32 activations (all formats; the reference CPU arithmetic): the split
+//    f16 kernels of zq_gemm_split.hip where the workspace allows, else weights
 //    are dequantised exactly into LDS (the reference's dequantize values) and
 //    multiplied with v_mfma_f32_32x32x2_f32 in fp32.
 //
@@ -31,6 +32,7 @@
 // (ids congruent mod 8) walk the token tiles of one weight panel before
 // moving on, keeping that panel in the XCD's L2.
 #include "zq_device.hpp"
+#include "zq_gemm_common.hpp"
 #include "zq_internal.hpp"
 
 #include <algorithm>
@@ -86,31 +88,6 @@ __global__ __launch_bounds__(kThreads) void quantize_acts_kernel(const float* __
         w |= (uint32_t(round_half_away(q)) & 0xffu) << (8 * k);
     }
     reinterpret_cast<uint32_t*>(xq)[g] = w;
-}
-
-// ------------------------------------------------------- tile mapping ---
-#ifndef ZQ_GEMM_XCD_BLOCKS
-#define ZQ_GEMM_XCD_BLOCKS 1
-#endif
-__device__ __forceinline__ void tile_of(uint32_t tiles_m, uint32_t tiles_n, uint32_t id, uint32_t& tm, uint32_t& tn) {
-    const uint32_t total = tiles_m * tiles_n;
-    uint32_t slot = id;
-    if (ZQ_GEMM_XCD_BLOCKS && tiles_m % 4 == 0 && tiles_n % 2 == 0) {
-        // XCD x (ids congruent to x mod 8) owns a quarter of the token tiles
-        // and half of the weight panels, walking its token tiles per panel:
-        // its activation rows stay in its L2, and each weight panel is read
-        // by two XCDs.
-        const uint32_t x = id % 8u, local = id / 8u, qm = tiles_m / 4;
-        tm = (x & 3u) * qm + local % qm;
-        tn = (x >> 2) * (tiles_n / 2) + local / qm;
-        return;
-    }
-    if (total % 8u == 0) {
-        const uint32_t per_xcd = total / 8u;
-        slot = (id % 8u) * per_xcd + id / 8u;
-    }
-    tn = slot / tiles_m;
-    tm = slot % tiles_m;
 }
 
 // ------------------------------------------------------- int8 GEMM -------
@@ -347,9 +324,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_i8_kernel(const uint8_t* __r
         }
 }
 
-// Y = sum of the ksplit partial planes in split order; four outputs a thread
-// (float4) when n % 4 == 0 and both buffers are 16-byte aligned, else one.
-template <bool VEC4>
+// Y = sum of the ksplit partial planes in split order (ADD: Y += that sum,
+// one plane after the other); four outputs a thread (float4) when n % 4 == 0
+// and both buffers are 16-byte aligned, else one.
+template <bool VEC4, bool ADD>
 __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(const float* __restrict__ part, float* __restrict__ Y,
                                                                  size_t n, uint32_t ksplit) {
     const size_t i = size_t(blockIdx.x) * kThreads + threadIdx.x;
@@ -357,16 +335,16 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(const float* __
         const size_t n4 = n / 4;
         if (i >= n4) return;
         const float4* p = reinterpret_cast<const float4*>(part);
-        float4 acc = p[i];
-        for (uint32_t s = 1; s < ksplit; ++s) {
+        float4 acc = ADD ? reinterpret_cast<const float4*>(Y)[i] : p[i];
+        for (uint32_t s = ADD ? 0 : 1; s < ksplit; ++s) {
             const float4 t = p[size_t(s) * n4 + i];
             acc.x += t.x; acc.y += t.y; acc.z += t.z; acc.w += t.w;
         }
         reinterpret_cast<float4*>(Y)[i] = acc;
     } else {
         if (i >= n) return;
-        float acc = part[i];
-        for (uint32_t s = 1; s < ksplit; ++s) acc += part[size_t(s) * n + i];
+        float acc = ADD ? Y[i] : part[i];
+        for (uint32_t s = ADD ? 0 : 1; s < ksplit; ++s) acc += part[size_t(s) * n + i];
         Y[i] = acc;
     }
 }
@@ -978,330 +956,6 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(const uint8_t* __res
         }
 }
 
-// ------------------------------------------- K-quants on the f16 MFMA ---
-// The fp32-activation GEMM of the super-block formats (Q6_K, Q4_K, Q5_K)
-// with its products on v_mfma_f32_32x32x16_f16 (16x the fp32 MFMA rate) at
-// fp32-level accuracy:
-//  * each activation row is scaled by a power of two (split_rows_kernel) and
-//    carried as f16 hi + lo;
-//  * each weight is dequantised as the reference does (Q6_K d*sc*(q-32),
-//    Q4_K / Q5_K d*sc*q - dmin*m, one fp32 rounding), scaled by a power of
-//    two per weight row (so the row's largest possible value lies below
-//    2^15) and carried as h = f16(w) and l = f16(w - h);
-//  * a product is Xh*Wh + Xl*Wh + Xh*Wl, accumulated in fp32 per super-block
-//    and the super-blocks summed; the row scales come off at the end.
-// Against the reference's dequantise-then-fp32 arithmetic the difference is
-// rounding order, the 22-bit operand splits and the dropped lo*lo products
-// (all below 2^-21 of each operand).
-// A workgroup barrier that orders LDS only: unlike __syncthreads it does not
-// wait for the wave's outstanding global loads (a prefetch stays in flight).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-#ifndef ZQ_KQ_HKS
-#define ZQ_KQ_HKS 32
-#endif
-
-// One workgroup per row.
-__global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __restrict__ X, _Float16* __restrict__ xh,
-                                                              _Float16* __restrict__ xl, float* __restrict__ inv,
-                                                              uint32_t K) {
-    __shared__ float red[kThreads / 64];
-    const float4* r = reinterpret_cast<const float4*>(X + size_t(blockIdx.x) * K);
-    const uint32_t K4 = K / 4;
-    float m = 0.0f;
-    for (uint32_t i = threadIdx.x; i < K4; i += kThreads) {
-        const float4 v = r[i];
-        m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = red[0];
-#pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, red[w]);
-    const int e = split_exp(m);
-    const float f = pow2f(e);
-    if (threadIdx.x == 0) inv[blockIdx.x] = pow2f(-e);
-    h4_t* oh = reinterpret_cast<h4_t*>(xh + size_t(blockIdx.x) * K);
-    h4_t* ol = reinterpret_cast<h4_t*>(xl + size_t(blockIdx.x) * K);
-    for (uint32_t i = threadIdx.x; i < K4; i += kThreads) {
-        const float4 v = r[i];
-        h4_t h, l;
-        split_h(v.x * f, h, l, 0);
-        split_h(v.y * f, h, l, 1);
-        split_h(v.z * f, h, l, 2);
-        split_h(v.w * f, h, l, 3);
-        oh[i] = h;
-        ol[i] = l;
-    }
-}
-
-// Split K as in gemm_f32_kernel; stages_per_split is a multiple of the
-// stages of a super-block.  HKS: K elements per stage (32 or 64).
-template <int FMT, int HKS>
-__global__ __launch_bounds__(kThreads, 2) void gemm_kq_h_kernel(const uint8_t* __restrict__ W,
-                                                                 const _Float16* __restrict__ XH,
-                                                                 const _Float16* __restrict__ XL,
-                                                                 const float* __restrict__ xinv, float* __restrict__ Y,
-                                                                 uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_m,
-                                                                 uint32_t tiles_n, uint32_t ksplit,
-                                                                 uint32_t stages_per_split) {
-    static_assert(FMT == kQ6_K || FMT == kQ4_K || FMT == kQ5_K, "super-block formats");
-    static_assert(HKS == 32 || HKS == 64, "stage depth");
-    constexpr bool Q6 = FMT == kQ6_K;
-    constexpr uint32_t BB = FMT == kQ6_K ? 210 : (FMT == kQ5_K ? 176 : 144);
-    constexpr int HR = HKS + 8;      // halves per LDS row (pad: 16 B)
-    constexpr int EPT = HKS / 2;     // elements per loader thread per stage
-    constexpr int XU = EPT / 8;      // 16-byte units of activations per thread, each of hi and lo
-    constexpr int QWN = EPT / 4;     // words of codes per thread (one byte per element)
-    __shared__ __align__(16) _Float16 Ah[BM * HR];
-    __shared__ __align__(16) _Float16 Al[BM * HR];
-    __shared__ __align__(16) _Float16 Bh[BN * HR];
-    __shared__ __align__(16) _Float16 Bl[BN * HR];
-    __shared__ float binv[BN];
-    const uint32_t total_tiles = tiles_m * tiles_n;
-    const uint32_t split = blockIdx.x / total_tiles;
-    uint32_t tm, tn;
-    tile_of(tiles_m, tiles_n, blockIdx.x % total_tiles, tm, tn);
-    const uint32_t m0 = tm * BM, n0 = tn * BN;
-    const uint32_t k_begin = split * stages_per_split * HKS;
-    const uint32_t k_end = min(K, k_begin + stages_per_split * HKS);
-    float* Yout = Y + (ksplit > 1 ? size_t(split) * M * N : 0);
-    const size_t rb = row_bytes_dev(FMT, K);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int l32 = lane & 31, lh = lane >> 5;
-    const uint32_t ld_row = tid >> 1, ld_half = tid & 1;  // loader: row, half of the stage
-    const _Float16* ah_src = XH + size_t(min(m0 + ld_row, M - 1)) * K + ld_half * EPT;
-    const _Float16* al_src = XL + size_t(min(m0 + ld_row, M - 1)) * K + ld_half * EPT;
-    const uint8_t* b_src = W + size_t(min(n0 + ld_row, N - 1)) * rb;
-
-    // The loader row's scale 2^e: its dequantised weights over this split's
-    // super-blocks, times 2^e, lie below 2^15 in magnitude (a bound from d,
-    // dmin and the largest code and scale), so each is h + l in f16 with
-    // normal h.  The two threads of a row scan alternate super-blocks.
-    float wscale;
-    {
-        float bound = 0.0f;
-        for (uint32_t sb = k_begin / 256 + ld_half; sb < (k_end + 255) / 256; sb += 2) {
-            const uint8_t* p = b_src + size_t(sb) * BB;
-            if constexpr (Q6) {
-                bound = fmaxf(bound, fabsf(half_bits_to_float(*reinterpret_cast<const uint16_t*>(p + 208))) * 4096.0f);
-            } else {
-                const uint32_t dd = *reinterpret_cast<const uint32_t*>(p);
-                const float dmax = FMT == kQ5_K ? 1953.0f : 945.0f;  // 63 x 31, 63 x 15
-                bound = fmaxf(bound, fmaf(fabsf(half_bits_to_float(dd & 0xffffu)), dmax,
-                                          fabsf(half_bits_to_float(dd >> 16)) * 63.0f));
-            }
-        }
-        bound = fmaxf(bound, __shfl_xor(bound, 1));
-        const int e = split_exp(bound);
-        wscale = pow2f(e);
-        if (ld_half == 0) binv[ld_row] = pow2f(-e);
-    }
-
-    // part: the current super-block's products; acc: the sum of the
-    // super-blocks' (a two-level sum, so rounding grows with the number of
-    // super-blocks rather than of MFMA steps)
-    v16f acc[2][2], part[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = part[i][j][v] = 0.0f;
-
-    // Raw stage data of this thread: EPT activations (hi, lo), the words of
-    // its EPT weight codes, their group scales and the super-block's d (and
-    // dmin).  The next stage's are loaded while the current one is converted
-    // and multiplied.  The thread's codes are one 32-element line of the
-    // super-block (a Q6_K quarter of a half, a Q4_K / Q5_K group): for HKS =
-    // 32 its half, for HKS = 64 line ld_half of the stage's two.
-    struct Raw {
-        u32x4_attn_t xa[XU], xb[XU];
-        uint32_t qw[QWN], hw[Q6 || FMT == kQ5_K ? QWN : 1];
-        uint32_t sc;   // Q6_K: the int8 scales of the thread's 16-element groups; else the 12 scale bytes' words
-        uint32_t sc1, sc2;
-        uint32_t dd;   // d (| dmin << 16)
-    };
-    auto line_of = [&](uint32_t k0, uint32_t& line, uint32_t& ls) {
-        const uint32_t in_sb = k0 & 255u;
-        line = (in_sb >> 5) + (HKS == 64 ? ld_half : 0u);
-        ls = HKS == 64 ? 0u : ld_half * 16u;
-    };
-    auto load_raw = [&](uint32_t k0, Raw& r) {
-#pragma unroll
-        for (int u = 0; u < XU; ++u) {
-            r.xa[u] = *reinterpret_cast<const u32x4_attn_t*>(ah_src + k0 + 8 * u);
-            r.xb[u] = *reinterpret_cast<const u32x4_attn_t*>(al_src + k0 + 8 * u);
-        }
-        const uint8_t* p = b_src + size_t(k0 >> 8) * BB;
-        uint32_t line, ls;
-        line_of(k0, line, ls);
-        if constexpr (Q6) {
-            const uint32_t h = line >> 2, q4 = line & 3u;
-            const uint8_t* lo = p + h * 64 + (q4 & 1u) * 32 + ls;
-            const uint8_t* hi = p + 128 + h * 32 + ls;
-#pragma unroll
-            for (int i = 0; i < QWN; ++i) {
-                r.qw[i] = load_u32_a2(lo + 4 * i);
-                r.hw[i] = load_u32_a2(hi + 4 * i);
-            }
-            const uint8_t* s = p + 192 + h * 8 + q4 * 2 + (ls >> 4);
-            r.sc = HKS == 64 ? uint32_t(*reinterpret_cast<const uint16_t*>(s)) : uint32_t(*s);
-            r.dd = *reinterpret_cast<const uint16_t*>(p + 208);
-            r.sc1 = r.sc2 = 0;
-        } else {
-            const uint32_t* qs =
-                reinterpret_cast<const uint32_t*>(p + (FMT == kQ5_K ? 48 : 16) + (line >> 1) * 32 + ls);
-#pragma unroll
-            for (int i = 0; i < QWN; ++i) r.qw[i] = qs[i];
-            if constexpr (FMT == kQ5_K) {
-                const uint32_t* qh = reinterpret_cast<const uint32_t*>(p + 16 + ls);
-#pragma unroll
-                for (int i = 0; i < QWN; ++i) r.hw[i] = qh[i];
-            }
-            const uint32_t* w = reinterpret_cast<const uint32_t*>(p);
-            r.dd = w[0];
-            r.sc = w[1];
-            r.sc1 = w[2];
-            r.sc2 = w[3];
-        }
-    };
-    // one stage from `cur`, prefetching the next into `nxt` (two named
-    // records used alternately: no copy between them)
-    auto stage = [&](uint32_t k0, Raw& cur, Raw& nxt) {
-        // unconditional (the last stage reloads itself), so the wait for the
-        // current stage's data counts the prefetch statically
-        load_raw(min(k0 + HKS, k_end - HKS), nxt);
-        u32x4_attn_t xa[XU], xb[XU];
-#pragma unroll
-        for (int u = 0; u < XU; ++u) {
-            xa[u] = cur.xa[u];
-            xb[u] = cur.xb[u];
-        }
-        h8_t wh[EPT / 8], wl[EPT / 8];
-        {
-            uint32_t line, ls;
-            line_of(k0, line, ls);
-            // per 16-element group: value = a * code - b (exact in fp32), times 2^e
-            float a[EPT / 16], b[EPT / 16];
-            if constexpr (Q6) {
-                const float ds = half_bits_to_float(cur.dd & 0xffffu) * wscale;
-#pragma unroll
-                for (int g = 0; g < EPT / 16; ++g) {
-                    a[g] = ds * float(int(int8_t(uint8_t(cur.sc >> (8 * g)))));
-                    b[g] = 32.0f * a[g];
-                }
-            } else {
-                // scale / min of group `line` (src/quant.cpp:133-141) from the
-                // words of scale bytes 0-3, 4-7, 8-11
-                const uint32_t sh = 8 * (line & 3u);
-                const uint32_t sa = cur.sc >> sh, sbb = cur.sc1 >> sh, scc = cur.sc2 >> sh;
-                const uint32_t sc = line < 4 ? sa & 63u : (scc & 15u) | ((sa >> 2) & 0x30u);
-                const uint32_t mn = line < 4 ? sbb & 63u : ((scc >> 4) & 15u) | ((sbb >> 2) & 0x30u);
-                const float d = half_bits_to_float(cur.dd & 0xffffu) * wscale;
-                const float dm = half_bits_to_float(cur.dd >> 16) * wscale;
-#pragma unroll
-                for (int g = 0; g < EPT / 16; ++g) {
-                    a[g] = d * float(sc);
-                    b[g] = dm * float(mn);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < QWN; ++i) {
-                const uint32_t qw = cur.qw[i];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    uint32_t q;
-                    if constexpr (Q6) {
-                        const uint32_t q4 = line & 3u;
-                        uint32_t l = (qw >> (8 * k)) & 0xffu;
-                        if (q4 >= 2) l >>= 4;
-                        const uint32_t hb = ((cur.hw[i] >> (8 * k)) >> (2 * q4)) & 3u;
-                        q = (l & 15u) | (hb << 4);
-                    } else {
-                        q = (qw >> (8 * k + 4 * (line & 1u))) & 15u;
-                        if constexpr (FMT == kQ5_K) q |= ((cur.hw[i] >> (8 * k + line)) & 1u) << 4;
-                    }
-                    const int e = 4 * i + k;
-                    const float v = fmaf(a[e / 16], float(q), -b[e / 16]);
-                    split_h(v, wh[e / 8], wl[e / 8], e % 8);
-                }
-            }
-        }
-        lds_barrier();  // the previous stage's readers are done (the prefetch stays in flight)
-#pragma unroll
-        for (int u = 0; u < XU; ++u) {
-            *reinterpret_cast<u32x4_attn_t*>(Ah + ld_row * HR + ld_half * EPT + 8 * u) = xa[u];
-            *reinterpret_cast<u32x4_attn_t*>(Al + ld_row * HR + ld_half * EPT + 8 * u) = xb[u];
-            *reinterpret_cast<h8_t*>(Bh + ld_row * HR + ld_half * EPT + 8 * u) = wh[u];
-            *reinterpret_cast<h8_t*>(Bl + ld_row * HR + ld_half * EPT + 8 * u) = wl[u];
-        }
-        lds_barrier();
-#pragma unroll
-        for (int ks = 0; ks < HKS / 16; ++ks) {
-            h8_t ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int r = (wm * 64 + i * 32 + l32) * HR + ks * 16 + 8 * lh;
-                ah[i] = *reinterpret_cast<const h8_t*>(Ah + r);
-                al[i] = *reinterpret_cast<const h8_t*>(Al + r);
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int r = (wn * 64 + j * 32 + l32) * HR + ks * 16 + 8 * lh;
-                bh[j] = *reinterpret_cast<const h8_t*>(Bh + r);
-                bl[j] = *reinterpret_cast<const h8_t*>(Bl + r);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], part[i][j], 0, 0, 0);
-                    part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], part[i][j], 0, 0, 0);
-                    part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], part[i][j], 0, 0, 0);
-                }
-        }
-        if (((k0 + HKS) & 255u) == 0) {  // end of a super-block
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        acc[i][j][v] += part[i][j][v];
-                        part[i][j][v] = 0.0f;
-                    }
-        }
-    };
-    Raw r0, r1;
-    if (k_begin < k_end) load_raw(k_begin, r0);
-    // a split holds whole super-blocks: an even number of stages
-    for (uint32_t k0 = k_begin; k0 < k_end; k0 += 2 * HKS) {
-        stage(k0, r0, r1);
-        stage(k0 + HKS, r1, r0);
-    }
-    lds_barrier();  // binv
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t nl = wn * 64 + j * 32 + l32;
-            const uint32_t n = n0 + nl;
-            const float bs = binv[nl];
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t m = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                if (m < M && n < N) Yout[size_t(m) * N + n] = acc[i][j][v] * xinv[m] * bs;
-            }
-        }
-}
-
 }  // namespace
 
 hipError_t launch_quantize_acts(const float* X, int8_t* xq, float* xs, size_t M, size_t K, hipStream_t stream) {
@@ -1390,10 +1044,10 @@ static hipError_t finish_splits(hipError_t e, const float* partial, float* Y, si
     const bool vec4 = total % 4 == 0 && !(reinterpret_cast<uintptr_t>(partial) & 15u) &&
                       !(reinterpret_cast<uintptr_t>(Y) & 15u);
     if (vec4)
-        hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3(static_cast<uint32_t>((total / 4 + kThreads - 1) / kThreads)),
+        hipLaunchKernelGGL((splitk_reduce_kernel<true, false>), dim3(static_cast<uint32_t>((total / 4 + kThreads - 1) / kThreads)),
                            dim3(kThreads), 0, stream, partial, Y, total, ks);
     else
-        hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3(static_cast<uint32_t>((total + kThreads - 1) / kThreads)),
+        hipLaunchKernelGGL((splitk_reduce_kernel<false, false>), dim3(static_cast<uint32_t>((total + kThreads - 1) / kThreads)),
                            dim3(kThreads), 0, stream, partial, Y, total, ks);
     return hipGetLastError();
 }
@@ -1505,6 +1159,19 @@ hipError_t launch_splitk_reduce(const float* partial, float* Y, size_t M, size_t
     return finish_splits(hipSuccess, partial, Y, M, N, splits, stream);
 }
 
+hipError_t launch_splitk_add(const float* partial, float* Y, size_t M, size_t N, uint32_t planes, hipStream_t stream) {
+    if (!partial || !Y || !planes) return hipErrorInvalidValue;
+    const size_t total = M * N;
+    const bool vec4 = total % 4 == 0 && !(reinterpret_cast<uintptr_t>(partial) & 15u) &&
+                      !(reinterpret_cast<uintptr_t>(Y) & 15u);
+    const dim3 grid(static_cast<uint32_t>(((vec4 ? total / 4 : total) + kThreads - 1) / kThreads));
+    if (vec4)
+        hipLaunchKernelGGL((splitk_reduce_kernel<true, true>), grid, dim3(kThreads), 0, stream, partial, Y, total, planes);
+    else
+        hipLaunchKernelGGL((splitk_reduce_kernel<false, true>), grid, dim3(kThreads), 0, stream, partial, Y, total, planes);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_i8(int fmt, const uint8_t* w, const int8_t* xq, const float* xs, float* Y, float* partial,
                           size_t M, size_t N, size_t K, hipStream_t stream, uint32_t* splits) {
     return launch_i8_common(fmt, w, xq, xs, Y, nullptr, partial, M, N, K, stream, splits);
@@ -1529,55 +1196,37 @@ size_t gemm_f32_partial_bytes(size_t M, size_t N, size_t K) {
     return ks > 1 ? size_t(ks) * M * N * sizeof(float) : 0;
 }
 
-// The super-block formats on the f16 MFMA: the split activations (hi and lo
-// halves, [M][K] each) and the row scales come first in the workspace, the
-// section rounded up to 256 bytes.
-static bool kq_f16(int fmt, size_t K) { return (fmt == kQ6_K || fmt == kQ4_K || fmt == kQ5_K) && K % 256 == 0; }
-static size_t a256(size_t v) { return (v + 255) / 256 * 256; }
-static size_t kq_split_bytes(int, size_t M, size_t K) { return a256(M * K * 2 * sizeof(_Float16) + M * sizeof(float)); }
-
+// What a caller is asked for: split-K partial sums for small grids and, for
+// the super-block formats, the split activations of the f16 MFMA kernels ([M]
+// rows of 4 K bytes and a scale, rounded up to 256 bytes).  With Q8_0 / Q4_0
+// the partial sums' room serves the split activations too, where they fit.
+static bool super_block(int fmt) { return fmt == kQ6_K || fmt == kQ4_K || fmt == kQ5_K; }
 size_t gemm_f32_workspace_bytes(int fmt, size_t M, size_t N, size_t K) {
-    return (kq_f16(fmt, K) ? kq_split_bytes(fmt, M, K) : 0) + gemm_f32_partial_bytes(M, N, K);
+    const size_t split = super_block(fmt) && K % 256 == 0 ? (M * K * 4 + M * sizeof(float) + 255) / 256 * 256 : 0;
+    return split + gemm_f32_partial_bytes(M, N, K);
+}
+size_t gemm_f32_best_bytes(int fmt, size_t M, size_t N, size_t K) {
+    const size_t ws = gemm_f32_workspace_bytes(fmt, M, N, K);
+    return gemm_split_supported(fmt, K) ? std::max(ws, gemm_split_bytes(fmt, M, K) + gemm_f32_partial_bytes(M, N, K)) : ws;
 }
 
 hipError_t launch_gemm_f32(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
-                           size_t N, size_t K, hipStream_t stream, uint32_t* launches) {
+                           size_t N, size_t K, hipStream_t stream, uint32_t* launches, bool best) {
+    // the plan, and so the rounding, is a function of the shape: a workspace
+    // larger than the shape asks for changes nothing
+    ws_bytes = std::min(ws_bytes, best ? gemm_f32_best_bytes(fmt, M, N, K) : gemm_f32_workspace_bytes(fmt, M, N, K));
     if (!w || !X || !Y || !M || !N || !row_bytes(fmt, K) || M > (1u << 24) || N > (1u << 24) || K > (1u << 24))
         return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(w) & 1u) || (reinterpret_cast<uintptr_t>(X) & 15u)) return hipErrorInvalidValue;
     if ((fmt == kQ4_K || fmt == kQ5_K) && (reinterpret_cast<uintptr_t>(w) & 3u)) return hipErrorInvalidValue;
+    if (const hipError_t e = launch_gemm_split(fmt, w, X, Y, ws, ws_bytes, M, N, K, stream, launches);
+        e != hipErrorInvalidConfiguration)
+        return e;
     const uint32_t tiles_m = static_cast<uint32_t>((M + BM - 1) / BM);
     const uint32_t tiles_n = static_cast<uint32_t>((N + BN - 1) / BN);
     const uint32_t stages = uint32_t((K + FK - 1) / FK);
     const uint32_t m = uint32_t(M), n = uint32_t(N), k = uint32_t(K);
     const size_t pbytes = gemm_f32_partial_bytes(M, N, K);
-    if (kq_f16(fmt, K) && ws && ws_bytes >= kq_split_bytes(fmt, M, K) && !(reinterpret_cast<uintptr_t>(ws) & 255u)) {
-        uint8_t* b = static_cast<uint8_t*>(ws);
-        _Float16* xh = reinterpret_cast<_Float16*>(b);
-        _Float16* xl = xh + M * K;
-        float* inv = reinterpret_cast<float*>(xl + M * K);
-        const size_t sb = kq_split_bytes(fmt, M, K);
-        float* partial = ws_bytes >= sb + pbytes && pbytes ? reinterpret_cast<float*>(b + sb) : nullptr;
-        uint32_t ks = partial ? choose_ksplit_f32(tiles_m * tiles_n, stages) : 1u;
-        constexpr uint32_t HKS = ZQ_KQ_HKS, SPB = 256 / HKS;  // stages per super-block
-        const uint32_t hstages = k / HKS;
-        const uint32_t spw = ((hstages + ks - 1) / ks + SPB - 1) / SPB * SPB;  // whole super-blocks per split
-        ks = (hstages + spw - 1) / spw;
-        float* out = ks > 1 ? partial : Y;
-        const dim3 grid(tiles_m * tiles_n * ks);
-        hipLaunchKernelGGL(split_rows_kernel, dim3(m), dim3(kThreads), 0, stream, X, xh, xl, inv, k);
-        if (fmt == kQ6_K)
-            hipLaunchKernelGGL((gemm_kq_h_kernel<kQ6_K, HKS>), grid, dim3(kThreads), 0, stream, w, xh, xl, inv, out, m, n,
-                               k, tiles_m, tiles_n, ks, spw);
-        else if (fmt == kQ4_K)
-            hipLaunchKernelGGL((gemm_kq_h_kernel<kQ4_K, HKS>), grid, dim3(kThreads), 0, stream, w, xh, xl, inv, out, m, n,
-                               k, tiles_m, tiles_n, ks, spw);
-        else
-            hipLaunchKernelGGL((gemm_kq_h_kernel<kQ5_K, HKS>), grid, dim3(kThreads), 0, stream, w, xh, xl, inv, out, m, n,
-                               k, tiles_m, tiles_n, ks, spw);
-        if (launches) *launches = ks > 1 ? 3 : 2;
-        return finish_splits(hipGetLastError(), partial, Y, M, N, ks, stream);
-    }
     float* partial = ws && pbytes && ws_bytes >= pbytes ? static_cast<float*>(ws) : nullptr;
     uint32_t ks = partial ? choose_ksplit_f32(tiles_m * tiles_n, stages) : 1u;
     const uint32_t spw = (stages + ks - 1) / ks;

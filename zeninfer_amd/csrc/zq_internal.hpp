@@ -100,16 +100,30 @@ hipError_t launch_gemm_i8(int fmt, const uint8_t* w, const int8_t* xq, const flo
 // Y[M][N] = the sum of `splits` partial planes in split order (the reduction
 // launch_gemm_i8 leaves to its caller when asked to).
 hipError_t launch_splitk_reduce(const float* partial, float* Y, size_t M, size_t N, uint32_t splits, hipStream_t stream);
+// Y[M][N] += `planes` partial planes, one after the other.
+hipError_t launch_splitk_add(const float* partial, float* Y, size_t M, size_t N, uint32_t planes, hipStream_t stream);
 
 // Prefill GEMM on fp32 activations (the reference CPU arithmetic).  `ws`
-// (ws_bytes, may be null) is the workspace: gemm_f32_workspace_bytes() lets
-// Q6_K run on the f16 MFMA (split activations) and any format split K; with
-// less the GEMM runs with what fits (fp32 MFMA, unsplit).  `launches`
-// (optional) receives the number of kernels enqueued.
+// (ws_bytes, may be null) is the workspace: with gemm_f32_workspace_bytes()
+// the super-block formats run on the f16 MFMA (split activations), Q8_0 / Q4_0
+// where it holds their split activations, and any format splits K; with less
+// the GEMM runs with what fits (fp32 MFMA, unsplit).  gemm_f32_best_bytes() is
+// the size for the library's own buffers, passed with `best`: room for both in
+// every format.  More than that is not used.
+// `launches` (optional) receives the number of kernels enqueued.
 size_t gemm_f32_partial_bytes(size_t M, size_t N, size_t K);
 size_t gemm_f32_workspace_bytes(int fmt, size_t M, size_t N, size_t K);
+size_t gemm_f32_best_bytes(int fmt, size_t M, size_t N, size_t K);
 hipError_t launch_gemm_f32(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
-                           size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr);
+                           size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr, bool best = false);
+
+// The fp32-activation GEMM on the f16 matrix cores over split activations
+// (zq_gemm_split.hip); hipErrorInvalidConfiguration when the format, shape or
+// workspace is not covered.
+bool gemm_split_supported(int fmt, size_t K);
+size_t gemm_split_bytes(int fmt, size_t M, size_t K);
+hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
+                             size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr);
 
 // Bit-exact tier helpers.
 hipError_t launch_dequantize(int fmt, const uint8_t* w, float* out, size_t rows, size_t cols,

@@ -165,7 +165,8 @@ bool alloc_runtime(zq_model& m, std::string& e) {
     for (uint32_t M = 1; M <= kPrefillChunk; ++M)
         for (auto nk : {std::pair<size_t, size_t>{QW, E}, {KW, E}, {QW + 2 * KW, E}, {E, QW}, {F, E}, {E, F}})
             partial = std::max({partial, zq::gemm_i8_partial_bytes(M, nk.first, nk.second),
-                                zq::gemm_f32_workspace_bytes(zq::kQ4_K, M, nk.first, nk.second)});
+                                zq::gemm_f32_best_bytes(zq::kQ4_K, M, nk.first, nk.second / 256 * 256),
+                                zq::gemm_f32_best_bytes(zq::kQ8_0, M, nk.first, nk.second)});
     const size_t xq_bytes = align_up(T * widest, kAlign), xs_bytes = align_up(T * widest / 32 * 4, kAlign);
     const size_t attn_bytes = align_up(zq::attention_decode_partial_floats(c.heads, c.head_dim, c.max_positions) * 4, kAlign);
     const size_t arg_bytes = align_up(zq::argmax_partial_bytes(), kAlign);
@@ -253,7 +254,7 @@ hipError_t project(zq_model& m, const Weight& w, const float* X, float* Y, uint3
     if (!m.fuse_quant) splits = nullptr;  // ZQ_MODEL_FUSED=0: the GEMM reduces its own split-K planes
     if (quantized)
         return zq::launch_gemm_i8(w.fmt, w.p, m.xq, m.xs, Y, m.partial, M, w.rows, w.cols, m.stream, splits);
-    return zq::launch_gemm_f32(w.fmt, w.p, X, Y, m.partial, m.partial_bytes, M, w.rows, w.cols, m.stream);
+    return zq::launch_gemm_f32(w.fmt, w.p, X, Y, m.partial, m.partial_bytes, M, w.rows, w.cols, m.stream, nullptr, true);
 }
 
 bool int8_ok(int fmt) { return fmt == zq::kQ8_0 || fmt == zq::kQ4_0; }
