@@ -1,5 +1,5 @@
-"""The fp32-activation GEMM on split f16 activations (zq_gemm_split.hip):
-edges of its tiles and of its K splits, rows of very different magnitude, and
+"""The fp32-activation GEMMs (zq_gemm_split.hip on split f16 activations,
+zq_gemm_skinny.hip for few tokens): edges of their tiles and K splits, rows of very different magnitude, and
 non-finite activations; and, on the CPU, that its kernels neither spill nor
 use packed fp32 arithmetic."""
 import os
@@ -22,13 +22,15 @@ def small(zq):
     zq.set_min_elements(old)
 
 
-# Tiles are 128 tokens by 128 or 256 rows, stages 32 k (three in flight),
-# super-blocks 256: one of each, one less and one more, an odd count of
-# stages, one stage, and K long enough to split.
+# Tiles are 128 tokens by 128 or 256 rows (32 or 64 by 32 for few tokens),
+# stages 32 k (three in flight), super-blocks 256: one of each, one less and one
+# more, an odd count of stages, one stage, fewer groups than waves, and K long
+# enough to split.
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ALL)
 @pytest.mark.parametrize("m,n,blocks", [(1, 1, 8), (2, 129, 8), (127, 255, 8), (128, 256, 16), (129, 257, 24), (257, 130, 8),
-                                        (70, 300, 128), (3, 33, 448), (130, 40, 264)])
+                                        (70, 300, 128), (3, 33, 448), (130, 40, 264), (32, 32, 8), (33, 31, 16),
+                                        (64, 65, 136), (300, 700, 256), (200, 3000, 256)])
 def test_edges(zq, orc, small, fmt, m, n, blocks):
     k = 32 * blocks
     w = orc.gen_weights(fmt, 500 + n, n, k)
@@ -41,9 +43,10 @@ def test_edges(zq, orc, small, fmt, m, n, blocks):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", (O.Q8_0, O.Q4_0))
-@pytest.mark.parametrize("blocks", (1, 2, 3, 5, 7, 31))
-def test_any_number_of_blocks(zq, orc, small, fmt, blocks):
-    m, n, k = 131, 270, 32 * blocks
+@pytest.mark.parametrize("m", (5, 47, 700))
+@pytest.mark.parametrize("blocks", (1, 2, 3, 5, 7, 31, 67))
+def test_any_number_of_blocks(zq, orc, small, fmt, m, blocks):
+    n, k = 270, 32 * blocks
     w = orc.gen_weights(fmt, 510 + blocks, n, k)
     X = orc.gen_normal(511, m * k)
     assert_close(zq.gemm(fmt, w, X, m, n, k, zq.ACT_F32), orc.gemm_f32(fmt, w, X, m, n, k), f"fmt={fmt} k={k}")
@@ -51,13 +54,13 @@ def test_any_number_of_blocks(zq, orc, small, fmt, blocks):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(140, 700, 2048), (20, 70, 512)])  # split activations; few tokens
 @pytest.mark.parametrize("fmt", ALL)
-def test_row_magnitudes_and_non_finite(zq, orc, small, fmt):
+def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k):
     """Each row has its own power of two, so a row's result does not depend on
     its scale; an infinite or NaN activation stays in its row, and with codes
     of one plane and no offset gives what the product of the dequantised
     weights gives."""
-    m, n, k = 140, 70, 512
     w = orc.gen_weights(fmt, 520, n, k)
     X = orc.gen_normal(521, m * k).reshape(m, k)
     base = zq.gemm(fmt, w, X, m, n, k, zq.ACT_F32).reshape(m, n)
@@ -83,13 +86,14 @@ def test_row_magnitudes_and_non_finite(zq, orc, small, fmt):
     zq.release(w)
 
 
-def test_generated_code(tmp_path):
+@pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))
+def test_generated_code(tmp_path, src):
     from zeninfer_amd.build import FLAGS, HIPCC, SRC
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not available")
     out = tmp_path / "split.s"
     flags = [f for f in FLAGS if f not in ("-shared", "-fPIC")]
-    r = subprocess.run([HIPCC, *flags, "--cuda-device-only", "-S", "-o", str(out), os.path.join(SRC, "zq_gemm_split.hip")],
+    r = subprocess.run([HIPCC, *flags, "--cuda-device-only", "-S", "-o", str(out), os.path.join(SRC, src)],
                        capture_output=True, text=True, timeout=900)
     assert r.returncode == 0, r.stderr[-2000:]
     asm = out.read_text()

@@ -365,14 +365,12 @@ int enqueue_gemm_batch(int fmt, const uint8_t* const* w, float* const* Y, const 
         }
         return ZQ_OK;
     }
-    for (size_t i = 0; i < count; ++i) {
-        uint32_t n = 0;
-        if (const int ls = launch_status(
-                zq::launch_gemm_f32(fmt, w[i], X, Y[i], ws, ws ? ws_bytes : 0, tokens, rows[i], cols, s, &n, own_ws));
-            ls != ZQ_OK)
-            return ls;
-        *dispatches += n;
-    }
+    uint32_t n = 0;
+    if (const int ls = launch_status(
+            zq::launch_gemm_f32_batch(fmt, w, Y, rows, count, X, ws, ws ? ws_bytes : 0, tokens, cols, s, &n, own_ws));
+        ls != ZQ_OK)
+        return ls;
+    *dispatches += n;
     return ZQ_OK;
 }
 

@@ -12,10 +12,9 @@
 //    arithmetic of gemv_q8_0_avx2_int8_prequant (kernels/avx2.cpp:562-585) and
 //    of the D3D12 int8 GEMM (shaders/q8_0_gemm_i8.hlsl:249-257).
 //
-//  * fp32 activations (all formats; the reference CPU arithmetic): the split
-//    f16 kernels of zq_gemm_split.hip where the workspace allows, else weights
-//    are dequantised exactly into LDS (the reference's dequantize values) and
-//    multiplied with v_mfma_f32_32x32x2_f32 in fp32.
+//  * fp32 activations (all formats; the reference CPU arithmetic): the kernels
+//    of zq_gemm_skinny.hip for few tokens and of zq_gemm_split.hip beyond,
+//    chosen at the end of this file.
 //
 // Kernels (int8 mode):
 //  * gemm_i8_direct4_kernel (K % 256 == 0, M > 64):
@@ -875,87 +874,6 @@ __global__ __launch_bounds__(256, 2) void gemm_i8_skinny_kernel(
     gemm_i8_skinny_body<FMT, DOTS>(W, XQ, XS, Y, dots, M, N, K, tiles_m, tiles_n, ksplit, stages_per_split);
 }
 
-// ------------------------------------------------------- fp32 GEMM -------
-constexpr int FK = 32;          // K elements per fp32 stage
-constexpr int FROW = FK + 4;    // LDS floats per row (pad)
-
-// Split K (ksplit > 1): workgroup blockIdx.x / tiles covers stages
-// [split * stages_per_split, ...) of FK elements and writes its partial sums
-// to Y + split * M * N; splitk_reduce_kernel adds them in split order.
-template <int FMT>
-__global__ __launch_bounds__(kThreads) void gemm_f32_kernel(const uint8_t* __restrict__ W, const float* __restrict__ X,
-                                                            float* __restrict__ Y, uint32_t M, uint32_t N, uint32_t K,
-                                                            uint32_t tiles_m, uint32_t tiles_n, uint32_t ksplit,
-                                                            uint32_t stages_per_split) {
-    __shared__ __align__(16) float As[BM * FROW];
-    __shared__ __align__(16) float Bs[BN * FROW];
-    const uint32_t total_tiles = tiles_m * tiles_n;
-    const uint32_t split = blockIdx.x / total_tiles;
-    uint32_t tm, tn;
-    tile_of(tiles_m, tiles_n, blockIdx.x % total_tiles, tm, tn);
-    const uint32_t m0 = tm * BM, n0 = tn * BN;
-    const uint32_t k_begin = split * stages_per_split * FK;
-    const uint32_t k_end = min(K, k_begin + stages_per_split * FK);
-    float* Yout = Y + (ksplit > 1 ? size_t(split) * M * N : 0);
-    const size_t rb = row_bytes_dev(FMT, K);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int l32 = lane & 31, lh = lane >> 5;
-    const int ld_row = tid >> 1, ld_half = tid & 1;
-    const float* a_src = X + size_t(min(m0 + ld_row, M - 1)) * K;
-    const uint8_t* b_src = W + size_t(min(n0 + ld_row, N - 1)) * rb;
-
-    v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    for (uint32_t k0 = k_begin; k0 < k_end; k0 += FK) {
-        __syncthreads();
-        {
-            const float4* s = reinterpret_cast<const float4*>(a_src + k0 + ld_half * 16);
-            float4* d = reinterpret_cast<float4*>(As + ld_row * FROW + ld_half * 16);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) d[i] = s[i];
-        }
-        if (ld_half == 0) {
-            float w[32];
-            dequant32<FMT>(b_src, k0, w);
-            float4* d = reinterpret_cast<float4*>(Bs + ld_row * FROW);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) d[i] = make_float4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < FK; kk += 2) {
-            float a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = As[(wm * 64 + i * 32 + l32) * FROW + kk + lh];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = Bs[(wn * 64 + j * 32 + l32) * FROW + kk + lh];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t n = n0 + wn * 64 + j * 32 + l32;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const uint32_t m = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                if (m < M && n < N) Yout[size_t(m) * N + n] = acc[i][j][v];
-            }
-        }
-}
-
 }  // namespace
 
 hipError_t launch_quantize_acts(const float* X, int8_t* xq, float* xs, size_t M, size_t K, hipStream_t stream) {
@@ -1183,8 +1101,8 @@ hipError_t launch_block_dots(int fmt, const uint8_t* w, const int8_t* xq, int32_
     return launch_i8_common(fmt, w, xq, nullptr, nullptr, out, nullptr, M, N, K, stream);
 }
 
-// Split factor of the fp32-activation GEMM: enough workgroups for two per CU,
-// at least 16 K stages per split.
+// Planes of partial sums that a caller of the fp32-activation GEMM is asked
+// for: two 128 x 128 tiles per CU, at least 16 groups of 32 per split.
 static uint32_t choose_ksplit_f32(uint32_t tiles, uint32_t stages) {
     const uint32_t want = (2u * uint32_t(device_cu_count()) + tiles - 1) / tiles;
     return std::max(1u, std::min(want, std::max(1u, stages / 16)));
@@ -1192,7 +1110,7 @@ static uint32_t choose_ksplit_f32(uint32_t tiles, uint32_t stages) {
 
 size_t gemm_f32_partial_bytes(size_t M, size_t N, size_t K) {
     const uint32_t tiles = uint32_t(((M + BM - 1) / BM) * ((N + BN - 1) / BN));
-    const uint32_t ks = choose_ksplit_f32(tiles, uint32_t((K + FK - 1) / FK));
+    const uint32_t ks = choose_ksplit_f32(tiles, uint32_t((K + 31) / 32));
     return ks > 1 ? size_t(ks) * M * N * sizeof(float) : 0;
 }
 
@@ -1210,49 +1128,57 @@ size_t gemm_f32_best_bytes(int fmt, size_t M, size_t N, size_t K) {
     return gemm_split_supported(fmt, K) ? std::max(ws, gemm_split_bytes(fmt, M, K) + gemm_f32_partial_bytes(M, N, K)) : ws;
 }
 
+hipError_t launch_gemm_f32_batch(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
+                                 const float* X, void* ws, size_t ws_bytes, size_t M, size_t K, hipStream_t stream,
+                                 uint32_t* launches, bool best) {
+    if (!w || !X || !Y || !M || !count || count > size_t(kMaxTasks) || !row_bytes(fmt, K) || M > (1u << 24) ||
+        K > (1u << 24) || (reinterpret_cast<uintptr_t>(X) & 15u))
+        return hipErrorInvalidValue;
+    const uintptr_t align = fmt == kQ4_K || fmt == kQ5_K ? 3u : 1u;
+    for (size_t i = 0; i < count; ++i)
+        if (!w[i] || !Y[i] || !rows[i] || rows[i] > (1u << 24) || (reinterpret_cast<uintptr_t>(w[i]) & align))
+            return hipErrorInvalidValue;
+    // Each matrix's kernel and split depend on its own shape and workspace
+    // alone, so a batch gives the bits of its single calls; those that the
+    // few-token kernel takes unsplit share one launch.
+    const uint8_t* sw[kMaxTasks];
+    float* sy[kMaxTasks];
+    size_t sn[kMaxTasks], shared = 0;
+    uint32_t total = 0;
+    for (size_t i = 0; i < count; ++i) {
+        const size_t N = rows[i];
+        // a workspace larger than the shape asks for changes nothing
+        const size_t use =
+            ws ? std::min(ws_bytes, best ? gemm_f32_best_bytes(fmt, M, N, K) : gemm_f32_workspace_bytes(fmt, M, N, K)) : 0;
+        const SkinnyPlan sk = plan_gemm_skinny_f32(fmt, M, N, K, use / (M * N * sizeof(float)));
+        if (sk.us > gemm_split_us(fmt, M, N, K, ws, use)) {
+            uint32_t n = 0;
+            if (const hipError_t e = launch_gemm_split(fmt, w[i], X, Y[i], ws, use, M, N, K, stream, &n); e != hipSuccess)
+                return e;
+            total += n;
+        } else if (sk.ks > 1) {
+            if (const hipError_t e = launch_gemm_skinny_f32(fmt, &w[i], &Y[i], &rows[i], 1, X, static_cast<float*>(ws), sk.ks,
+                                                            M, K, stream);
+                e != hipSuccess)
+                return e;
+            total += 2;
+        } else {
+            sw[shared] = w[i], sy[shared] = Y[i], sn[shared] = N;
+            ++shared;
+        }
+    }
+    if (shared) {
+        if (const hipError_t e = launch_gemm_skinny_f32(fmt, sw, sy, sn, shared, X, nullptr, 1, M, K, stream); e != hipSuccess)
+            return e;
+        ++total;
+    }
+    if (launches) *launches = total;
+    return hipSuccess;
+}
+
 hipError_t launch_gemm_f32(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
                            size_t N, size_t K, hipStream_t stream, uint32_t* launches, bool best) {
-    // the plan, and so the rounding, is a function of the shape: a workspace
-    // larger than the shape asks for changes nothing
-    ws_bytes = std::min(ws_bytes, best ? gemm_f32_best_bytes(fmt, M, N, K) : gemm_f32_workspace_bytes(fmt, M, N, K));
-    if (!w || !X || !Y || !M || !N || !row_bytes(fmt, K) || M > (1u << 24) || N > (1u << 24) || K > (1u << 24))
-        return hipErrorInvalidValue;
-    if ((reinterpret_cast<uintptr_t>(w) & 1u) || (reinterpret_cast<uintptr_t>(X) & 15u)) return hipErrorInvalidValue;
-    if ((fmt == kQ4_K || fmt == kQ5_K) && (reinterpret_cast<uintptr_t>(w) & 3u)) return hipErrorInvalidValue;
-    if (const hipError_t e = launch_gemm_split(fmt, w, X, Y, ws, ws_bytes, M, N, K, stream, launches);
-        e != hipErrorInvalidConfiguration)
-        return e;
-    const uint32_t tiles_m = static_cast<uint32_t>((M + BM - 1) / BM);
-    const uint32_t tiles_n = static_cast<uint32_t>((N + BN - 1) / BN);
-    const uint32_t stages = uint32_t((K + FK - 1) / FK);
-    const uint32_t m = uint32_t(M), n = uint32_t(N), k = uint32_t(K);
-    const size_t pbytes = gemm_f32_partial_bytes(M, N, K);
-    float* partial = ws && pbytes && ws_bytes >= pbytes ? static_cast<float*>(ws) : nullptr;
-    uint32_t ks = partial ? choose_ksplit_f32(tiles_m * tiles_n, stages) : 1u;
-    const uint32_t spw = (stages + ks - 1) / ks;
-    ks = (stages + spw - 1) / spw;  // no empty splits
-    float* out = ks > 1 ? partial : Y;
-    const dim3 grid(tiles_m * tiles_n * ks);
-    switch (fmt) {
-    case kQ8_0:
-        hipLaunchKernelGGL(gemm_f32_kernel<kQ8_0>, grid, dim3(kThreads), 0, stream, w, X, out, m, n, k, tiles_m, tiles_n, ks, spw);
-        break;
-    case kQ4_0:
-        hipLaunchKernelGGL(gemm_f32_kernel<kQ4_0>, grid, dim3(kThreads), 0, stream, w, X, out, m, n, k, tiles_m, tiles_n, ks, spw);
-        break;
-    case kQ6_K:
-        hipLaunchKernelGGL(gemm_f32_kernel<kQ6_K>, grid, dim3(kThreads), 0, stream, w, X, out, m, n, k, tiles_m, tiles_n, ks, spw);
-        break;
-    case kQ4_K:
-        hipLaunchKernelGGL(gemm_f32_kernel<kQ4_K>, grid, dim3(kThreads), 0, stream, w, X, out, m, n, k, tiles_m, tiles_n, ks, spw);
-        break;
-    case kQ5_K:
-        hipLaunchKernelGGL(gemm_f32_kernel<kQ5_K>, grid, dim3(kThreads), 0, stream, w, X, out, m, n, k, tiles_m, tiles_n, ks, spw);
-        break;
-    default: return hipErrorInvalidValue;
-    }
-    if (launches) *launches = ks > 1 ? 2 : 1;
-    return finish_splits(hipGetLastError(), partial, Y, M, N, ks, stream);
+    return launch_gemm_f32_batch(fmt, &w, &Y, &N, 1, X, ws, ws_bytes, M, K, stream, launches, best);
 }
 
 }  // namespace zq

@@ -699,6 +699,7 @@ struct SplitPlan {
     int wn = 4;           // waves per tile row: 4 (256 columns) or 2 (128)
     uint32_t ks = 1;      // K splits
     uint32_t blocks = 0;  // blocks per split
+    double us = 1e300;    // estimated kernel time
 };
 // The cheapest tile width and split with at most `planes` planes beside Y;
 // splits are whole super-blocks where the format has them, and at least 8
@@ -707,14 +708,13 @@ static SplitPlan plan_split(bool super, size_t M, size_t N, size_t K, size_t pla
     const uint32_t unit = super ? 8 : 1, units = uint32_t(K / 32) / unit;
     const uint32_t most = uint32_t(std::min<size_t>({planes + 1, 32, std::max(1u, units * unit / 8)}));
     SplitPlan best;
-    double best_t = 1e300;
     for (int wn : {4, 2}) {
         const uint32_t tiles = uint32_t(((M + 127) / 128) * ((N + 64 * wn - 1) / (64 * wn)));
         for (uint32_t ks = 1; ks <= most; ++ks) {
             const uint32_t ups = (units + ks - 1) / ks;
             if ((units + ups - 1) / ups != ks) continue;  // would leave empty splits
             const double t = split_cost(super, wn, tiles, ks, ups * unit, M, N);
-            if (t < best_t) best_t = t, best = SplitPlan{wn, ks, ups * unit};
+            if (t < best.us) best = SplitPlan{wn, ks, ups * unit, t};
         }
     }
     return best;
@@ -762,21 +762,54 @@ size_t gemm_split_bytes(int fmt, size_t M, size_t K) {
     return (M * K * 4 + sums + M * sizeof(int) + 255) / 256 * 256;
 }
 
+// Tokens whose split activations the workspace holds: M, or whole tiles.
+static size_t tokens_that_fit(int fmt, size_t M, size_t K, size_t ws_bytes) {
+    if (gemm_split_bytes(fmt, M, K) <= ws_bytes) return M;
+    size_t t = (M - 1) / 128 * 128;
+    while (t && gemm_split_bytes(fmt, t, K) > ws_bytes) t -= 128;
+    return t;
+}
+// The rest of the tokens after such a part: by the cheaper kernel, unsplit.
+static bool rest_on_skinny(int fmt, size_t rest, size_t N, size_t K, const void* ws, size_t ws_bytes, double& us) {
+    const double a = plan_gemm_skinny_f32(fmt, rest, N, K, 0).us, b = gemm_split_us(fmt, rest, N, K, ws, ws_bytes);
+    us = std::min(a, b);
+    return a <= b;
+}
+
+double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size_t ws_bytes) {
+    if (!gemm_split_supported(fmt, K) || !ws || (reinterpret_cast<uintptr_t>(ws) & 15u)) return 1e300;
+    const size_t fit = tokens_that_fit(fmt, M, K, ws_bytes), sb = gemm_split_bytes(fmt, M, K);
+    if (fit < M) {
+        // (Q4_K / Q5_K at the asked-for size, which has no room for the group
+        // sums: 97 of 100 tokens fit; less than half is not worth it)
+        if (fit < (M + 1) / 2) return 1e300;
+        double rest;
+        (void)rest_on_skinny(fmt, M - fit, N, K, ws, ws_bytes, rest);
+        return gemm_split_us(fmt, fit, N, K, ws, ws_bytes) + rest;
+    }
+    // beside the GEMM: two launches and the activations read and written once
+    return 8.0 + double(M) * double(K) * 8.0 / 4.0e6 +
+           plan_split(fmt != kQ8_0 && fmt != kQ4_0, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float))).us;
+}
+
 hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
                              size_t N, size_t K, hipStream_t stream, uint32_t* launches) {
     const size_t sb = gemm_split_bytes(fmt, M, K);
     if (!gemm_split_supported(fmt, K) || !ws || (reinterpret_cast<uintptr_t>(ws) & 15u)) return hipErrorInvalidConfiguration;
-    if (ws_bytes < sb) {
-        // two halves of the tokens, one after the other, where only they fit
-        const size_t half = (M / 2 + 127) / 128 * 128;
-        if (M <= 256 || ws_bytes < gemm_split_bytes(fmt, half, K)) return hipErrorInvalidConfiguration;
-        uint32_t l0 = 0, l1 = 0;
-        const hipError_t e = launch_gemm_split(fmt, w, X, Y, ws, ws_bytes, half, N, K, stream, &l0);
-        if (e != hipSuccess) return e;
-        const hipError_t e1 =
-            launch_gemm_split(fmt, w, X + half * K, Y + half * N, ws, ws_bytes, M - half, N, K, stream, &l1);
-        if (launches) *launches = l0 + l1;
-        return e1;
+    const size_t fit = tokens_that_fit(fmt, M, K, ws_bytes);
+    if (fit < M) {
+        if (fit < (M + 1) / 2) return hipErrorInvalidConfiguration;
+        uint32_t n = 0, rest_n = 1;
+        if (const hipError_t e = launch_gemm_split(fmt, w, X, Y, ws, ws_bytes, fit, N, K, stream, &n); e != hipSuccess) return e;
+        const float* rx = X + fit * K;
+        float* ry = Y + fit * N;
+        double us;
+        const hipError_t e =
+            rest_on_skinny(fmt, M - fit, N, K, ws, ws_bytes, us)
+                ? launch_gemm_skinny_f32(fmt, &w, &ry, &N, 1, rx, nullptr, 1, M - fit, K, stream)
+                : launch_gemm_split(fmt, w, rx, ry, ws, ws_bytes, M - fit, N, K, stream, &rest_n);
+        if (launches) *launches = n + rest_n;
+        return e;
     }
     uint8_t* xs = static_cast<uint8_t*>(ws);
     uint8_t* ss = xs + M * K * 4;

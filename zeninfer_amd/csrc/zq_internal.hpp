@@ -104,12 +104,10 @@ hipError_t launch_splitk_reduce(const float* partial, float* Y, size_t M, size_t
 hipError_t launch_splitk_add(const float* partial, float* Y, size_t M, size_t N, uint32_t planes, hipStream_t stream);
 
 // Prefill GEMM on fp32 activations (the reference CPU arithmetic).  `ws`
-// (ws_bytes, may be null) is the workspace: with gemm_f32_workspace_bytes()
-// the super-block formats run on the f16 MFMA (split activations), Q8_0 / Q4_0
-// where it holds their split activations, and any format splits K; with less
-// the GEMM runs with what fits (fp32 MFMA, unsplit).  gemm_f32_best_bytes() is
-// the size for the library's own buffers, passed with `best`: room for both in
-// every format.  More than that is not used.
+// (ws_bytes, may be null) is the workspace, for split activations and split-K
+// planes; with less than gemm_f32_workspace_bytes() the GEMM runs with what
+// fits.  gemm_f32_best_bytes() is the size for the library's own buffers, passed
+// with `best`: room for both in every format.  More than that is not used.
 // `launches` (optional) receives the number of kernels enqueued.
 size_t gemm_f32_partial_bytes(size_t M, size_t N, size_t K);
 size_t gemm_f32_workspace_bytes(int fmt, size_t M, size_t N, size_t K);
@@ -117,13 +115,32 @@ size_t gemm_f32_best_bytes(int fmt, size_t M, size_t N, size_t K);
 hipError_t launch_gemm_f32(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
                            size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr, bool best = false);
 
+// `count` (at most kMaxTasks) matrices sharing X: the bits of the single calls.
+hipError_t launch_gemm_f32_batch(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
+                                 const float* X, void* ws, size_t ws_bytes, size_t M, size_t K, hipStream_t stream,
+                                 uint32_t* launches = nullptr, bool best = false);
+
 // The fp32-activation GEMM on the f16 matrix cores over split activations
 // (zq_gemm_split.hip); hipErrorInvalidConfiguration when the format, shape or
-// workspace is not covered.
+// workspace is not covered.  gemm_split_us: its estimated time (infinite when
+// not covered).
 bool gemm_split_supported(int fmt, size_t K);
 size_t gemm_split_bytes(int fmt, size_t M, size_t K);
+double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size_t ws_bytes);
 hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
                              size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr);
+
+// The fp32-activation GEMM for few tokens or without a workspace
+// (zq_gemm_skinny.hip): the K splits for at most `planes` planes beside Y and
+// the estimated time; then `count` matrices sharing X in one launch (ks > 1:
+// one matrix, its partial planes, and a second launch that adds them).
+struct SkinnyPlan {
+    uint32_t ks;
+    double us;
+};
+SkinnyPlan plan_gemm_skinny_f32(int fmt, size_t M, size_t N, size_t K, size_t planes);
+hipError_t launch_gemm_skinny_f32(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
+                                  const float* X, float* partial, uint32_t ks, size_t M, size_t K, hipStream_t stream);
 
 // Bit-exact tier helpers.
 hipError_t launch_dequantize(int fmt, const uint8_t* w, float* out, size_t rows, size_t cols,
