@@ -7,6 +7,7 @@ streams only) or raw integer device pointers.
 """
 import ctypes
 import os
+import struct
 
 import numpy as np
 
@@ -223,20 +224,27 @@ def _check_device(t, what):
         raise ValueError(f"{what}: tensor is on {t.device}, the library runs on cuda:{_device_index()}")
 
 
-def _need(t, nbytes, what):
-    """A torch tensor passed as a device buffer must live on the library's GPU,
-    be contiguous and hold at least nbytes: the kernels index it from the sizes
-    alone, so a short buffer would be read or written past its end, and the
-    address of a host tensor handed to a kernel faults the GPU.  Raw addresses
-    are the caller's responsibility."""
+def _need(t, nbytes, what, dev=None):
+    """Device address of a torch tensor passed as a device buffer (or of a raw
+    address, or None).  A tensor must live on the library's GPU, be contiguous
+    and hold at least nbytes: the kernels index it from the sizes alone, so a
+    short buffer would be read or written past its end, and the address of a
+    host tensor handed to a kernel faults the GPU.  Raw addresses are the
+    caller's responsibility.  dev: _device_index(), where the caller has it."""
     if t is None or isinstance(t, int):
-        return
+        return t
+    # one pass of cheap queries where all is well (this runs for every buffer
+    # of every call); the messages otherwise
+    if (getattr(t, "is_cuda", False) and t.get_device() == (_device_index() if dev is None else dev) and t.is_contiguous()
+            and t.nbytes >= nbytes):
+        return t.data_ptr()
     _check_device(t, what)
     if not t.is_contiguous():
         raise ValueError(f"{what}: tensor must be contiguous")
     have = t.numel() * t.element_size()
     if have < nbytes:
         raise ValueError(f"{what}: buffer holds {have} bytes, the call needs {nbytes}")
+    return t.data_ptr()
 
 
 def _stream(stream):
@@ -393,23 +401,39 @@ def release_all():
 
 
 # ---- device-pointer API (torch tensors or raw addresses) ------------------
+# These calls only enqueue work, so at decode sizes the Python in front of the
+# launch is the call's time: each buffer is checked and its address taken in
+# one step (_need), and a batch's task table is packed in one.
+_U64 = (1 << 64) - 1
+_GEMV_TASKS = [GemvTask * n for n in range(MAX_BATCH + 1)]
+_GEMM_TASKS = [GemmTask * n for n in range(MAX_BATCH + 1)]
+
+
+def _task_table(types, task, flat):
+    """ctypes array of {address, address, count} tasks from their flat values."""
+    n = len(flat) // 3
+    t = types[n] if n < len(types) else task * n
+    return t.from_buffer_copy(struct.pack("=%dQ" % len(flat), *flat)) if n else t()
+
+
 def gemv_dev(fmt, w, x, y, rows, cols, stream=None):
-    _need(w, weight_bytes(fmt, rows, cols), "gemv_dev weights")
-    _need(x, 4 * cols, "gemv_dev x")
-    _need(y, 4 * rows, "gemv_dev y")
-    return check(lib().zq_hip_gemv_dev(fmt, _dptr(w), _dptr(x), _dptr(y), rows, cols, _stream(stream)),
-                 "zq_hip_gemv_dev")
+    dev = _device_index()
+    w = _need(w, weight_bytes(fmt, rows, cols), "gemv_dev weights", dev)
+    x = _need(x, 4 * cols, "gemv_dev x", dev)
+    y = _need(y, 4 * rows, "gemv_dev y", dev)
+    return check(lib().zq_hip_gemv_dev(fmt, w, x, y, rows, cols, _stream(stream)), "zq_hip_gemv_dev")
 
 
 def gemv_batch_dev(fmt, x, tasks, cols, stream=None):
     """tasks: list of (weights, y, rows)."""
-    _need(x, 4 * cols, "gemv_batch_dev x")
+    dev = _device_index()
+    x = _need(x, 4 * cols, "gemv_batch_dev x", dev)
+    flat = []
     for w, y, r in tasks:
-        _need(w, weight_bytes(fmt, r, cols), "gemv_batch_dev weights")
-        _need(y, 4 * r, "gemv_batch_dev y")
-    arr = (GemvTask * len(tasks))(*[GemvTask(_dptr(w), _dptr(y), r) for w, y, r in tasks])
-    return check(lib().zq_hip_gemv_batch_dev(fmt, _dptr(x), arr, len(tasks), cols, _stream(stream)),
-                 "zq_hip_gemv_batch_dev")
+        flat += (_need(w, weight_bytes(fmt, r, cols), "gemv_batch_dev weights", dev) or 0,
+                 _need(y, 4 * r, "gemv_batch_dev y", dev) or 0, r & _U64)
+    return check(lib().zq_hip_gemv_batch_dev(fmt, x, _task_table(_GEMV_TASKS, GemvTask, flat), len(tasks), cols,
+                                             _stream(stream)), "zq_hip_gemv_batch_dev")
 
 
 def gemm_workspace_bytes(fmt, tokens, rows, cols, act=ACT_DEFAULT):
@@ -417,16 +441,13 @@ def gemm_workspace_bytes(fmt, tokens, rows, cols, act=ACT_DEFAULT):
 
 
 def gemm_dev(fmt, w, X, Y, tokens, rows, cols, act=ACT_DEFAULT, workspace=None, workspace_bytes=0, stream=None):
-    _need(w, weight_bytes(fmt, rows, cols), "gemm_dev weights")
-    _need(X, 4 * tokens * cols, "gemm_dev X")
-    _need(Y, 4 * tokens * rows, "gemm_dev Y")
-    _need(workspace, workspace_bytes, "gemm_dev workspace")
-    return check(lib().zq_hip_gemm_dev(fmt, _dptr(w), _dptr(X), _dptr(Y), tokens, rows, cols, act,
-                                       _dptr(workspace), workspace_bytes, _stream(stream)), "zq_hip_gemm_dev")
-
-
-def _gemm_tasks(tasks):
-    return (GemmTask * len(tasks))(*[GemmTask(_dptr(w), _dptr(Y), r) for w, Y, r in tasks])
+    dev = _device_index()
+    w = _need(w, weight_bytes(fmt, rows, cols), "gemm_dev weights", dev)
+    X = _need(X, 4 * tokens * cols, "gemm_dev X", dev)
+    Y = _need(Y, 4 * tokens * rows, "gemm_dev Y", dev)
+    workspace = _need(workspace, workspace_bytes, "gemm_dev workspace", dev)
+    return check(lib().zq_hip_gemm_dev(fmt, w, X, Y, tokens, rows, cols, act, workspace, workspace_bytes,
+                                       _stream(stream)), "zq_hip_gemm_dev")
 
 
 def gemm_batch_workspace_bytes(fmt, rows, tokens, cols, act=ACT_DEFAULT):
@@ -436,14 +457,15 @@ def gemm_batch_workspace_bytes(fmt, rows, tokens, cols, act=ACT_DEFAULT):
 
 def gemm_batch_dev(fmt, X, tasks, tokens, cols, act=ACT_DEFAULT, workspace=None, workspace_bytes=0, stream=None):
     """tasks: list of (weights, Y, rows)."""
-    _need(X, 4 * tokens * cols, "gemm_batch_dev X")
+    dev = _device_index()
+    X = _need(X, 4 * tokens * cols, "gemm_batch_dev X", dev)
+    flat = []
     for w, Y, r in tasks:
-        _need(w, weight_bytes(fmt, r, cols), "gemm_batch_dev weights")
-        _need(Y, 4 * tokens * r, "gemm_batch_dev Y")
-    _need(workspace, workspace_bytes, "gemm_batch_dev workspace")
-    return check(lib().zq_hip_gemm_batch_dev(fmt, _dptr(X), _gemm_tasks(tasks), len(tasks), tokens, cols, act,
-                                             _dptr(workspace), workspace_bytes, _stream(stream)),
-                 "zq_hip_gemm_batch_dev")
+        flat += (_need(w, weight_bytes(fmt, r, cols), "gemm_batch_dev weights", dev) or 0,
+                 _need(Y, 4 * tokens * r, "gemm_batch_dev Y", dev) or 0, r & _U64)
+    workspace = _need(workspace, workspace_bytes, "gemm_batch_dev workspace", dev)
+    return check(lib().zq_hip_gemm_batch_dev(fmt, X, _task_table(_GEMM_TASKS, GemmTask, flat), len(tasks), tokens, cols, act,
+                                             workspace, workspace_bytes, _stream(stream)), "zq_hip_gemm_batch_dev")
 
 
 def rms_norm_dev(x, w, y, rows, cols, eps, stream=None):
@@ -460,19 +482,20 @@ def ffn_residual_workspace_bytes(hidden, ffn_rows):
 
 def ffn_residual_fused_dev(fmt, wo, wg, wu, wd, norm_w, x, attn_out, out, hidden, attn_width, ffn_rows, eps,
                            workspace, workspace_bytes, stream=None):
-    _need(wo, weight_bytes(fmt, hidden, attn_width), "ffn_residual_fused_dev attn_output")
-    for w, what in ((wg, "gate"), (wu, "up")):
-        _need(w, weight_bytes(fmt, ffn_rows, hidden), f"ffn_residual_fused_dev {what}")
-    _need(wd, weight_bytes(fmt, hidden, ffn_rows), "ffn_residual_fused_dev down")
-    _need(norm_w, 4 * hidden, "ffn_residual_fused_dev norm_weight")
-    _need(x, 4 * hidden, "ffn_residual_fused_dev x")
-    _need(attn_out, 4 * attn_width, "ffn_residual_fused_dev attn_out")
-    _need(out, 4 * hidden, "ffn_residual_fused_dev out")
-    _need(workspace, workspace_bytes, "ffn_residual_fused_dev workspace")
-    return check(lib().zq_hip_ffn_residual_fused_dev(fmt, _dptr(wo), _dptr(wg), _dptr(wu), _dptr(wd), _dptr(norm_w),
-                                                     _dptr(x), _dptr(attn_out), _dptr(out), hidden, attn_width,
-                                                     ffn_rows, eps, _dptr(workspace), workspace_bytes,
-                                                     _stream(stream)), "zq_hip_ffn_residual_fused_dev")
+    dev = _device_index()
+    wo = _need(wo, weight_bytes(fmt, hidden, attn_width), "ffn_residual_fused_dev attn_output", dev)
+    n = weight_bytes(fmt, ffn_rows, hidden)
+    wg = _need(wg, n, "ffn_residual_fused_dev gate", dev)
+    wu = _need(wu, n, "ffn_residual_fused_dev up", dev)
+    wd = _need(wd, weight_bytes(fmt, hidden, ffn_rows), "ffn_residual_fused_dev down", dev)
+    norm_w = _need(norm_w, 4 * hidden, "ffn_residual_fused_dev norm_weight", dev)
+    x = _need(x, 4 * hidden, "ffn_residual_fused_dev x", dev)
+    attn_out = _need(attn_out, 4 * attn_width, "ffn_residual_fused_dev attn_out", dev)
+    out = _need(out, 4 * hidden, "ffn_residual_fused_dev out", dev)
+    workspace = _need(workspace, workspace_bytes, "ffn_residual_fused_dev workspace", dev)
+    return check(lib().zq_hip_ffn_residual_fused_dev(fmt, wo, wg, wu, wd, norm_w, x, attn_out, out, hidden, attn_width,
+                                                     ffn_rows, eps, workspace, workspace_bytes, _stream(stream)),
+                 "zq_hip_ffn_residual_fused_dev")
 
 
 def noalloc_scratch_bytes():
