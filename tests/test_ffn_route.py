@@ -1,0 +1,61 @@
+"""The routes of ffn_residual_fused: gate|up with SiLU * up in its store, the
+residual in the down GEMV's store (fp32 and MFMA streaming kernels, with and
+without SiLU * up in front) and the separate launches, at each one's edges."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+DEV = "cuda:0"
+
+
+# (hidden, ffn): pair + fp32 store with 8 / 16 waves; pair + MFMA store at one
+# and four row blocks per workgroup and at its longest rows; pair + separate add
+# (ffn not whole 256); SiLU * up in front (hidden past 4096) with one, two and
+# four slices per row; nothing fused (hidden not whole 256)
+@pytest.mark.parametrize("hidden,ffn", [(256, 256), (2304, 1024), (512, 4352), (4096, 8192), (768, 16384), (512, 2880),
+                                        (4352, 512), (4352, 4352), (4352, 8448), (288, 512)])
+@pytest.mark.parametrize("fmt", (O.Q8_0, O.Q4_0))
+def test_down_stores_the_residual_sum(zq, orc, fmt, hidden, ffn):
+    """With Wo = 0 and a norm weight of 0 every product is 0 and out is x, bit
+    for bit.  Otherwise the result is the chain's of separate calls: the GEMV
+    sums are the same kernels', so the two differ by the SiLU's expf (2 ulp) and
+    the kernels' orders of addition, both within the GEMV bar taken relative to
+    the magnitudes the last projection sums."""
+    aw = 256
+    w = {k: orc.gen_weights(fmt, s, r, c) for k, s, r, c in
+         (("o", 900, hidden, aw), ("g", 901, ffn, hidden), ("u", 902, ffn, hidden), ("d", 903, hidden, ffn))}
+    dev = {}
+    for k, (r, c) in {"o": (hidden, aw), "g": (ffn, hidden), "u": (ffn, hidden), "d": (hidden, ffn)}.items():
+        dev[k] = torch.zeros(zq.weight_bytes(fmt, r, c), dtype=torch.uint8, device=DEV)
+        dev[k][: w[k].size] = torch.from_numpy(w[k]).to(DEV)
+    x, nw, a = (torch.from_numpy(orc.gen_normal(s, n)).to(DEV) for s, n in ((904, hidden), (905, hidden), (906, aw)))
+    wsb = zq.ffn_residual_workspace_bytes(hidden, ffn)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=DEV)
+
+    def run(att, norm, out):
+        zq.ffn_residual_fused_dev(fmt, dev["o"], dev["g"], dev["u"], dev["d"], norm, x, att, out, hidden, aw, ffn,
+                                  1e-5, ws, wsb)
+        return out
+
+    out = torch.full((hidden + 64,), 7.0, device=DEV)
+    run(torch.zeros_like(a), torch.zeros_like(nw), out)
+    assert torch.equal(out[:hidden], x) and bool((out[hidden:] == 7.0).all())
+
+    run(a, nw, out)
+    t0, h2, g, u, d = (torch.empty(n, device=DEV) for n in (hidden, hidden, ffn, ffn, hidden))
+    zq.gemv_dev(fmt, dev["o"], a, t0, hidden, aw)
+    h1 = t0 + x
+    zq.rms_norm_dev(h1, nw, h2, 1, hidden, 1e-5)
+    zq.gemv_dev(fmt, dev["g"], h2, g, ffn, hidden)
+    zq.gemv_dev(fmt, dev["u"], h2, u, ffn, hidden)
+    f = g / (1.0 + torch.exp(-g)) * u
+    zq.gemv_dev(fmt, dev["d"], f, d, hidden, ffn)
+    dd = orc.dequantize(fmt, w["d"], hidden * ffn).reshape(hidden, ffn).astype(np.float64)
+    mag = np.abs(dd) @ f.abs().double().cpu().numpy() + h1.abs().double().cpu().numpy()
+    got, want = out[:hidden].double().cpu().numpy(), (h1 + d).double().cpu().numpy()
+    assert np.all(np.abs(got - want) <= 1e-4 + 1e-5 * mag)
+    assert torch.equal(run(a, nw, x)[:hidden], out[:hidden])  # in place of x

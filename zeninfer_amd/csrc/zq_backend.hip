@@ -387,9 +387,10 @@ bool ffn_residual_args_ok(int fmt, const void* wo, const void* wg, const void* w
 //   t0 = Wo . attn_out;  h1 = t0 + x;  h2 = rmsnorm(h1) * norm_w;
 //   g = Wg . h2;  u = Wu . h2;  f = silu(g) * u;  d = Wd . f;  out = h1 + d.
 // Q8_0 / Q4_0 on the streaming shapes fold the add + norm into the gate|up
-// GEMV and silu * up into the down GEMV; Q4_K / Q5_K / Q6_K form silu * up
-// in a paired gate|up GEMV; otherwise they run as kernels of their own.  x
-// is read before out is written, so out may alias x.
+// GEMV, silu * up into its store or into the down GEMV, and the residual add
+// into the down GEMV's store; Q4_K / Q5_K / Q6_K form silu * up in a paired
+// gate|up GEMV; otherwise they run as kernels of their own.  x is read before
+// out is written, so out may alias x.
 int enqueue_ffn_residual(int fmt, const uint8_t* wo, const uint8_t* wg, const uint8_t* wu, const uint8_t* wd,
                          const float* norm_w, const float* x, const float* attn_out, float* out, size_t hidden,
                          size_t attn_width, size_t ffn_rows, float eps, void* ws, size_t ws_bytes, hipStream_t s,
@@ -420,43 +421,55 @@ int enqueue_ffn_residual(int fmt, const uint8_t* wo, const uint8_t* wg, const ui
     if (const int ls = launch_status(zq::launch_gemv(fmt, &to, 1, attn_out, attn_width, s)); ls != ZQ_OK) return ls;
     zq::GemvTask gu[2] = {{wg, g, F}, {wu, u, F}};
     const zq::XPrologue norm{zq::kAddNorm, t0, x, norm_w, h1, eps};
-    hipError_t e = zq::launch_gemv_prologue(fmt, gu, 2, norm, hidden, s);
-    zq::GemvTask dn{wd, d, H};
-    bool paired = false;  // g already holds silu(gate) * up
+    const zq::GemvTask dn{wd, d, H}, to_out{wd, out, H};
+    uint64_t n = 1;
+    auto done = [&](hipError_t e, uint64_t launches) {
+        n += launches;
+        return e == hipSuccess;
+    };
+    // gate|up: with the add and norm as its prologue and SiLU * up as its
+    // epilogue where both fit (Q8_0 / Q4_0 up to 4096 columns), so that the down
+    // GEMV is a plain one and not one whose every workgroup recomputes SiLU * up.
+    // With the residual add in the down GEMV's store, Q8_0 with hidden 4096: ffn
+    // 14336 45.2 -> 42.2 us a call, ffn 4096 23.5 -> 21.7; 512 / 1024, bound by
+    // its launches, 22.2 -> 14.0 (three instead of four).  The add alone, with
+    // hidden 5120 / 13824: 61.9 -> 59.7 us.
+    bool paired = true;  // g holds silu(gate) * up
+    hipError_t e = zq::launch_gemv_prologue_silu_pair(fmt, gu[0], gu[1], norm, hidden, s);
+    if (e == hipErrorInvalidConfiguration) {
+        paired = false;
+        e = zq::launch_gemv_prologue(fmt, gu, 2, norm, hidden, s);
+    }
     if (e == hipErrorInvalidConfiguration) {
         // unfused: h1 = t0 + x, h2 = rmsnorm(h1) * w (into d), then gate|up
         // of h2 -- as one paired GEMV storing silu(gate) * up into g where the
         // format takes it (Q4_K / Q5_K / Q6_K), else as a 2-task GEMV
-        if (zq::launch_add_to(t0, x, h1, hidden, s) != hipSuccess ||
-            zq::launch_rmsnorm(h1, norm_w, d, 1, H, eps, s) != hipSuccess)
+        if (!done(zq::launch_add_to(t0, x, h1, hidden, s), 1) ||
+            !done(zq::launch_rmsnorm(h1, norm_w, d, 1, H, eps, s), 1))
             return ZQ_ERR_HIP;
-        *dispatches += 2;
-        const hipError_t pe = zq::launch_gemv_silu_pair(fmt, gu[0], gu[1], d, hidden, s);
-        if (pe != hipSuccess && pe != hipErrorInvalidConfiguration) return ZQ_ERR_HIP;
-        paired = pe == hipSuccess;
-        if (!paired && zq::launch_gemv(fmt, gu, 2, d, hidden, s) != hipSuccess) return ZQ_ERR_HIP;
-        ++*dispatches;
-    } else if (e != hipSuccess) {
-        return ZQ_ERR_HIP;
-    } else {
-        ++*dispatches;
+        e = zq::launch_gemv_silu_pair(fmt, gu[0], gu[1], d, hidden, s);
+        paired = e == hipSuccess;
+        if (e == hipErrorInvalidConfiguration) e = zq::launch_gemv(fmt, gu, 2, d, hidden, s);
     }
-    const zq::XPrologue act{zq::kSiluMul, g, u, nullptr, nullptr, 0.0f};
-    e = paired ? hipErrorInvalidConfiguration : zq::launch_gemv_prologue(fmt, &dn, 1, act, ffn_rows, s);
+    if (!done(e, 1)) return ZQ_ERR_HIP;
+    // down, with the residual add in its store where the format's kernel has it
+    bool added = true;
     if (paired) {
-        if (zq::launch_gemv(fmt, &dn, 1, g, ffn_rows, s) != hipSuccess) return ZQ_ERR_HIP;
-        ++*dispatches;
-    } else if (e == hipErrorInvalidConfiguration) {
-        if (zq::launch_silu_mul(g, u, g, ffn_rows, s) != hipSuccess || zq::launch_gemv(fmt, &dn, 1, g, ffn_rows, s) != hipSuccess)
-            return ZQ_ERR_HIP;
-        *dispatches += 2;
-    } else if (e != hipSuccess) {
-        return ZQ_ERR_HIP;
+        e = zq::launch_gemv_add(fmt, to_out, g, h1, ffn_rows, s);
     } else {
-        ++*dispatches;
+        zq::XPrologue act{zq::kSiluMul, g, u, nullptr, nullptr, 0.0f};
+        act.res = h1;
+        e = zq::launch_gemv_prologue(fmt, &to_out, 1, act, ffn_rows, s);
     }
-    if (const int ls = launch_status(zq::launch_add_to(h1, d, out, hidden, s)); ls != ZQ_OK) return ls;
-    *dispatches += 2;
+    if (e == hipErrorInvalidConfiguration) {
+        added = false;
+        if (!paired && !done(zq::launch_silu_mul(g, u, g, ffn_rows, s), 1)) return ZQ_ERR_HIP;
+        e = zq::launch_gemv(fmt, &dn, 1, g, ffn_rows, s);
+    }
+    if (!done(e, 1)) return ZQ_ERR_HIP;
+    if (!added)
+        if (const int ls = launch_status(zq::launch_add_to(h1, d, out, hidden, s)); ls != ZQ_OK) return ls;
+    *dispatches += n + (added ? 0 : 1);
     return ZQ_OK;
 }
 

@@ -278,9 +278,10 @@ __global__ __launch_bounds__(kThreads) void gemv_xreg_kernel(TaskTable tt, const
 // up rows, and the block stores f = silu(gate.x) * (up.x) into the first
 // task's y (the expression of silu_mul_kernel), so the down projection reads
 // f as a plain vector.
-template <int FMT, int R, int S, int NW, int D, int XK, int EP = 0>
+template <int FMT, int R, int S, int NW, int D, int XK, int EP = 0, bool RES = false>
 __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, const float* __restrict__ x,
                                                                uint32_t cols, uint32_t total_blocks, XPrologue pro) {
+    static_assert(!RES || (XK != kAddNorm && EP == 0));
     static_assert(EP == 0 || (S == 1 && R == 1 && NW == 16), "the SiLU pair epilogue takes one row per wave");
     constexpr int DW = FMT == kQ8_0 ? 17 : 9;
     constexpr int NT = NW * 64;
@@ -446,6 +447,11 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                 stash(u[d]);
                 const uint32_t row0 = row0s[d];
                 const int ti = tis[d];
+                // the residual ahead of the next block's weights: loads
+                // retire in order, so behind them its use would wait for them
+                float rv = 0.0f;
+                if constexpr (RES)
+                    if (slice == 0 && lane < R) rv = pro.res[min(row0 + lane, tt.t[ti].rows - 1)];
                 const uint32_t nblk = blk + uint32_t(D) * gridDim.x;
                 if (nblk < total_blocks) {
                     const uint8_t* rowp[R];
@@ -475,7 +481,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                 } else if constexpr (S == 1) {
 #pragma unroll
                     for (int r = 0; r < R; ++r)
-                        if (lane == r && row0 + r < t.rows) t.y[row0 + r] = acc[r];
+                        if (lane == r && row0 + r < t.rows) t.y[row0 + r] = RES ? rv + acc[r] : acc[r];
                 } else {
                     if (lane == 0) {
 #pragma unroll
@@ -486,7 +492,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                         float v = 0.0f;
 #pragma unroll
                         for (int s2 = 0; s2 < S; ++s2) v += red[parity][team * S + s2][lane];
-                        if (row0 + lane < t.rows) t.y[row0 + lane] = v;
+                        if (row0 + lane < t.rows) t.y[row0 + lane] = RES ? rv + v : v;
                     }
                     parity ^= 1;
                 }
@@ -1199,7 +1205,7 @@ struct MfmaGeo {
     static constexpr int NU = (ROWS * UPR + 63) / 64;       // 16 B loads per lane per row block
 };
 
-template <int FMT, int XPT, int D, int XK>
+template <int FMT, int XPT, int D, int XK, bool RES>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const float* __restrict__ x, uint32_t cols,
                                                           uint32_t total_blocks, uint32_t S, uint32_t TEAMS,
                                                           XPrologue pro) {
@@ -1381,6 +1387,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
         stash(u[d]);
         const uint32_t row0 = row0s[d];
         const int ti = tis[d];
+        float rv = 0.0f;  // the residual, ahead of the next block's weights (loads retire in order)
+        if constexpr (RES)
+            if (slice == 0 && lane < G::ROWS) rv = pro.res[min(row0 + lane, tt.t[ti].rows - 1)];
         const uint32_t nblk = blk + uint32_t(D) * gridDim.x;
         if (nblk < total_blocks) {
             locate(nblk, row0s[d], tis[d]);
@@ -1458,7 +1467,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
             for (uint32_t s2 = 0; s2 < 16; ++s2)
                 if (s2 < S) s += ((w[s2].x + w[s2].y) + w[s2].z) + w[s2].w;
             const GemvTask& t = tt.t[ti];
-            if (row0 + lane < t.rows) t.y[row0 + lane] = nan_out ? __builtin_nanf("") : s;
+            if (nan_out) s = __builtin_nanf("");
+            if constexpr (RES) s = rv + s;
+            if (row0 + lane < t.rows) t.y[row0 + lane] = s;
         }
         parity ^= 1;
         blk += gridDim.x;
@@ -1529,7 +1540,7 @@ int cu_count() {
 // Workgroups per CU of the x-in-registers kernel.
 constexpr int kXregWgPerCu = 4;
 
-template <int FMT, int R, int S, int NW, int D, int XK = kXPlain, int EP = 0>
+template <int FMT, int R, int S, int NW, int D, int XK = kXPlain, int EP = 0, bool RES = false>
 hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
                          const XPrologue& pro = XPrologue{}) {
     constexpr uint32_t RB = (NW / S) * R;
@@ -1557,14 +1568,14 @@ hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream
         if (i < nkeys) {
             resident = vals[i];
         } else {
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, gemv_stream_kernel<FMT, R, S, NW, D, XK, EP>,
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES>,
                                                              NW * 64, lds) != hipSuccess || resident < 1)
                 resident = 1;
             if (nkeys < 8) keys[nkeys] = lds, vals[nkeys++] = resident;
         }
     }
     const uint32_t grid = std::min<uint32_t>(blocks, uint32_t(cu_count() * resident));
-    hipLaunchKernelGGL((gemv_stream_kernel<FMT, R, S, NW, D, XK, EP>), dim3(grid), dim3(NW * 64), lds, stream, tt, x,
+    hipLaunchKernelGGL((gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES>), dim3(grid), dim3(NW * 64), lds, stream, tt, x,
                        cols, blocks, pro);
     return hipGetLastError();
 }
@@ -1573,25 +1584,27 @@ hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream
 // (8 waves x 2-3 blocks, 16 waves x 2 blocks) measured slower.  Outputs of at
 // most 2048 rows with one slice per row take 8-wave workgroups, two per CU
 // (Q8_0 1024x4096: 4.9 -> 4.5 us; 4096x4096 was slower: 5.9 -> 6.5 us).
-template <int FMT, int S>
-hipError_t launch_stream_r(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream) {
+template <int FMT, int S, bool RES>
+hipError_t launch_stream_r(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
+                           const XPrologue& pro) {
     (void)R;
     uint32_t rows = 0;
     for (int i = 0; i < tt.count; ++i) rows += tt.t[i].rows;
-    if (S == 1 && rows <= 2048) return launch_stream<FMT, 1, S, 8, 1>(tt, x, cols, stream);
-    return launch_stream<FMT, 1, S, 16, 1>(tt, x, cols, stream);
+    if (S == 1 && rows <= 2048) return launch_stream<FMT, 1, S, 8, 1, kXPlain, 0, RES>(tt, x, cols, stream, pro);
+    return launch_stream<FMT, 1, S, 16, 1, kXPlain, 0, RES>(tt, x, cols, stream, pro);
 }
-template <int FMT>
-hipError_t launch_stream_any(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream) {
+template <int FMT, bool RES>
+hipError_t launch_stream_any(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
+                             const XPrologue& pro = XPrologue{}) {
     const uint32_t pairs = cols >> 6;
-    if (pairs <= 64) return launch_stream_r<FMT, 1>(R, tt, x, cols, stream);
-    if (pairs <= 128) return launch_stream_r<FMT, 2>(R, tt, x, cols, stream);
-    return launch_stream_r<FMT, 4>(R, tt, x, cols, stream);
+    if (pairs <= 64) return launch_stream_r<FMT, 1, RES>(R, tt, x, cols, stream, pro);
+    if (pairs <= 128) return launch_stream_r<FMT, 2, RES>(R, tt, x, cols, stream, pro);
+    return launch_stream_r<FMT, 4, RES>(R, tt, x, cols, stream, pro);
 }
 
 // The MFMA streaming GEMV (gemv_mfma_kernel): S slices of 16 pairs per row,
 // TEAMS = 16 / S teams, one workgroup per CU.
-template <int FMT, int XK = kXPlain>
+template <int FMT, int XK = kXPlain, bool RES = false>
 hipError_t launch_mfma(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
                        const XPrologue& pro = XPrologue{}) {
     using G = MfmaGeo<FMT>;
@@ -1612,7 +1625,7 @@ hipError_t launch_mfma(TaskTable& tt, const float* x, uint32_t cols, hipStream_t
     const uint32_t grid = std::min<uint32_t>(blocks, uint32_t(cu_count()));
     const uint32_t xpt = (S * kMfmaPairs * 16 + NW * 64 - 1) / (NW * 64);  // float4 per thread, padded pairs included
 #define ZQ_MFMA_LAUNCH(XPT)                                                                                        \
-    hipLaunchKernelGGL((gemv_mfma_kernel<FMT, XPT, 1, XK>), dim3(grid), dim3(NW * 64), lds, stream, tt, x, cols, \
+    hipLaunchKernelGGL((gemv_mfma_kernel<FMT, XPT, 1, XK, RES>), dim3(grid), dim3(NW * 64), lds, stream, tt, x, cols, \
                        blocks, S, TEAMS, pro)
     if (xpt <= 1) ZQ_MFMA_LAUNCH(1);
     else if (xpt <= 2) ZQ_MFMA_LAUNCH(2);
@@ -1808,6 +1821,20 @@ hipError_t launch_blocks(TaskTable& tt, const float* x, uint32_t cols, hipStream
 
 int device_cu_count() { return cu_count(); }
 
+namespace {
+// Q8_0 / Q4_0 with cols % 256 == 0, cols <= 16384 and 16-byte aligned
+// operands; with RES, y = pro.res + W . x.
+template <int FMT, bool RES>
+hipError_t launch_streamed(TaskTable& tt, const float* x, uint32_t c, uint32_t total_rows, const XPrologue& pro,
+                           hipStream_t stream) {
+    if (mfma_gemv_for(FMT, c, total_rows)) {
+        const hipError_t e = launch_mfma<FMT, kXPlain, RES>(tt, x, c, stream, pro);
+        if (e != hipErrorInvalidConfiguration) return e;
+    }
+    return launch_stream_any<FMT, RES>(xreg_rows(total_rows), tt, x, c, stream, pro);
+}
+}  // namespace
+
 hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x, size_t cols,
                        hipStream_t stream) {
     if (count < 1 || count > kMaxTasks || !x || !row_bytes(fmt, cols) || cols > (1u << 24))
@@ -1859,12 +1886,8 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
     bool w16 = true;
     for (int i = 0; i < count; ++i) w16 = w16 && (reinterpret_cast<uintptr_t>(tasks[i].w) & 15u) == 0;
     if (w16 && x16 && c % 256 == 0 && c / 64 <= 256) {
-        if (mfma_gemv_for(fmt, c, total_rows)) {
-            const hipError_t e = fmt == kQ8_0 ? launch_mfma<kQ8_0>(tt, x, c, stream) : launch_mfma<kQ4_0>(tt, x, c, stream);
-            if (e != hipErrorInvalidConfiguration) return e;
-        }
-        const int Rx = xreg_rows(total_rows);
-        return fmt == kQ8_0 ? launch_stream_any<kQ8_0>(Rx, tt, x, c, stream) : launch_stream_any<kQ4_0>(Rx, tt, x, c, stream);
+        return fmt == kQ8_0 ? launch_streamed<kQ8_0, false>(tt, x, c, total_rows, XPrologue{}, stream)
+                            : launch_streamed<kQ4_0, false>(tt, x, c, total_rows, XPrologue{}, stream);
     }
     if (aligned && x16 && c % 64 == 0 && c / 64 <= 256) {
         const int Rx = xreg_rows(total_rows);
@@ -1884,12 +1907,12 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
 
 
 namespace {
-template <int FMT, int XK>
+template <int FMT, int XK, bool RES = false>
 hipError_t launch_prologue_s(TaskTable& tt, uint32_t cols, const XPrologue& pro, hipStream_t stream) {
     const uint32_t pairs = cols >> 6;
-    if (pairs <= 64) return launch_stream<FMT, 1, 1, 16, 1, XK>(tt, nullptr, cols, stream, pro);
-    if (pairs <= 128) return launch_stream<FMT, 1, 2, 16, 1, XK>(tt, nullptr, cols, stream, pro);
-    return launch_stream<FMT, 1, 4, 16, 1, XK>(tt, nullptr, cols, stream, pro);
+    if (pairs <= 64) return launch_stream<FMT, 1, 1, 16, 1, XK, 0, RES>(tt, nullptr, cols, stream, pro);
+    if (pairs <= 128) return launch_stream<FMT, 1, 2, 16, 1, XK, 0, RES>(tt, nullptr, cols, stream, pro);
+    return launch_stream<FMT, 1, 4, 16, 1, XK, 0, RES>(tt, nullptr, cols, stream, pro);
 }
 }  // namespace
 
@@ -1899,7 +1922,7 @@ hipError_t launch_gemv_prologue(int fmt, const GemvTask* tasks, int count, const
     if ((fmt != kQ8_0 && fmt != kQ4_0) || cols % 256 || cols / 64 > 256) return hipErrorInvalidConfiguration;
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (!a16(pro.a) || !a16(pro.b) || !a16(pro.w) || !a16(pro.r_out)) return hipErrorInvalidConfiguration;
-    if ((pro.kind == kSiluMul && !pro.b) || (pro.kind == kAddNorm && !pro.w) ||
+    if ((pro.kind == kSiluMul && !pro.b) || (pro.kind == kAddNorm && (!pro.w || pro.res)) || (pro.res && count != 1) ||
         (pro.kind != kSiluMul && pro.kind != kAddNorm))
         return hipErrorInvalidValue;
     TaskTable tt{};
@@ -1912,7 +1935,7 @@ hipError_t launch_gemv_prologue(int fmt, const GemvTask* tasks, int count, const
     const uint32_t c = static_cast<uint32_t>(cols);
     uint32_t total_rows = 0;
     for (int i = 0; i < count; ++i) total_rows += tasks[i].rows;
-    if (mfma_gemv_for(fmt, c, total_rows, pro.kind)) {
+    if (mfma_gemv_for(fmt, c, total_rows, pro.kind) && !pro.res) {
         hipError_t e;
         if (pro.kind == kSiluMul)
             e = fmt == kQ8_0 ? launch_mfma<kQ8_0, kSiluMul>(tt, nullptr, c, stream, pro)
@@ -1922,11 +1945,29 @@ hipError_t launch_gemv_prologue(int fmt, const GemvTask* tasks, int count, const
                              : launch_mfma<kQ4_0, kAddNorm>(tt, nullptr, c, stream, pro);
         if (e != hipErrorInvalidConfiguration) return e;
     }
+    if (pro.kind == kSiluMul && pro.res)
+        return fmt == kQ8_0 ? launch_prologue_s<kQ8_0, kSiluMul, true>(tt, c, pro, stream)
+                            : launch_prologue_s<kQ4_0, kSiluMul, true>(tt, c, pro, stream);
     if (pro.kind == kSiluMul)
         return fmt == kQ8_0 ? launch_prologue_s<kQ8_0, kSiluMul>(tt, c, pro, stream)
                             : launch_prologue_s<kQ4_0, kSiluMul>(tt, c, pro, stream);
     return fmt == kQ8_0 ? launch_prologue_s<kQ8_0, kAddNorm>(tt, c, pro, stream)
                         : launch_prologue_s<kQ4_0, kAddNorm>(tt, c, pro, stream);
+}
+
+hipError_t launch_gemv_add(int fmt, const GemvTask& task, const float* x, const float* res, size_t cols,
+                           hipStream_t stream) {
+    if (!x || !res || !row_bytes(fmt, cols) || !task.w || !task.y || !task.rows) return hipErrorInvalidValue;
+    if ((fmt != kQ8_0 && fmt != kQ4_0) || cols % 256 || cols / 64 > 256) return hipErrorInvalidConfiguration;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(task.w)) & 15u) return hipErrorInvalidConfiguration;
+    TaskTable tt{};
+    tt.count = 1;
+    tt.t[0] = task;
+    XPrologue pro{};
+    pro.res = res;
+    const uint32_t c = static_cast<uint32_t>(cols);
+    return fmt == kQ8_0 ? launch_streamed<kQ8_0, true>(tt, x, c, task.rows, pro, stream)
+                        : launch_streamed<kQ4_0, true>(tt, x, c, task.rows, pro, stream);
 }
 
 hipError_t launch_gemv_prologue_silu_pair(int fmt, const GemvTask& gate, const GemvTask& up, const XPrologue& pro,
@@ -1937,7 +1978,7 @@ hipError_t launch_gemv_prologue_silu_pair(int fmt, const GemvTask& gate, const G
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (!a16(pro.a) || !a16(pro.b) || !a16(pro.w) || !a16(pro.r_out) || !a16(gate.w) || !a16(up.w))
         return hipErrorInvalidConfiguration;
-    if (pro.kind != kAddNorm || !pro.w) return hipErrorInvalidValue;
+    if (pro.kind != kAddNorm || !pro.w || pro.res) return hipErrorInvalidValue;
     TaskTable tt{};
     tt.count = 2;
     tt.t[0] = gate;

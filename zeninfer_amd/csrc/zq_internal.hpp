@@ -30,6 +30,8 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
 //   kAddNorm   v = a + b (b may be null), x = rmsnorm(v) * w as
 //              launch_add_rmsnorm; r_out (may be null) receives v, written by
 //              workgroup 0 only, so it must not alias a or b.
+// and, without kAddNorm, the residual add that follows a projection: with res,
+// y[i] = res[i] + W_i . x (one task; res may be y).
 struct XPrologue {
     int kind;
     const float* a;
@@ -37,6 +39,7 @@ struct XPrologue {
     const float* w;
     float* r_out;
     float eps;
+    const float* res = nullptr;
 };
 constexpr int kXPlain = 0, kSiluMul = 1, kAddNorm = 2;
 // Q8_0 / Q4_0 only, on the streaming kernel's shapes (cols % 256 == 0,
@@ -45,6 +48,11 @@ constexpr int kXPlain = 0, kSiluMul = 1, kAddNorm = 2;
 // kernels instead.
 hipError_t launch_gemv_prologue(int fmt, const GemvTask* tasks, int count, const XPrologue& pro, size_t cols,
                                 hipStream_t stream);
+// y = res + W . x: the streaming kernel launch_gemv takes for the shape, so
+// the sums are its sums, with the add in its store.  Coverage as
+// launch_gemv_prologue's.
+hipError_t launch_gemv_add(int fmt, const GemvTask& task, const float* x, const float* res, size_t cols,
+                           hipStream_t stream);
 // gate|up with the add+RMSNorm prologue that stores f = silu(gate.x) *
 // (up.x) into gate.y (up.y unused): Q8_0 / Q4_0, cols % 256 == 0 and
 // cols <= 4096, equal rows; hipErrorInvalidConfiguration otherwise.
