@@ -33,11 +33,11 @@
 // of a super-block: 3 data dwords (ql low/high streams and qh), 4 int8
 // sub-scales and d.  The four 4-element groups are decoded byte-parallel:
 // q = lo4 | hi2 << 4, then ((q ^ 0x20) << 2) is 4*(q-32) as a signed byte.
-// The streaming Q6_K kernel (cols % 2048 == 0) instead gives each lane 16
+// The streaming Q6_K kernel (16 B aligned weights) instead gives each lane 16
 // consecutive elements of one quarter (one sub-block scale), builds the
-// 6-bit codes four per dword and converts each with one v_cvt_f32_ubyteN,
-// the code offset applied once per unit through a precomputed sum of x; see
-// gemv_q6k_stream_kernel.
+// 6-bit codes four per dword and converts each with one instruction (for rows
+// of whole chunks v_cvt_f32_ubyteN, the code offset applied once per unit
+// through a precomputed sum of x); see gemv_q6k_stream_kernel.
 #include "zq_device.hpp"
 #include "zq_internal.hpp"
 #include "zq_pairs.hpp"
@@ -278,36 +278,47 @@ __global__ __launch_bounds__(kThreads) void gemv_xreg_kernel(TaskTable tt, const
 // up rows, and the block stores f = silu(gate.x) * (up.x) into the first
 // task's y (the expression of silu_mul_kernel), so the down projection reads
 // f as a plain vector.
-template <int FMT, int R, int S, int NW, int D, int XK, int EP = 0, bool RES = false>
+// RAG is the form for rows of any number of blocks (cols % 256 != 0): the row
+// starts at any even byte, so it is fetched from the 16 B unit that holds its
+// start (at the matrix's end up to 14 bytes of the tail pad come with it), and a
+// lane reads its pair `sh` bytes further on, one dword more and each through
+// v_alignbyte.  An odd last block is a pair whose second half is x = 0, scale 0.
+// The pairs are decoded as the kernels of those rows do (for Q4_0 without the
+// nibble sum's offset, whose cancellation doubles the error).  Q4_0, 20000 rows:
+// 2080 columns 29.2 -> 13.5 us, 11040 121 -> 48.7, 14400 62.4 -> 48.8.
+template <int FMT, int R, int S, int NW, int D, int XK, int EP = 0, bool RES = false, bool RAG = false>
 __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, const float* __restrict__ x,
                                                                uint32_t cols, uint32_t total_blocks, XPrologue pro) {
+    static_assert(!RAG || (XK == kXPlain && EP == 0 && !RES));
     static_assert(!RES || (XK != kAddNorm && EP == 0));
     static_assert(EP == 0 || (S == 1 && R == 1 && NW == 16), "the SiLU pair epilogue takes one row per wave");
     constexpr int DW = FMT == kQ8_0 ? 17 : 9;
     constexpr int NT = NW * 64;
     constexpr int TEAMS = NW / S;
-    constexpr int UMAX = 64 * DW / 4;        // 16 B units of a full 64-pair slice-row
+    constexpr int UMAX = 64 * DW / 4 + RAG;  // 16 B units of a full 64-pair slice-row (one more from a shifted start)
     constexpr int NU = (UMAX + 63) / 64;     // dwordx4 loads per lane per row
-    constexpr int WBUF = 64 * DW;            // dwords per slice-row buffer
+    constexpr int WBUF = 4 * UMAX;           // dwords per slice-row buffer
     constexpr bool XLDS = S == 1 || NW > S;  // teams share the x slices: stage x once per workgroup
     constexpr int XPT = XLDS ? (S * 1024 + NT - 1) / NT : 16;  // float4 of x per thread (cols <= S * 4096)
     extern __shared__ uint32_t lds[];        // [waves][R][WBUF]; the padded x is staged over it first
     __shared__ float red[2][NW][R];
-    const uint32_t pairs = cols >> 6;
+    const uint32_t pairs = (cols + 63) >> 6;
     const uint32_t W = min(64u, (((pairs + S - 1) / S) + 3u) & ~3u);
-    const uint32_t rb = pairs * DW * 4;
+    const uint32_t rb = (cols >> 5) * DW * 2;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int team = wave / S, slice = wave % S;
     const uint32_t p0 = slice * W;
-    const uint32_t np = p0 < pairs ? min(W, pairs - p0) : 0u;   // pairs in this wave's slice (multiple of 4)
+    const uint32_t np = p0 < pairs ? min(W, pairs - p0) : 0u;   // pairs in this wave's slice (multiple of 4, but RAG)
     const uint32_t nunits = np * DW / 4;
+    const uint32_t nbytes = np ? min(np * DW * 4, rb - p0 * DW * 4) : 0u;  // RAG: of the slice of a row
     const bool active = uint32_t(lane) < np;
     const uint32_t p = p0 + lane;
     uint32_t* buf = lds + wave * (R * WBUF);
     float* xs = reinterpret_cast<float*>(lds);
 
-    auto locate = [&](uint32_t blk, const uint8_t*(&rowp)[R], uint32_t& row0, int& ti) {
+    // RAG: rowp is the unit that holds the slice's start, sh the start in it
+    auto locate = [&](uint32_t blk, const uint8_t*(&rowp)[R], uint32_t (&sh)[R], uint32_t& row0, int& ti) {
         if constexpr (EP == 1) {
             ti = team >> 3;
             row0 = blk * 8 + (team & 7);
@@ -317,14 +328,18 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
         }
         const GemvTask& t = tt.t[ti];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            rowp[r] = t.w + (size_t)min(row0 + r, t.rows - 1) * rb + (size_t)(np ? p0 : 0) * DW * 4;
+        for (int r = 0; r < R; ++r) {
+            size_t off = (size_t)min(row0 + r, t.rows - 1) * rb + (size_t)(np ? p0 : 0) * DW * 4;
+            sh[r] = RAG ? uint32_t(off) & 15u : 0u;
+            if constexpr (RAG) off -= sh[r];
+            rowp[r] = t.w + off;
+        }
     };
     // units past the slice read 0 without a memory request
-    auto load = [&](const uint8_t*(&rowp)[R], uint4 (&u)[R][NU]) {
+    auto load = [&](const uint8_t*(&rowp)[R], const uint32_t (&sh)[R], uint4 (&u)[R][NU]) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const __amdgpu_buffer_rsrc_t rs = span_rsrc(rowp[r], nunits * 16);
+            const __amdgpu_buffer_rsrc_t rs = span_rsrc(rowp[r], !RAG ? nunits * 16 : np ? (sh[r] + nbytes + 15) & ~15u : 0u);
 #pragma unroll
             for (int i = 0; i < NU; ++i) u[r][i] = span_load16(rs, uint32_t(lane + 64 * i) * 16);
         }
@@ -356,21 +371,21 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                 xw[k] = reinterpret_cast<const float4*>(pro.w)[idx];
             }
         } else {
-            xr[k] = x4[(active ? p : 0u) * 16 + k];
+            xr[k] = x4[RAG ? min((active ? p : 0u) * 16 + k, nx4 - 1) : (active ? p : 0u) * 16 + k];
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the x loads ahead of the weight loads
     // D row blocks in flight
     uint32_t blk = blockIdx.x;
     uint4 u[D][R][NU];
-    uint32_t row0s[D];
+    uint32_t row0s[D], shs[D][R];
     int tis[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {  // branch-free, so the x loads stay first: a slot past the end re-reads the last block
         const uint32_t b = min(blk + uint32_t(d) * gridDim.x, total_blocks - 1);
         const uint8_t* rowp[R];
-        locate(b, rowp, row0s[d], tis[d]);
-        load(rowp, u[d]);
+        locate(b, rowp, shs[d], row0s[d], tis[d]);
+        load(rowp, shs[d], u[d]);
     }
     float xv[64];
     if constexpr (XK == kSiluMul) {
@@ -429,8 +444,14 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
             xv[4 * i] = xr[i].x; xv[4 * i + 1] = xr[i].y; xv[4 * i + 2] = xr[i].z; xv[4 * i + 3] = xr[i].w;
         }
     }
+    const bool half = RAG && active && (p << 1) + 1 >= (cols >> 5);  // the pair's second block is past the row
+    if constexpr (RAG) {
+#pragma unroll
+        for (int i = 0; i < 64; ++i)
+            if (!active || (i >= 32 && half)) xv[i] = 0.0f;
+    }
     float sx0 = 0.0f, sx1 = 0.0f;  // Q4_0: sum of x over the lane's two blocks
-    if constexpr (FMT == kQ4_0) {
+    if constexpr (FMT == kQ4_0 && !RAG) {
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
             sx0 += xv[i];
@@ -447,6 +468,9 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                 stash(u[d]);
                 const uint32_t row0 = row0s[d];
                 const int ti = tis[d];
+                uint32_t sh[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) sh[r] = shs[d][r];
                 // the residual ahead of the next block's weights: loads
                 // retire in order, so behind them its use would wait for them
                 float rv = 0.0f;
@@ -455,16 +479,26 @@ __global__ __launch_bounds__(NW * 64) void gemv_stream_kernel(TaskTable tt, cons
                 const uint32_t nblk = blk + uint32_t(D) * gridDim.x;
                 if (nblk < total_blocks) {
                     const uint8_t* rowp[R];
-                    locate(nblk, rowp, row0s[d], tis[d]);
-                    load(rowp, u[d]);
+                    locate(nblk, rowp, shs[d], row0s[d], tis[d]);
+                    load(rowp, shs[d], u[d]);
                 }
                 float acc[R];
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     uint32_t q[DW];
 #pragma unroll
-                    for (int j = 0; j < DW; ++j) q[j] = active ? buf[r * WBUF + DW * lane + j] : 0u;
+                    for (int j = 0; j < DW; ++j) {
+                        if constexpr (RAG) {
+                            const uint32_t* b = buf + r * WBUF + (sh[r] >> 2) + DW * lane;
+                            q[j] = active ? __builtin_amdgcn_alignbyte(b[j + 1], b[j], sh[r] & 2u) : 0u;
+                        } else {
+                            q[j] = active ? buf[r * WBUF + DW * lane + j] : 0u;
+                        }
+                    }
+                    if constexpr (RAG)
+                        if (half) q[DW / 2] &= 0xffffu;  // its scale
                     if constexpr (FMT == kQ8_0) acc[r] = q8_pair_dot(q, xv);
+                    else if constexpr (RAG) acc[r] = q4_pair_dot(q, xv);
                     else acc[r] = q4_pair_dot_mix(q, xv, sx0, sx1);
                     acc[r] = wave_sum(acc[r]);
                 }
@@ -577,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void gemv_q6k_kernel(TaskTable tt, const 
     }
 }
 
-// Q6_K streaming kernel (cols % 2048 == 0, 16 B aligned rows).  A row is cut
+// Q6_K streaming kernel (cols <= 16384, 16 B aligned weights).  A row is cut
 // into chunks of 8 super-blocks (1680 B, a multiple of 16 B); a team of S =
 // chunks-per-row waves covers a row, wave s owning chunk s, so each lane's x
 // values (two 16-element units: 32 floats) stay in VGPRs for the whole
@@ -587,13 +621,21 @@ __global__ __launch_bounds__(kThreads) void gemv_q6k_kernel(TaskTable tt, const 
 // from LDS.  Fields of odd super-blocks sit at 2 mod 4 and are assembled
 // with v_alignbyte.  PAIR as in the K-quant streaming kernel below: gate
 // row i and up row i per team, silu(gate_i) * up_i stored into gate's y.
-template <int R, int S, int NW, bool PAIR = false>
+// RAG is the form for rows of any number of super-blocks: the row starts at any
+// even byte, so it is fetched from the 16 B unit that holds its start (at the
+// matrix's end up to 14 bytes of the tail pad come with it) and read back
+// `sh` bytes further on, every field through v_alignbyte; the last slice has
+// fewer super-blocks, and the lanes past them hold x = 0 and read zeros.
+// 20000 rows: cols 2816 58.8 -> 18.6 us, 5120 96.6 -> 30.1, 11008 228 -> 57.0,
+// 15104 393 -> 62.3 against the wave-per-row kernel, which fetches in pieces of
+// 4 bytes; whole chunks keep the form without the shift (4096: 17.3 us).
+template <int R, int S, int NW, bool PAIR = false, bool RAG = false>
 __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, const float* __restrict__ x,
                                                                  uint32_t cols, uint32_t total_blocks) {
     constexpr int TEAMS = NW / S;
     static_assert(!PAIR || R == 2, "a pair step holds one gate row and one up row");
     constexpr uint32_t CHUNK = 8 * 210;                  // bytes
-    constexpr uint32_t CUNITS = CHUNK / 16;              // 105 dwordx4 units
+    constexpr uint32_t CUNITS = CHUNK / 16 + RAG;        // 105 dwordx4 units, one more from a shifted start
     constexpr uint32_t BUFW = CHUNK / 4 + 4;             // dwords per row buffer (+pad for alignbyte reads)
     extern __shared__ uint32_t lds[];                    // [waves][R][BUFW]
     __shared__ float red[2][NW][R];
@@ -602,6 +644,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int team = wave / S, slice = wave % S;
     uint32_t* wbuf = lds + wave * (R * BUFW);
+    const uint32_t nsb = RAG ? min(8u, (cols >> 8) - slice * 8) : 8u;  // super-blocks of this slice
 
     // A lane's unit k (two per lane) is 16 consecutive elements of one
     // quarter, so one sub-block scale covers it: super-block 2*(lane/16) + k
@@ -615,19 +658,24 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
     for (int k = 0; k < 2; ++k) {
         const uint32_t sb = slice * 8 + ((uint32_t(lane) >> 4) << 1) + k, h = (lane >> 3) & 1u, q = (lane >> 1) & 3u,
                        l0 = (lane & 1u) * 16u;
-        const float4* xp = reinterpret_cast<const float4*>(x + sb * 256 + h * 128 + q * 32 + l0);
+        const bool in = !RAG || sb < slice * 8 + nsb;
+        const float4* xp = reinterpret_cast<const float4*>(x + (in ? sb * 256 + h * 128 + q * 32 + l0 : 0u));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float4 v = xp[i];
+            float4 v = xp[i];
+            if (!in) v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             xv[k][4 * i] = v.x; xv[k][4 * i + 1] = v.y; xv[k][4 * i + 2] = v.z; xv[k][4 * i + 3] = v.w;
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    auto locate = [&](uint32_t blk, const uint8_t*(&rowp)[R], uint32_t& row0, int& ti) {
+    // RAG: rowp is the unit that holds the row's start, sh the start in it
+    auto locate = [&](uint32_t blk, const uint8_t*(&rowp)[R], uint32_t (&sh)[R], uint32_t& row0, int& ti) {
         if constexpr (PAIR) {
             ti = 0;
             row0 = blk * TEAMS + team;
-            const size_t off = (size_t)min(row0, tt.t[0].rows - 1) * rb + (size_t)slice * CHUNK;
+            size_t off = (size_t)min(row0, tt.t[0].rows - 1) * rb + (size_t)slice * CHUNK;
+            sh[0] = sh[1] = RAG ? uint32_t(off) & 15u : 0u;
+            off -= sh[0];
             rowp[0] = tt.t[0].w + off;
             rowp[1] = tt.t[1].w + off;
             return;
@@ -636,13 +684,17 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
         const GemvTask& t = tt.t[ti];
         row0 = (blk - tt.group_start[ti]) * (TEAMS * R) + team * R;
 #pragma unroll
-        for (int r = 0; r < R; ++r) rowp[r] = t.w + (size_t)min(row0 + r, t.rows - 1) * rb + (size_t)slice * CHUNK;
+        for (int r = 0; r < R; ++r) {
+            const size_t off = (size_t)min(row0 + r, t.rows - 1) * rb + (size_t)slice * CHUNK;
+            sh[r] = RAG ? uint32_t(off) & 15u : 0u;
+            rowp[r] = t.w + (off - sh[r]);
+        }
     };
-    // the second unit of lanes past the chunk reads 0 without a memory request
-    auto load = [&](const uint8_t*(&rowp)[R], uint4 (&u)[R][2]) {
+    // the units of lanes past the chunk read 0 without a memory request
+    auto load = [&](const uint8_t*(&rowp)[R], const uint32_t (&sh)[R], uint4 (&u)[R][2]) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const __amdgpu_buffer_rsrc_t rs = span_rsrc(rowp[r], CUNITS * 16);
+            const __amdgpu_buffer_rsrc_t rs = span_rsrc(rowp[r], RAG ? (sh[r] + nsb * 210 + 15) & ~15u : CUNITS * 16);
             u[r][0] = span_load16(rs, uint32_t(lane) * 16);
             u[r][1] = span_load16(rs, uint32_t(lane + 64) * 16);
         }
@@ -650,16 +702,17 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
 
     uint32_t blk = blockIdx.x;
     uint4 u[R][2];
+    uint32_t sh[R];
     uint32_t row0 = 0;
     int ti = 0;
     {
         const uint8_t* rowp[R];
-        locate(min(blk, total_blocks - 1), rowp, row0, ti);
-        load(rowp, u);
+        locate(min(blk, total_blocks - 1), rowp, sh, row0, ti);
+        load(rowp, sh, u);
     }
-    float nsx[2];  // -32 * sum of x over each of the lane's two units
+    float nsx[2] = {0.0f, 0.0f};  // -32 * sum of x over each of the lane's two units
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+    for (int kk = 0; kk < (RAG ? 0 : 2); ++kk) {
         float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) a0 += xv[kk][i], a1 += xv[kk][i + 1];
@@ -675,10 +728,13 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
         const uint32_t nblk = blk + gridDim.x;
         const uint32_t row0c = row0;
         const int tic = ti;
+        uint32_t shc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) shc[r] = sh[r];
         if (nblk < total_blocks) {
             const uint8_t* rowp[R];
-            locate(nblk, rowp, row0, ti);
-            load(rowp, u);
+            locate(nblk, rowp, sh, row0, ti);
+            load(rowp, sh, u);
         }
         float acc[R];
 #pragma unroll
@@ -690,7 +746,13 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
             // v_alignbyte)
             auto lds16 = [&](uint32_t off, bool odd, uint32_t (&o)[4]) {
                 const uint32_t* w = buf + (off >> 2);
-                if (!odd) {
+                if constexpr (RAG) {
+                    uint32_t t5[5];
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) t5[i] = w[i];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbyte(t5[i + 1], t5[i], off & 2u);
+                } else if (!odd) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) o[i] = w[i];
                 } else {
@@ -706,7 +768,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
             for (int k = 0; k < 2; ++k) {
                 const uint32_t sbl = ((uint32_t(lane) >> 4) << 1) + k, h = (lane >> 3) & 1u, q = (lane >> 1) & 3u,
                                l0 = (lane & 1u) * 16u;
-                const uint32_t base = sbl * 210;
+                const uint32_t base = sbl * 210 + shc[r];
                 uint32_t ql[4], qh[4];
                 lds16(base + h * 64 + (q & 1u) * 32 + l0, k == 1, ql);  // low nibbles (q < 2) or high (q >= 2)
                 lds16(base + 128 + h * 32 + l0, k == 1, qh);            // 2-bit fields, quarter q at bit 2q
@@ -717,6 +779,24 @@ __global__ __launch_bounds__(NW * 64) void gemv_q6k_stream_kernel(TaskTable tt, 
                 // neighbouring bytes land outside the masks)
                 const uint32_t nrot = (q >> 1) * 4, hrot = (2 * q + 28) & 31u;
                 float t0 = 0.0f, t1 = 0.0f;
+                if constexpr (RAG) {
+                    // signed bytes 4 * (u - 32): the nibble at bits 2-5, the field at
+                    // 6-7.  No difference of sums, which in the form below takes the
+                    // error against 64 bits from 1.0e-7 of the result to 1.9e-7
+                    float t2 = 0.0f, t3 = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const uint32_t lo4 = __builtin_amdgcn_alignbit(ql[j], ql[j], (nrot + 30) & 31u);
+                        const uint32_t hi2 = __builtin_amdgcn_alignbit(qh[j], qh[j], (hrot + 30) & 31u) & 0xC0C0C0C0u;
+                        const uint32_t codes = ((lo4 & 0x3C3C3C3Cu) | hi2) ^ 0x80808080u;
+                        t0 = fmaf(sbyte(codes, 0), xv[k][4 * j], t0);
+                        t1 = fmaf(sbyte(codes, 1), xv[k][4 * j + 1], t1);
+                        t2 = fmaf(sbyte(codes, 2), xv[k][4 * j + 2], t2);
+                        t3 = fmaf(sbyte(codes, 3), xv[k][4 * j + 3], t3);
+                    }
+                    a = fmaf(0.25f * d * sc, (t0 + t1) + (t2 + t3), a);
+                    continue;
+                }
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     // the four 6-bit codes u = q + 32 of elements 4j..4j+3, one per
@@ -1126,8 +1206,9 @@ __global__ __launch_bounds__(kThreads) void gemv_kquant_generic_kernel(TaskTable
 }
 
 // ------------------------------------------------------------- generic ---
-// Lane-per-block fallback for Q8_0 / Q4_0 rows whose block count is odd or
-// whose base is not dword-aligned.  x is read from global memory.
+// Lane-per-block fallback for Q8_0 / Q4_0: weights that are not dword-aligned,
+// and rows of an odd block count that the streaming form does not take.  x is
+// read from global memory.
 template <int FMT>
 __global__ __launch_bounds__(kThreads) void gemv_block_kernel(TaskTable tt, const float* __restrict__ x,
                                                               uint32_t cols, uint32_t total_groups) {
@@ -1540,7 +1621,8 @@ int cu_count() {
 // Workgroups per CU of the x-in-registers kernel.
 constexpr int kXregWgPerCu = 4;
 
-template <int FMT, int R, int S, int NW, int D, int XK = kXPlain, int EP = 0, bool RES = false>
+template <int FMT, int R, int S, int NW, int D, int XK = kXPlain, int EP = 0, bool RES = false,
+          bool RAG = false>
 hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
                          const XPrologue& pro = XPrologue{}) {
     constexpr uint32_t RB = (NW / S) * R;
@@ -1552,8 +1634,8 @@ hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream
     }
     if (EP == 1) blocks = (tt.t[0].rows + 7) / 8;  // 8 rows of each task per block
     tt.group_start[tt.count] = blocks;
-    size_t lds = size_t(NW) * R * 64 * DW * 4;
-    if (S == 1 || NW > S) lds = std::max(lds, size_t(cols >> 6) * kPadStride * sizeof(float));
+    size_t lds = size_t(NW) * R * (64 * DW + (RAG ? 4 : 0)) * 4;
+    if (S == 1 || NW > S) lds = std::max(lds, size_t((cols + 63) >> 6) * kPadStride * sizeof(float));
     if (lds > lds_limit()) return hipErrorInvalidConfiguration;
     // workgroups per CU: one at 16 waves, else the occupancy at this LDS size
     // (it depends on cols), cached per size
@@ -1568,14 +1650,14 @@ hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream
         if (i < nkeys) {
             resident = vals[i];
         } else {
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES>,
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES, RAG>,
                                                              NW * 64, lds) != hipSuccess || resident < 1)
                 resident = 1;
             if (nkeys < 8) keys[nkeys] = lds, vals[nkeys++] = resident;
         }
     }
     const uint32_t grid = std::min<uint32_t>(blocks, uint32_t(cu_count() * resident));
-    hipLaunchKernelGGL((gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES>), dim3(grid), dim3(NW * 64), lds, stream, tt, x,
+    hipLaunchKernelGGL((gemv_stream_kernel<FMT, R, S, NW, D, XK, EP, RES, RAG>), dim3(grid), dim3(NW * 64), lds, stream, tt, x,
                        cols, blocks, pro);
     return hipGetLastError();
 }
@@ -1584,22 +1666,22 @@ hipError_t launch_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream
 // (8 waves x 2-3 blocks, 16 waves x 2 blocks) measured slower.  Outputs of at
 // most 2048 rows with one slice per row take 8-wave workgroups, two per CU
 // (Q8_0 1024x4096: 4.9 -> 4.5 us; 4096x4096 was slower: 5.9 -> 6.5 us).
-template <int FMT, int S, bool RES>
+template <int FMT, int S, bool RES, bool RAG>
 hipError_t launch_stream_r(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
                            const XPrologue& pro) {
     (void)R;
     uint32_t rows = 0;
     for (int i = 0; i < tt.count; ++i) rows += tt.t[i].rows;
-    if (S == 1 && rows <= 2048) return launch_stream<FMT, 1, S, 8, 1, kXPlain, 0, RES>(tt, x, cols, stream, pro);
-    return launch_stream<FMT, 1, S, 16, 1, kXPlain, 0, RES>(tt, x, cols, stream, pro);
+    if (S == 1 && rows <= 2048) return launch_stream<FMT, 1, S, 8, 1, kXPlain, 0, RES, RAG>(tt, x, cols, stream, pro);
+    return launch_stream<FMT, 1, S, 16, 1, kXPlain, 0, RES, RAG>(tt, x, cols, stream, pro);
 }
-template <int FMT, bool RES>
+template <int FMT, bool RES, bool RAG = false>
 hipError_t launch_stream_any(int R, TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream,
                              const XPrologue& pro = XPrologue{}) {
-    const uint32_t pairs = cols >> 6;
-    if (pairs <= 64) return launch_stream_r<FMT, 1, RES>(R, tt, x, cols, stream, pro);
-    if (pairs <= 128) return launch_stream_r<FMT, 2, RES>(R, tt, x, cols, stream, pro);
-    return launch_stream_r<FMT, 4, RES>(R, tt, x, cols, stream, pro);
+    const uint32_t pairs = (cols + 63) >> 6;
+    if (pairs <= 64) return launch_stream_r<FMT, 1, RES, RAG>(R, tt, x, cols, stream, pro);
+    if (pairs <= 128) return launch_stream_r<FMT, 2, RES, RAG>(R, tt, x, cols, stream, pro);
+    return launch_stream_r<FMT, 4, RES, RAG>(R, tt, x, cols, stream, pro);
 }
 
 // The MFMA streaming GEMV (gemv_mfma_kernel): S slices of 16 pairs per row,
@@ -1705,7 +1787,7 @@ hipError_t launch_q6k(TaskTable& tt, const float* x, uint32_t cols, hipStream_t 
                            x, cols, groups);
     return hipGetLastError();
 }
-template <int R, int S, int NW, bool PAIR = false>
+template <int R, int S, int NW, bool PAIR = false, bool RAG = false>
 hipError_t launch_q6k_stream(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream, uint32_t wg_per_cu = 1) {
     constexpr uint32_t TEAMS = NW / S;
     uint32_t blocks = 0;
@@ -1720,7 +1802,7 @@ hipError_t launch_q6k_stream(TaskTable& tt, const float* x, uint32_t cols, hipSt
     }
     const uint32_t grid = std::min<uint32_t>(blocks, uint32_t(cu_count()) * wg_per_cu);
     const size_t lds = size_t(NW) * R * (8 * 210 / 4 + 4) * 4;
-    hipLaunchKernelGGL((gemv_q6k_stream_kernel<R, S, NW, PAIR>), dim3(grid), dim3(NW * 64), lds, stream, tt, x, cols,
+    hipLaunchKernelGGL((gemv_q6k_stream_kernel<R, S, NW, PAIR, RAG>), dim3(grid), dim3(NW * 64), lds, stream, tt, x, cols,
                        blocks);
     return hipGetLastError();
 }
@@ -1728,19 +1810,24 @@ hipError_t launch_q6k_stream(TaskTable& tt, const float* x, uint32_t cols, hipSt
 // 8-wave workgroups measured faster than one 16-wave one (the per-step
 // slice reduction then synchronises 8 waves, not 16), and 2 rows per step
 // faster than 1 or 4: 14336x4096 19.6 -> 17.0 us, lm_head 96.6 -> 89.5 us.
-template <int R, bool PAIR = false>
-hipError_t launch_q6k_stream_s(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream) {
-    switch ((cols >> 8) / 8) {
-    case 1: return launch_q6k_stream<R, 1, 8, PAIR>(tt, x, cols, stream, 2);
-    case 2: return launch_q6k_stream<R, 2, 8, PAIR>(tt, x, cols, stream, 2);
-    case 3: return launch_q6k_stream<R, 3, 6, PAIR>(tt, x, cols, stream, 2);
-    case 4: return launch_q6k_stream<R, 4, 8, PAIR>(tt, x, cols, stream, 2);
-    case 5: return launch_q6k_stream<R, 5, 5, PAIR>(tt, x, cols, stream, 2);
-    case 6: return launch_q6k_stream<R, 6, 6, PAIR>(tt, x, cols, stream, 2);
-    case 7: return launch_q6k_stream<R, 7, 7, PAIR>(tt, x, cols, stream, 2);
-    case 8: return launch_q6k_stream<R, 8, 8, PAIR>(tt, x, cols, stream, 2);
+template <int R, bool PAIR, bool RAG>
+hipError_t launch_q6k_slices(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream) {
+    switch (((cols >> 8) + 7) / 8) {
+    case 1: return launch_q6k_stream<R, 1, 8, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 2: return launch_q6k_stream<R, 2, 8, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 3: return launch_q6k_stream<R, 3, 6, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 4: return launch_q6k_stream<R, 4, 8, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 5: return launch_q6k_stream<R, 5, 5, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 6: return launch_q6k_stream<R, 6, 6, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 7: return launch_q6k_stream<R, 7, 7, PAIR, RAG>(tt, x, cols, stream, 2);
+    case 8: return launch_q6k_stream<R, 8, 8, PAIR, RAG>(tt, x, cols, stream, 2);
     default: return hipErrorInvalidConfiguration;
     }
+}
+template <int R, bool PAIR = false>
+hipError_t launch_q6k_stream_s(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream) {
+    return cols % 2048 ? launch_q6k_slices<R, PAIR, true>(tt, x, cols, stream)
+                       : launch_q6k_slices<R, PAIR, false>(tt, x, cols, stream);
 }
 hipError_t launch_q6k_stream_any(TaskTable& tt, const float* x, uint32_t cols, hipStream_t stream, uint32_t total_rows) {
     return total_rows >= 4096 ? launch_q6k_stream_s<2>(tt, x, cols, stream) : launch_q6k_stream_s<1>(tt, x, cols, stream);
@@ -1872,7 +1959,7 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
         if (reinterpret_cast<uintptr_t>(x) & 15u) return hipErrorInvalidValue;
         bool w16 = true;
         for (int i = 0; i < count; ++i) w16 = w16 && (reinterpret_cast<uintptr_t>(tasks[i].w) & 15u) == 0;
-        if (w16 && c % 2048 == 0 && c / 2048 <= 8) {
+        if (w16 && c <= 16384) {
             const hipError_t e = launch_q6k_stream_any(tt, x, c, stream, total_rows);
             if (e != hipErrorInvalidConfiguration) return e;
         }
@@ -1888,6 +1975,17 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
     if (w16 && x16 && c % 256 == 0 && c / 64 <= 256) {
         return fmt == kQ8_0 ? launch_streamed<kQ8_0, false>(tt, x, c, total_rows, XPrologue{}, stream)
                             : launch_streamed<kQ4_0, false>(tt, x, c, total_rows, XPrologue{}, stream);
+    }
+    // From 704 columns the streaming form takes the rows that are not whole
+    // 16 B units.  At 20000 rows of Q8_0 against the kernels below: 480 columns
+    // 12.6 us there, 13.9 streamed; 736 14.9 / 14.0; 2080 31.9 / 15.4; 11040
+    // 140 / 59; 14400, whose pairs are dword-aligned, 84.9 / 58.6.  Under 704 a
+    // wave has little to do between the barriers of its workgroup.
+    if (w16 && x16 && c >= 704 && c <= 16384) {
+        const int Rx = xreg_rows(total_rows);
+        const hipError_t e = fmt == kQ8_0 ? launch_stream_any<kQ8_0, false, true>(Rx, tt, x, c, stream)
+                                          : launch_stream_any<kQ4_0, false, true>(Rx, tt, x, c, stream);
+        if (e != hipErrorInvalidConfiguration) return e;
     }
     if (aligned && x16 && c % 64 == 0 && c / 64 <= 256) {
         const int Rx = xreg_rows(total_rows);
@@ -1993,7 +2091,7 @@ hipError_t launch_gemv_silu_pair(int fmt, const GemvTask& gate, const GemvTask& 
     if (!x || !row_bytes(fmt, cols) || cols > (1u << 24) || !gate.w || !gate.y || !up.w || !gate.rows)
         return hipErrorInvalidValue;
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-    const bool q6k = fmt == kQ6_K && cols % 2048 == 0;  // whole 8-super-block chunks
+    const bool q6k = fmt == kQ6_K;
     if ((fmt != kQ4_K && fmt != kQ5_K && !q6k) || cols > 16384 || up.rows != gate.rows || !a16(x) || !a16(gate.w) ||
         !a16(up.w))
         return hipErrorInvalidConfiguration;

@@ -81,7 +81,7 @@ hipError_t launch_gemv_resid(int fmt, int mode, const GemvTask* tasks, int count
 bool gemv_resid_supported(int fmt, size_t cols);
 
 // gate|up over a plain x that stores f = silu(gate.x) * (up.x) into gate.y
-// (up.y unused): Q4_K / Q5_K, and Q6_K with cols % 2048 == 0; cols <= 16384,
+// (up.y unused): Q4_K / Q5_K / Q6_K; cols <= 16384,
 // equal rows, 16-byte aligned x and weights; hipErrorInvalidConfiguration
 // otherwise.
 // With rn (Q4_K / Q5_K only), x is the residual and is normalised as a
