@@ -572,11 +572,18 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
                     const h8_t sa = *reinterpret_cast<const h8_t*>(Sa + (ar + i * 32) * 32 + lh * 16);
                     part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sa, os, part[i][j], 0, 0, 0);
                     const v16f t = __builtin_amdgcn_mfma_f32_32x32x16_f16(sa, om, zero, 0, 0, 0);
+                    // One addition to acc per super-block, since its rounding is
+                    // the larger part of a long K's error; and the two products,
+                    // which largely cancel, without that of t * dm.
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(t[v], dm, acc[i][j][v]);
+                    for (int v = 0; v < 16; ++v) {
+                        const float p = t[v] * dm;
+                        acc[i][j][v] += fmaf(part[i][j][v], d, p) + fmaf(t[v], dm, -p);
+                    }
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(part[i][j][v], d, acc[i][j][v]);
                 }
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(part[i][j][v], d, acc[i][j][v]);
                 part[i][j] = zero;
             }
         }
