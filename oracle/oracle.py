@@ -21,9 +21,9 @@ _U64 = ctypes.c_uint64
 
 
 def build(reference_root="/root/reference"):
-    """Compile liboracle.so, and _ref/libzenref.so when the reference tree exists."""
+    """Compile liboracle.so, and _ref/libzenref.so when the reference tree is there (an empty folder is not)."""
     targets = ["oracle"]
-    if os.path.isdir(reference_root):
+    if os.path.exists(os.path.join(reference_root, "src", "quant.cpp")):
         targets.append("ref")
     subprocess.check_call(["make", "-s", "-C", HERE, f"REF={reference_root}", "-j8", *targets])
 
