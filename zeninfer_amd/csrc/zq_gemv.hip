@@ -1468,8 +1468,10 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
         stash(u[d]);
         const uint32_t row0 = row0s[d];
         const int ti = tis[d];
-        float rv = 0.0f;  // the residual, ahead of the next block's weights (loads retire in order)
-        if constexpr (RES)
+        // the residual, ahead of the next block's weights (loads retire in
+        // order); Q4_0's two row groups leave no register for it and read it last
+        float rv = 0.0f;
+        if constexpr (RES && FMT == kQ8_0)
             if (slice == 0 && lane < G::ROWS) rv = pro.res[min(row0 + lane, tt.t[ti].rows - 1)];
         const uint32_t nblk = blk + uint32_t(D) * gridDim.x;
         if (nblk < total_blocks) {
@@ -1549,6 +1551,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
                 if (s2 < S) s += ((w[s2].x + w[s2].y) + w[s2].z) + w[s2].w;
             const GemvTask& t = tt.t[ti];
             if (nan_out) s = __builtin_nanf("");
+            if constexpr (RES && FMT != kQ8_0) rv = pro.res[min(row0 + lane, t.rows - 1)];
             if constexpr (RES) s = rv + s;
             if (row0 + lane < t.rows) t.y[row0 + lane] = s;
         }
