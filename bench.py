@@ -61,7 +61,6 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 INT8_PEAK_TOPS = 5000.0        # MI355X dense int8 MFMA (POP/s x 1000)
-FP32_PEAK_TFLOPS = 157.3       # MI355X dense fp32 MFMA
 F16_PEAK_TFLOPS = 2500.0       # MI355X dense fp16 / bf16 MFMA
 
 HIDDEN, FFN, KV, VOCAB, LAYERS = 4096, 14336, 1024, 128256, 32
@@ -376,7 +375,7 @@ def format_sweep(torch, zq, dev):
     distinct replicas (>= 320 MB) that no launch reads from the MALL.  The
     GEMM uses each format's default activations: int8 for Q4_0, fp32 for the
     super-block formats (their only reference routes), reported against the
-    int8 or the fp32 MFMA peak.  Each GEMV is set beside the plain streaming
+    int8 or the f16 MFMA peak.  Each GEMV is set beside the plain streaming
     read of the same weight bytes (read_ceiling_us).  Also the Q8_0 GEMM M
     sweep of config 2."""
     out = {}
@@ -408,15 +407,13 @@ def format_sweep(torch, zq, dev):
             ms = timed_launches_on(torch, lambda i: zq.gemm_dev(fmt, ws[i % nrep], X[: 512 * K], Y, 512, N, K, act,
                                                                 wsp, wsb), 2 * nrep, 2)
             tops = 2.0 * 512 * N * K / (ms * 1e-3) / 1e12
-            # the MFMA each path runs on: int8; the super-block formats' split-f16
-            # products (three f16 MFMA products per multiply-add: both operands
-            # split); fp32 otherwise
+            # the MFMA each path runs on: int8, or the split activations' f16
+            # products, two per multiply-add (three for Q6_K, whose codes take two f16)
             if act == zq.ACT_INT8:
                 peak, mfma = INT8_PEAK_TOPS, "int8"
-            elif fmt in (zq.Q6_K, zq.Q4_K, zq.Q5_K):
-                peak, mfma = F16_PEAK_TFLOPS / 3.0, "f16 x3 (split operands)"
             else:
-                peak, mfma = FP32_PEAK_TFLOPS, "fp32"
+                products = 3 if fmt == zq.Q6_K else 2
+                peak, mfma = F16_PEAK_TFLOPS / products, f"f16 x{products} (split activations)"
             entry.update({"gemm_M512_ms": round(ms, 4), "gemm_M512_TOPS": round(tops, 1),
                           "gemm_act": "int8" if act == zq.ACT_INT8 else "f32", "gemm_mfma": mfma,
                           "gemm_frac_peak": round(tops / peak, 4)})

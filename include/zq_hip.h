@@ -204,7 +204,7 @@ int zq_hip_gemv_batch_dev(int fmt, const float* x, const zq_gemv_task* tasks, si
  * Q4_K, Q5_K: f16 hi + lo and row scales; they let the GEMM run on the f16
  * MFMA) and split-K partial sums for small grids, else 0 (Q8_0 / Q4_0 use
  * that room for split activations as well; a smaller or null workspace runs
- * with what fits: the fp32 MFMA, unsplit). */
+ * with what fits, down to the few-token kernel, which needs none). */
 size_t zq_hip_gemm_workspace_bytes(int fmt, size_t tokens, size_t rows, size_t cols, int act_mode);
 int zq_hip_gemm_dev(int fmt, const void* weights, const float* X, float* Y, size_t tokens, size_t rows,
                     size_t cols, int act_mode, void* workspace, size_t workspace_bytes, void* stream);

@@ -5,9 +5,10 @@
 // tokens the weights are the traffic and the launches the time, so this kernel
 // needs no activation pass, no workspace and no K planes: a workgroup takes 32
 // (or 64) tokens x 32 weight rows, its waves share the tile's K (a group
-// of 32 elements each in turn) and add their sums through LDS at the end.  Weights
-// and activations go from memory straight to the matrix core's operand
-// registers; there is no LDS and no barrier in the loop.
+// of 32 elements each in turn) and add their sums through LDS at the end.  The
+// weights go from memory straight to the matrix core's operand registers, the
+// activations through a part of LDS that belongs to the wave, in whole lines;
+// there is no barrier in the loop.
 //
 // Products: an fp32 activation is the exact sum of three bf16 values (8 + 8 +
 // 8 significant bits), a weight code is a whole number of at most 8 bits, so
@@ -15,6 +16,12 @@
 // instructions for each 16 k.  A group's sum is scaled by its fp32 scale into
 // the accumulator; the offset of Q4_K / Q5_K multiplies the group's sum of x on
 // the fp32 MFMA.
+//
+// Bound: at a few tokens the launch and the chain of a wave's K groups (loads,
+// decoding, products; 16 and 8 waves sharing K measured the same), past ~100
+// tokens the VALU work of decoding each weight again for every 64 tokens, which
+// is where the estimates in plan_gemm_skinny_f32 and plan_split cross.  Q4_K,
+// 19 tokens, 4096 + 1024 + 1024 rows x 4096: 94 us in nine launches -> 17.3 in one.
 #include "zq_device.hpp"
 #include "zq_internal.hpp"
 

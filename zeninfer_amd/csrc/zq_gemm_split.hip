@@ -8,6 +8,16 @@
 //  * the GEMM multiplies codes by hi and lo on v_mfma_f32_32x32x16_f16 (exact
 //    products, fp32 sums: two instructions where one fp32 MFMA of the same
 //    size would take sixteen) and applies the group scales in fp32.
+// Bound: the matrix cores at the chip's power limit.  With random data the clock
+// falls to ~1.5 GHz, and a loop of these MFMAs with the stage's LDS reads and
+// VALU work reaches 1.3-1.4 PF of f16 products; the kernels run at 0.8-0.9 PF.
+// A tile of 128 x 256 (128 x 128 for small grids, see plan_split) because the
+// next operand reads, the staging and the scale FMAs of a stage then just fit
+// between its MFMAs.  Measured, fp32-MFMA or three-product f16 kernel -> here:
+//   Q8_0  512 x 14336 x 4096   555 -> 151 us (108 -> 398 TFLOP/s of the GEMM)
+//   Q6_K 1000 x 14336 x 4096   534 -> 379 us; 512 tokens 0.32-0.37 -> 0.22 ms
+//   Q4_K / Q5_K 512 x 14336 x 4096   0.29-0.32 -> 0.18 / 0.30-0.34 -> 0.19 ms
+// and an error against 64 bits that is no larger in any format.
 #include "zq_device.hpp"
 #include "zq_gemm_common.hpp"
 #include "zq_internal.hpp"
