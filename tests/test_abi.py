@@ -164,3 +164,30 @@ def test_host_wrappers_reject_strided_or_short_arrays():
         zq.ffn_gemv(zq.Q8_0, w, w, w[: 10], x, rows, cols, cols)
     with pytest.raises(ValueError, match="rms_norm weight"):
         zq.rms_norm(np.zeros(2 * cols, np.float32), np.zeros(cols - 1, np.float32), 2, cols, 1e-5)
+
+
+def test_batch_wrappers_take_any_integer_row_count(monkeypatch):
+    """The device batch wrappers pass on the row counts of numpy integers (a
+    table of sizes, an array's shape arithmetic) as they do Python's, and
+    refuse a count that is no whole number."""
+    import types
+    from zeninfer_amd import zq
+    seen = []
+
+    def capture(tasks, count):
+        seen.append([(int(tasks[i].weights), int(tasks[i].rows)) for i in range(count)])
+        return zq.OK
+
+    fake = types.SimpleNamespace(
+        zq_weight_bytes=zq.lib().zq_weight_bytes,
+        zq_hip_gemv_batch_dev=lambda fmt, x, tasks, count, cols, stream: capture(tasks, count),
+        zq_hip_gemm_batch_dev=lambda fmt, X, tasks, count, *rest: capture(tasks, count))
+    monkeypatch.setattr(zq, "lib", lambda: fake)
+    table = np.array([64, 4096], np.int32)
+    for rows in ([64, 4096], [np.int64(64), np.int64(4096)], list(table), [np.uint64(64), np.uint16(4096)]):
+        tasks = [((1 + i) << 20, (8 + i) << 20, r) for i, r in enumerate(rows)]
+        zq.gemv_batch_dev(zq.Q8_0, 1 << 24, tasks, 256)
+        zq.gemm_batch_dev(zq.Q8_0, 1 << 24, tasks, 3, 256)
+    assert seen == [[(1 << 20, 64), (2 << 20, 4096)]] * len(seen)
+    with pytest.raises(TypeError):
+        zq.gemv_batch_dev(zq.Q8_0, 1 << 24, [(1 << 20, 2 << 20, 64.0)], 256)

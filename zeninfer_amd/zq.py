@@ -6,6 +6,7 @@ take numpy arrays; the *_dev calls take torch tensors (device memory and
 streams only) or raw integer device pointers.
 """
 import ctypes
+import operator
 import os
 import struct
 
@@ -410,10 +411,10 @@ _GEMM_TASKS = [GemmTask * n for n in range(MAX_BATCH + 1)]
 
 
 def _task_table(types, task, flat):
-    """ctypes array of {address, address, count} tasks from their flat values."""
+    """ctypes array of {address, address, count} tasks from their flat values (taken modulo 2^64, as ctypes does)."""
     n = len(flat) // 3
     t = types[n] if n < len(types) else task * n
-    return t.from_buffer_copy(struct.pack("=%dQ" % len(flat), *flat)) if n else t()
+    return t.from_buffer_copy(struct.pack("=%dQ" % len(flat), *[v & _U64 for v in flat])) if n else t()
 
 
 def gemv_dev(fmt, w, x, y, rows, cols, stream=None):
@@ -430,8 +431,9 @@ def gemv_batch_dev(fmt, x, tasks, cols, stream=None):
     x = _need(x, 4 * cols, "gemv_batch_dev x", dev)
     flat = []
     for w, y, r in tasks:
+        r = operator.index(r)  # numpy integers too
         flat += (_need(w, weight_bytes(fmt, r, cols), "gemv_batch_dev weights", dev) or 0,
-                 _need(y, 4 * r, "gemv_batch_dev y", dev) or 0, r & _U64)
+                 _need(y, 4 * r, "gemv_batch_dev y", dev) or 0, r)
     return check(lib().zq_hip_gemv_batch_dev(fmt, x, _task_table(_GEMV_TASKS, GemvTask, flat), len(tasks), cols,
                                              _stream(stream)), "zq_hip_gemv_batch_dev")
 
@@ -461,8 +463,9 @@ def gemm_batch_dev(fmt, X, tasks, tokens, cols, act=ACT_DEFAULT, workspace=None,
     X = _need(X, 4 * tokens * cols, "gemm_batch_dev X", dev)
     flat = []
     for w, Y, r in tasks:
+        r = operator.index(r)
         flat += (_need(w, weight_bytes(fmt, r, cols), "gemm_batch_dev weights", dev) or 0,
-                 _need(Y, 4 * tokens * r, "gemm_batch_dev Y", dev) or 0, r & _U64)
+                 _need(Y, 4 * tokens * r, "gemm_batch_dev Y", dev) or 0, r)
     workspace = _need(workspace, workspace_bytes, "gemm_batch_dev workspace", dev)
     return check(lib().zq_hip_gemm_batch_dev(fmt, X, _task_table(_GEMM_TASKS, GemmTask, flat), len(tasks), tokens, cols, act,
                                              workspace, workspace_bytes, _stream(stream)), "zq_hip_gemm_batch_dev")
