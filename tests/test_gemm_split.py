@@ -9,6 +9,8 @@ import subprocess
 import numpy as np
 import pytest
 
+torch = pytest.importorskip("torch")
+
 from oracle import oracle as O
 from tests.tolerance import assert_close
 
@@ -84,6 +86,52 @@ def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k):
                 want = Z[r, c] * W[:, c]  # the finite terms do not matter beside it
                 assert np.array_equal(got[r], want, equal_nan=True)
     zq.release(w)
+
+
+def extremes(orc, m, k):
+    """Activations with, in rows of their own, infinities (one, two of one sign,
+    two of opposite signs, every element), a NaN beside one, and magnitudes at
+    the two ends of the fp32 range."""
+    X = orc.gen_normal(531, m * k).reshape(m, k)
+    X[3, 17] = np.inf
+    X[4, 40] = -np.inf
+    X[5, [1, k - 1]] = np.inf
+    X[6, [2, 300]] = np.inf, -np.inf
+    X[7, [9, 33]] = np.inf, np.nan
+    X[8] = np.where(np.arange(k) % 2, np.inf, -np.inf)
+    X[9] *= np.float32(2.0 ** 120)
+    X[10] *= np.float32(2.0 ** -116)
+    X[11, 5] *= np.float32(2.0 ** 124)
+    return X
+
+
+def check_extremes(orc, fmt, w, X, got, m, n, k):
+    """Against the sums of products with the dequantised weights: infinite and NaN
+    where those are, with their signs, and otherwise within 16 roundings of the
+    magnitudes summed (2^-24 of them each: the products', the split's and, as a
+    random walk, the k additions')."""
+    W = orc.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
+    for r in range(m):
+        with np.errstate(invalid="ignore", over="ignore"):
+            terms = X[r].astype(np.float64) * W
+            want = terms.sum(1)
+        finite = np.isfinite(want)
+        assert np.array_equal(got[r][~finite], want[~finite].astype(np.float32), equal_nan=True), f"row {r}"
+        mag = np.abs(terms).sum(1)[finite]
+        assert np.all(np.abs(got[r][finite].astype(np.float64) - want[finite]) <= 16 * 2.0 ** -24 * mag), f"row {r}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(20, 70, 512), (50, 33, 768)])  # one and two token tiles
+@pytest.mark.parametrize("fmt", ALL)
+def test_extremes_on_few_tokens(zq, orc, fmt, m, n, k):
+    w = orc.gen_weights(fmt, 530, n, k)
+    X = extremes(orc, m, k)
+    dw = torch.zeros(zq.weight_bytes(fmt, n, k), dtype=torch.uint8, device="cuda:0")
+    dw[: w.size] = torch.from_numpy(w).to("cuda:0")
+    Y = torch.empty(m * n, device="cuda:0")
+    zq.gemm_dev(fmt, dw, torch.from_numpy(X).to("cuda:0"), Y, m, n, k, zq.ACT_F32)
+    check_extremes(orc, fmt, w, X, Y.cpu().numpy().reshape(m, n), m, n, k)
 
 
 @pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))

@@ -15,7 +15,9 @@
 // v_mfma_f32_32x32x16_bf16 gives exact products in fp32 sums, three
 // instructions for each 16 k.  A group's sum is scaled by its fp32 scale into
 // the accumulator; the offset of Q4_K / Q5_K multiplies the group's sum of x on
-// the fp32 MFMA.
+// the fp32 MFMA.  Activations for which that would not be exact (infinite, at
+// the ends of the fp32 range: needs_f32) are multiplied in fp32 by the dequantised
+// weights instead.
 //
 // Bound: at a few tokens the launch and the chain of a wave's K groups (loads,
 // decoding, products; 16 and 8 waves sharing K measured the same), past ~100
@@ -26,6 +28,7 @@
 #include "zq_internal.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace zq {
 namespace {
@@ -59,20 +62,12 @@ __device__ __forceinline__ uint32_t hi_pair(float a, float b) {
     return __builtin_amdgcn_perm(fbits(b), fbits(a), 0x07060302u);
 }
 
-// x (8 elements) as bf16 planes: p0 + p1 + p2 == x exactly.  A non-finite x
-// is p0 alone, so it reaches the sum as it would in fp32.
+// x (8 elements) as bf16 planes: p0 + p1 + p2 == x exactly, for those that
+// needs_f32() does not take.  A NaN is one in p0 or p1.
 __device__ __forceinline__ void split3(const float (&x)[8], b8_t& p0, b8_t& p1, b8_t& p2) {
     float r1[8], r2[8];
-    float top = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        top = fmaxf(top, fabsf(x[i]));
-        r1[i] = x[i] - bitsf(fbits(x[i]) & 0xffff0000u);
-    }
-    if (__any(top == __builtin_inff())) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r1[i] = fabsf(x[i]) == __builtin_inff() ? 0.0f : r1[i];
-    }
+    for (int i = 0; i < 8; ++i) r1[i] = x[i] - bitsf(fbits(x[i]) & 0xffff0000u);
 #pragma unroll
     for (int i = 0; i < 8; ++i) r2[i] = r1[i] - bitsf(fbits(r1[i]) & 0xffff0000u);
     u4_t a, b, c;
@@ -85,6 +80,18 @@ __device__ __forceinline__ void split3(const float (&x)[8], b8_t& p0, b8_t& p1, 
     p0 = __builtin_bit_cast(b8_t, a);
     p1 = __builtin_bit_cast(b8_t, b);
     p2 = __builtin_bit_cast(b8_t, c);
+}
+
+// Whether four activations need fp32 products: the largest is infinite (an
+// infinity times a centred code and times the group's offset can have opposite
+// signs where the weight's own sign decides), so large that a code times it
+// could overflow where the weight times it does not (from 2^112: 32 products
+// by codes below 2^7 stay under 2^124), or so small that its third part falls
+// below the smallest bf16 (under 2^-108, but not all 0).
+__device__ __forceinline__ bool needs_f32(f4_t x) {
+    const float top = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+    constexpr uint32_t lo = (127u - 108u) << 23, hi = (127u + 112u) << 23;
+    return fbits(top) - lo >= hi - lo && top != 0.0f;
 }
 
 // Eight signed code bytes as bf16 (|value| <= 128: exact).
@@ -144,13 +151,14 @@ __device__ __forceinline__ void load_group(const uint8_t* row, uint32_t b, uint3
         r.d = *reinterpret_cast<const uint16_t*>(p + 208);
     }
 }
-// The group's codes, its scale(s) -- per step for Q6_K -- and its offset.
+// The group's codes, its scale(s) -- per step for Q6_K --, its offset and the
+// min that the offset holds.
 template <int FMT>
 __device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, uint32_t h, b8_t (&w)[2], float (&s)[2],
-                                             float& off) {
+                                             float& off, float& min) {
     const uint32_t g = b & 7u;
     uint32_t c[4];
-    off = 0.0f;
+    off = min = 0.0f;
     if constexpr (FMT == kQ8_0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) c[i] = r.q[i];
@@ -165,7 +173,8 @@ __device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, ui
         const uint32_t sc = g < 4 ? (hd[1] >> sh) & 63u : ((hd[3] >> sh) & 15u) | ((hd[1] >> (sh + 2)) & 0x30u);
         const uint32_t mn = g < 4 ? (hd[2] >> sh) & 63u : ((hd[3] >> (sh + 4)) & 15u) | ((hd[2] >> (sh + 2)) & 0x30u);
         const float ds = half_bits_to_float(hd[0]) * float(sc);
-        off = fmaf(half_bits_to_float(hd[0] >> 16), -float(mn), (FMT == kQ4_K ? 8.0f : 16.0f) * ds);
+        min = half_bits_to_float(hd[0] >> 16) * float(mn);  // exact
+        off = (FMT == kQ4_K ? 8.0f : 16.0f) * ds - min;
         s[0] = s[1] = ds * (FMT == kQ4_K ? 0.0625f : 0.125f);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -204,15 +213,22 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t l32 = lane & 31, lh = lane >> 5;
     const uint32_t first = split * tasks.groups, end = min(K >> 5, first + tasks.groups);
-    const uint8_t* row = tasks.w[t] + size_t(min(n0 + l32, N - 1)) * row_bytes_dev(FMT, K);
     // loads cover whole lines: 8 lanes a row's 128 bytes (a lane reading its own
     // operand row touched 32 lines an instruction and bound the kernel)
-    const float* x[MT][4];
+    struct Source {
+        const uint8_t* row;
+        const float* x[MT][4];
+    };
+    auto source = [&](uint32_t lane) {
+        Source o;
+        o.row = tasks.w[t] + size_t(min(n0 + (lane & 31), N - 1)) * row_bytes_dev(FMT, K);
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            x[i][q] = X + size_t(min(m0 + 32 * i + 8 * q + (lane >> 3), M - 1)) * K + 4 * (lane & 7);
+            for (int q = 0; q < 4; ++q)
+                o.x[i][q] = X + size_t(min(m0 + 32 * i + 8 * q + (lane >> 3), M - 1)) * K + 4 * (lane & 7);
+        return o;
+    };
     float* stage = &lds[wave][0][0];
     const uint32_t st_w = (uint32_t(lane >> 3) * 8 + ((lane & 7) ^ ((lane >> 4) & 7))) * 4;  // + 8 rows: swizzle + 4 mod 8
 
@@ -229,22 +245,54 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
         Group<FMT> w;
         f4_t x[MT][4];  // [token tile][8 rows]
     };
-    auto load = [&](uint32_t b, Data& d) {
-        load_group<FMT>(row, b, lh, d.w);
+    auto load = [&](const Source& from, uint32_t b, Data& d) {
+        load_group<FMT>(from.row, b, lh, d.w);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) d.x[i][q] = *reinterpret_cast<const f4_t*>(x[i][q] + 32 * b);
+            for (int q = 0; q < 4; ++q) d.x[i][q] = *reinterpret_cast<const f4_t*>(from.x[i][q] + 32 * b);
+    };
+    // Those that need fp32 products are staged as 0, and multiplied after the
+    // loop; REST: those alone.
+    bool rest = false;
+    auto stage_x = [&](const Data& d, auto rest_c) {
+        constexpr bool REST = decltype(rest_c)::value;
+        bool f[MT][4], any = false;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) any |= f[i][q] = needs_f32(d.x[i][q]);
+        auto put = [&](int i, int q, f4_t v) {  // row 8q + lane / 8 of the tile, unit lane % 8
+            *reinterpret_cast<f4_t*>(stage + i * 1024 + q * 256 + (st_w ^ (q & 1 ? 16u : 0u))) = v;
+        };
+        const f4_t none = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (REST || __any(any)) {
+            rest = true;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) put(i, q, f[i][q] == REST ? d.x[i][q] : none);
+        } else {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) put(i, q, d.x[i][q]);
+        }
+    };
+    auto read_x = [&](int i, int s, float (&e)[8]) {
+#pragma unroll
+        for (uint32_t q = 0; q < 2; ++q) {
+            const uint32_t unit = step_k<FMT>(s, lh) / 4 + q;
+            const f4_t f = *reinterpret_cast<const f4_t*>(stage + i * 1024 + l32 * 32 + ((unit ^ ((l32 >> 1) & 7)) * 4));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[4 * q + c] = f[c];
+        }
     };
     auto multiply = [&](uint32_t b, const Data& d) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)  // row 8q + lane / 8 of the tile, unit lane % 8
-                *reinterpret_cast<f4_t*>(stage + i * 1024 + q * 256 + (st_w ^ (q & 1 ? 16u : 0u))) = d.x[i][q];
+        stage_x(d, std::false_type{});
         b8_t w[2];
-        float sc[2], off;
-        decode_group<FMT>(d.w, b, lh, w, sc, off);
+        float sc[2], off, min;
+        decode_group<FMT>(d.w, b, lh, w, sc, off, min);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             v16f p = zero;
@@ -252,13 +300,7 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
                 float e[8];
-#pragma unroll
-                for (uint32_t q = 0; q < 2; ++q) {
-                    const uint32_t unit = step_k<FMT>(s, lh) / 4 + q;
-                    const f4_t f = *reinterpret_cast<const f4_t*>(stage + i * 1024 + l32 * 32 + ((unit ^ ((l32 >> 1) & 7)) * 4));
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) e[4 * q + c] = f[c];
-                }
+                read_x(i, s, e);
                 if constexpr (kOffset<FMT>) sum += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
                 b8_t p0, p1, p2;
                 split3(e, p0, p1, p2);
@@ -275,17 +317,45 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
         }
     };
     if (first + wave < end) {
+        const Source from = source(lane);
         Data d0, d1;
-        load(first + wave, d0);
+        load(from, first + wave, d0);
         for (uint32_t b = first + wave;;) {
-            load(min(b + NW, end - 1), d1);
+            load(from, min(b + NW, end - 1), d1);
             __builtin_amdgcn_sched_barrier(0);
             multiply(b, d0);
             if ((b += NW) >= end) break;
-            load(min(b + NW, end - 1), d0);
+            load(from, min(b + NW, end - 1), d0);
             __builtin_amdgcn_sched_barrier(0);
             multiply(b, d1);
             if ((b += NW) >= end) break;
+        }
+    }
+    // the products left out above, in fp32 with the dequantised weights
+    if (rest) {
+        uint32_t l = lane;  // opaque: the addresses are formed here again, not kept through the loop above
+        asm volatile("" : "+v"(l));
+        const Source from = source(l);
+        for (uint32_t b = first + wave; b < end; b += NW) {
+            Data d;
+            load(from, b, d);
+            stage_x(d, std::true_type{});
+            b8_t w[2];
+            float sc[2], off, min;
+            decode_group<FMT>(d.w, b, lh, w, sc, off, min);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    float e[8];
+                    read_x(i, s, e);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        const float q = float(w[s][c]);
+                        const float wd = kOffset<FMT> ? fmaf(sc[s], q + 128.0f, -min) : sc[s] * q;
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(e[c], wd, acc[i], 0, 0, 0);
+                    }
+                }
         }
     }
     // the waves' sums, added in wave order (a wave's own region: no wait before)
