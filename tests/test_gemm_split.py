@@ -2,6 +2,7 @@
 zq_gemm_skinny.hip for few tokens): edges of their tiles and K splits, rows of very different magnitude, and
 non-finite activations; and, on the CPU, that its kernels neither spill nor
 use packed fp32 arithmetic."""
+import ctypes
 import os
 import re
 import subprocess
@@ -88,11 +89,16 @@ def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k):
     zq.release(w)
 
 
-def extremes(orc, m, k):
+def extremes(orc, fmt, w, m, n, k):
     """Activations with, in rows of their own, infinities (one, two of one sign,
-    two of opposite signs, every element), a NaN beside one, and magnitudes at
-    the two ends of the fp32 range."""
+    two of opposite signs, every element), a NaN beside one, magnitudes at the
+    two ends of the fp32 range, and one element far above the others, where it
+    meets most zero weights."""
     X = orc.gen_normal(531, m * k).reshape(m, k)
+    zeros = (orc.dequantize(fmt, w, n * k).reshape(n, k) == 0).sum(0).argmax()
+    X[12, zeros] = 1e8
+    X[13, zeros] = -3e12
+    X[14, zeros] = 1e5
     X[3, 17] = np.inf
     X[4, 40] = -np.inf
     X[5, [1, k - 1]] = np.inf
@@ -107,31 +113,62 @@ def extremes(orc, m, k):
 
 def check_extremes(orc, fmt, w, X, got, m, n, k):
     """Against the sums of products with the dequantised weights: infinite and NaN
-    where those are, with their signs, and otherwise within 16 roundings of the
-    magnitudes summed (2^-24 of them each: the products', the split's and, as a
-    random walk, the k additions')."""
+    where those are, with their signs, and otherwise within 8 + sqrt(k) roundings
+    of the magnitudes summed (2^-24 of them each: the products', the split's and,
+    as a random walk, those of k additions to a sum that one element can make
+    large from the start).  Q4_K / Q5_K multiply a code and its group's offset
+    apart, so there the group's largest weight counts for each."""
     W = orc.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
-    for r in range(m):
+    top = np.abs(W)
+    if fmt in (O.Q4_K, O.Q5_K):
+        top = np.repeat(top.reshape(n, k // 32, 32).max(2), 32, axis=1)
+    for r in range(min(m, 24)):
         with np.errstate(invalid="ignore", over="ignore"):
             terms = X[r].astype(np.float64) * W
             want = terms.sum(1)
         finite = np.isfinite(want)
         assert np.array_equal(got[r][~finite], want[~finite].astype(np.float32), equal_nan=True), f"row {r}"
-        mag = np.abs(terms).sum(1)[finite]
-        assert np.all(np.abs(got[r][finite].astype(np.float64) - want[finite]) <= 16 * 2.0 ** -24 * mag), f"row {r}"
+        if finite.any():
+            mag = (np.abs(X[r].astype(np.float64)) * top).sum(1)[finite]
+            err = np.abs(got[r][finite].astype(np.float64) - want[finite])
+            assert np.all(err <= (8 + k ** 0.5) * 2.0 ** -24 * mag), f"row {r}: {np.nanmax(err / mag) * 2.0 ** 24} roundings"
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(20, 70, 512), (50, 33, 768)])  # one and two token tiles
-@pytest.mark.parametrize("fmt", ALL)
-def test_extremes_on_few_tokens(zq, orc, fmt, m, n, k):
-    w = orc.gen_weights(fmt, 530, n, k)
-    X = extremes(orc, m, k)
+class SkinnyPlan(ctypes.Structure):
+    _fields_ = [("ks", ctypes.c_uint32), ("us", ctypes.c_double)]
+
+
+def takes_split(zq, fmt, m, n, k, ws_bytes):
+    """Whether the library's planners send this call to the split kernels (else
+    to the few-token kernel): the comparison launch_gemm_f32_batch makes."""
+    L, z = zq.lib(), ctypes.c_size_t
+    skinny, split = L._ZN2zq20plan_gemm_skinny_f32Eimmmm, L._ZN2zq13gemm_split_usEimmmPKvm
+    skinny.restype, skinny.argtypes = SkinnyPlan, [ctypes.c_int, z, z, z, z]
+    split.restype, split.argtypes = ctypes.c_double, [ctypes.c_int, z, z, z, ctypes.c_void_p, z]
+    use = min(ws_bytes, zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32))
+    return skinny(fmt, m, n, k, use // (m * n * 4)).us > split(fmt, m, n, k, 256 if use else None, use)
+
+
+def run_dev(zq, fmt, w, X, m, n, k, ws_bytes):
     dw = torch.zeros(zq.weight_bytes(fmt, n, k), dtype=torch.uint8, device="cuda:0")
     dw[: w.size] = torch.from_numpy(w).to("cuda:0")
-    Y = torch.empty(m * n, device="cuda:0")
-    zq.gemm_dev(fmt, dw, torch.from_numpy(X).to("cuda:0"), Y, m, n, k, zq.ACT_F32)
-    check_extremes(orc, fmt, w, X, Y.cpu().numpy().reshape(m, n), m, n, k)
+    Y = torch.full((m * n + 64,), 7.0, device="cuda:0")
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device="cuda:0")
+    zq.gemm_dev(fmt, dw, torch.from_numpy(X).to("cuda:0"), Y, m, n, k, zq.ACT_F32, ws if ws_bytes else None, ws_bytes)
+    assert bool((Y[m * n:] == 7.0).all())
+    return Y[: m * n].cpu().numpy().reshape(m, n)
+
+
+# one and two token tiles without a workspace; split activations with K splits
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,split", [(20, 70, 512, False), (50, 33, 768, False), (130, 1500, 4096, True)])
+@pytest.mark.parametrize("fmt", ALL)
+def test_extreme_activations(zq, orc, fmt, m, n, k, split):
+    w = orc.gen_weights(fmt, 530, n, k)
+    X = extremes(orc, fmt, w, m, n, k)
+    ws_bytes = zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32) if split else 0
+    assert takes_split(zq, fmt, m, n, k, ws_bytes) == split
+    check_extremes(orc, fmt, w, X, run_dev(zq, fmt, w, X, m, n, k, ws_bytes), m, n, k)
 
 
 @pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))

@@ -45,8 +45,13 @@ typedef uint32_t u4a4_t __attribute__((ext_vector_type(4), aligned(4)));
 // magnitude lies in [2^14, 2^15): out[r][block] = 32 hi halves, 32 lo halves;
 // ex[r] = e.  x - hi is exact in fp32, so hi + lo carries x to 2^-23 of
 // itself (2^-40 of the row's maximum for elements so small that lo is
-// subnormal).  A non-finite x is carried as hi alone (lo = 0), so it reaches
-// the sum as it would in fp32, and does not take part in the maximum.
+// subnormal).  A NaN reaches every output of its row.  A row with an infinity
+// (whose products with a weight's parts can have opposite signs where the
+// weight's own sign decides), or with so large a span that 2^-40 of its maximum
+// shows (a quarter of its elements 2^20 below it: a huge one that meets a zero
+// code would leave the others with less than fp32's precision), is marked
+// instead: ex[r] = kExactRow, and exact_tile() multiplies it in fp32.
+constexpr int kExactRow = 1 << 20;
 __device__ __forceinline__ float finite_abs(float v) {
     const float a = fabsf(v);
     return a < __builtin_inff() ? a : 0.0f;
@@ -72,7 +77,7 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, red[w]);
     const int e = m > 0.0f ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
-    if (threadIdx.x == 0) ex[blockIdx.x] = e;
+    float wide = 0.0f;  // > 0 for a row to mark
     _Float16* o = out + size_t(blockIdx.x) * K * 2;
     auto split = [](float f, _Float16& h, _Float16& l) {
         h = _Float16(f);
@@ -89,6 +94,8 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
             split(f[k], a, b);
             h[k] = a;
             l[k] = b;
+            const float t = fabsf(f[k]);
+            wide += t == __builtin_inff() ? 1e9f : t == 0.0f ? 0.0f : t < 0x1p-6f ? 3.0f : -1.0f;
         }
         _Float16* d = o + size_t(i >> 3) * 64 + (i & 7u) * 4;
         *reinterpret_cast<h4_t*>(d) = h;
@@ -104,6 +111,11 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
             }
         }
     }
+    wide = wave_sum(wide);  // whole numbers below 2^24, or past 2^28
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wide;
+    __syncthreads();
+    if (threadIdx.x == 0) ex[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]) > 0.0f ? kExactRow : e;
 }
 
 // ------------------------------------------------------------- decoders ---
@@ -160,6 +172,82 @@ __device__ __forceinline__ h8_t decode_raw(const Raw<FMT>& r, uint32_t h, uint32
     return o;
 }
 
+// A thread's 16 dequantised weights of block b, element order as above.
+template <int FMT>
+__device__ __forceinline__ void weights16(const uint8_t* base, uint32_t off, uint32_t b, uint32_t h, float (&w)[16]) {
+    Raw<FMT> r;
+    load_raw<FMT>(base, b, off + code_offset<FMT>(h), off, r);
+    const float d = half_bits_to_float(r.d);
+#pragma unroll
+    for (uint32_t j = 0; j < 2; ++j) {
+        const h8_t q = decode_raw<FMT>(r, h, j);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[8 * j + i] = float(q[i]) * d;
+    }
+}
+
+// The 32 x 32 outputs of a wave's activation rows (x: the lane's, from its
+// first element of block 0) and weight rows (load(b, w): weights16 of the
+// lane's), on the fp32 MFMA: what marked rows take.  A lane half holds 16 k of
+// a block, one of each pair that an instruction multiplies.
+template <class Load>
+__device__ __forceinline__ v16f exact_tile(const float* x, uint32_t b_begin, uint32_t b_end, Load load) {
+    v16f t;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+    for (uint32_t b = b_begin; b < b_end; ++b) {
+        float4 a[4];
+        float w[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = reinterpret_cast<const float4*>(x + 32 * b)[q];
+        load(b, w);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].x, w[4 * q], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].y, w[4 * q + 1], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].z, w[4 * q + 2], t, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].w, w[4 * q + 3], t, 0, 0, 0);
+        }
+    }
+    return t;
+}
+// The end of both kernels: a wave's 64 x 64 sums (from row m, column n) to Y,
+// scaled back; marked rows from exact_tile.
+template <class Load>
+__device__ __forceinline__ void store_tile(v16f (&acc)[2][2], const int* __restrict__ ex, const float* __restrict__ X,
+                                           float* __restrict__ Y, uint32_t m0, uint32_t n0, uint32_t M, uint32_t N,
+                                           uint32_t K, uint32_t b_begin, uint32_t b_end, Load load) {
+    uint32_t lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // opaque: nothing below is formed before the main loop
+    const uint32_t l32 = lane & 31, lh = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t r = min(m0 + i * 32 + l32, M - 1);
+        if (__any(ex[r] == kExactRow)) {
+            const float* x = X + size_t(r) * K + 16 * lh;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t n = min(n0 + j * 32 + l32, N - 1);
+                const v16f t = exact_tile(x, b_begin, b_end, [&](uint32_t b, float (&w)[16]) { load(n, lh, b, w); });
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (ex[min(m0 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3), M - 1)] == kExactRow) acc[i][j][v] = t[v];
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const uint32_t m = m0 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+            if (m >= M) continue;
+            const int e = ex[m] == kExactRow ? 0 : -ex[m];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t n = n0 + j * 32 + l32;
+                if (n < N) Y[size_t(m) * N + n] = ldexpf(acc[i][j][v], e);
+            }
+        }
+    }
+}
+
 // --------------------------------------------------------------- kernel ---
 // One K stage of a tile in LDS: activations [BM][128 B] (the row's 32 hi and
 // 32 lo halves), weight codes [BN][64 B] as f16, group scales [BN].  16-byte
@@ -174,7 +262,7 @@ struct SplitStage {
 // WM x WN waves of a 64 x 64 tile each.
 template <int FMT, int WM, int WN>
 __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t* XS,
-                                                const int* __restrict__ ex, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
+                                                const int* __restrict__ ex, const float* __restrict__ X, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
                                                 uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n,
                                                 uint32_t blocks_per_split) {
     constexpr int BM = 64 * WM, BN = 64 * WN, TH = 64 * WM * WN;
@@ -347,25 +435,14 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
         if (last) acc[1][1][v] = fmaf(p[1][v], dc, acc[1][1][v]);
         else acc[1][0][v] = fmaf(p[1][v], dc, acc[1][0][v]);
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const uint32_t m = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-            if (m >= M) continue;
-            const int e = -ex[m];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t n = n0 + wn * 64 + j * 32 + l32;
-                if (n < N) Yout[size_t(m) * N + n] = ldexpf(acc[i][j][v], e);
-            }
-        }
+    store_tile(acc, ex, X, Yout, m0 + wm * 64, n0 + wn * 64, M, N, K, b_begin, b_end,
+               [&](uint32_t n, uint32_t h, uint32_t b, float (&o)[16]) { weights16<FMT>(w_base, (n - n0) * uint32_t(rb), b, h, o); });
 }
 template <int FMT, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(
-    const uint8_t* W, const uint8_t* XS, const int* __restrict__ ex, float* __restrict__ Y,
+    const uint8_t* W, const uint8_t* XS, const int* __restrict__ ex, const float* __restrict__ X, float* __restrict__ Y,
     float* __restrict__ partial, uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n, uint32_t blocks_per_split) {
-    gemm_split_body<FMT, WM, WN>(W, XS, ex, Y, partial, M, N, K, tiles_m, tiles_n, blocks_per_split);
+    gemm_split_body<FMT, WM, WN>(W, XS, ex, X, Y, partial, M, N, K, tiles_m, tiles_n, blocks_per_split);
 }
 
 
@@ -449,6 +526,30 @@ __device__ __forceinline__ void decode_rawk(const RawK<FMT>& r, uint32_t g, uint
     }
 }
 
+// A thread's 16 dequantised weights of block b: its exact parts, rounded once
+// as the reference's dequantisation is.
+template <int FMT>
+__device__ __forceinline__ void weights16k(const uint8_t* base, uint32_t off, uint32_t b, uint32_t h, float (&w)[16]) {
+    const uint32_t g = b & 7u;
+    RawK<FMT> r;
+    load_rawk<FMT>(base + size_t(b >> 3) * kSuperBytes<FMT>, off, g, h, r);
+#pragma unroll
+    for (uint32_t j = 0; j < 2; ++j) {
+        h8_t o[kPlanes<FMT>];
+        decode_rawk<FMT>(r, g, j, o);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if constexpr (kOffsets<FMT>) {
+                const float sq = float(o[0][i]) + (FMT == kQ4_K ? 8.0f : 16.0f) * float(kq_scale(r.head[0], g));
+                w[8 * j + i] = fmaf(half_bits_to_float(r.head[0][0]), sq,
+                                    -(half_bits_to_float(r.head[0][0] >> 16) * float(kq_min(r.head[0], g))));
+            } else {
+                w[8 * j + i] = half_bits_to_float(r.d) * (float(o[0][i]) + float(o[1][i]));
+            }
+        }
+    }
+}
+
 template <int FMT, int BM, int BN>
 struct SplitStageK {
     static constexpr int A = BM * 128, W = BN * 64 * kPlanes<FMT>;
@@ -461,7 +562,7 @@ struct SplitStageK {
 
 template <int FMT, int WM, int WN>
 __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8_t* XS, const uint8_t* SS,
-                                                   const int* __restrict__ ex, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
+                                                   const int* __restrict__ ex, const float* __restrict__ X, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
                                                    uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n,
                                                    uint32_t blocks_per_split) {
     constexpr int BM = 64 * WM, BN = 64 * WN, TH = 64 * WM * WN, P = kPlanes<FMT>;
@@ -678,25 +779,14 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
         stage(I2{}, b);
         if (++b >= b_end) break;
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const uint32_t m = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-            if (m >= M) continue;
-            const int e = -ex[m];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t n = n0 + wn * 64 + j * 32 + l32;
-                if (n < N) Yout[size_t(m) * N + n] = ldexpf(acc[i][j][v], e);
-            }
-        }
+    store_tile(acc, ex, X, Yout, m0 + wm * 64, n0 + wn * 64, M, N, K, b_begin, b_end,
+               [&](uint32_t n, uint32_t h, uint32_t b, float (&o)[16]) { weights16k<FMT>(w_base, (n - n0) * uint32_t(rb), b, h, o); });
 }
 template <int FMT, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, WN == 4 ? 2 : 1) void gemm_split_kq_kernel(
-    const uint8_t* W, const uint8_t* XS, const uint8_t* SS, const int* __restrict__ ex, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
+    const uint8_t* W, const uint8_t* XS, const uint8_t* SS, const int* __restrict__ ex, const float* __restrict__ X, float* __restrict__ Y, float* __restrict__ partial, uint32_t M,
     uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n, uint32_t blocks_per_split) {
-    gemm_split_kq_body<FMT, WM, WN>(W, XS, SS, ex, Y, partial, M, N, K, tiles_m, tiles_n, blocks_per_split);
+    gemm_split_kq_body<FMT, WM, WN>(W, XS, SS, ex, X, Y, partial, M, N, K, tiles_m, tiles_n, blocks_per_split);
 }
 
 }  // namespace
@@ -741,6 +831,7 @@ namespace {
 struct SplitArgs {
     const uint8_t *w, *xs, *ss;
     const int* ex;
+    const float* X;
     float *Y, *partial;
     uint32_t m, n, k;
     hipStream_t stream;
@@ -754,10 +845,10 @@ static hipError_t launch_tile(const SplitArgs& a, const SplitPlan& plan) {
     const dim3 grid(tiles_m * tiles_n * plan.ks), block(128 * WN);
     if constexpr (FMT == kQ8_0 || FMT == kQ4_0)
         hipLaunchKernelGGL((gemm_split_kernel<FMT, 2, WN>), grid, block, (SplitStage<BM, BN>::LDS), a.stream, a.w, a.xs,
-                           a.ex, a.Y, a.partial, a.m, a.n, a.k, tiles_m, tiles_n, plan.blocks);
+                           a.ex, a.X, a.Y, a.partial, a.m, a.n, a.k, tiles_m, tiles_n, plan.blocks);
     else
         hipLaunchKernelGGL((gemm_split_kq_kernel<FMT, 2, WN>), grid, block, (SplitStageK<FMT, BM, BN>::LDS), a.stream, a.w,
-                           a.xs, a.ss, a.ex, a.Y, a.partial, a.m, a.n, a.k, tiles_m, tiles_n, plan.blocks);
+                           a.xs, a.ss, a.ex, a.X, a.Y, a.partial, a.m, a.n, a.k, tiles_m, tiles_n, plan.blocks);
     return hipGetLastError();
 }
 template <int FMT>
@@ -832,7 +923,7 @@ hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y
     uint8_t* ss = xs + M * K * 4;
     const bool sums = fmt == kQ4_K || fmt == kQ5_K;
     int* ex = reinterpret_cast<int*>(ss + (sums ? M * (K / 256) * 32 : 0));
-    const SplitArgs a{w, xs, ss, ex, Y, reinterpret_cast<float*>(xs + sb), uint32_t(M), uint32_t(N), uint32_t(K), stream};
+    const SplitArgs a{w, xs, ss, ex, X, Y, reinterpret_cast<float*>(xs + sb), uint32_t(M), uint32_t(N), uint32_t(K), stream};
     const SplitPlan plan =
         plan_split(fmt != kQ8_0 && fmt != kQ4_0, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float)));
     if (sums)
