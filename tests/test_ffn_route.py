@@ -59,3 +59,51 @@ def test_down_stores_the_residual_sum(zq, orc, fmt, hidden, ffn):
     got, want = out[:hidden].double().cpu().numpy(), (h1 + d).double().cpu().numpy()
     assert np.all(np.abs(got - want) <= 1e-4 + 1e-5 * mag)
     assert torch.equal(run(a, nw, x)[:hidden], out[:hidden])  # in place of x
+
+
+@pytest.mark.parametrize("ffn", (4096, 4352, 14336))  # down on the fp32 and the MFMA streaming kernel
+@pytest.mark.parametrize("u0", (np.inf, 3e11))
+def test_a_huge_activation_in_front_of_down(zq, orc, ffn, u0):
+    """One SiLU * up is infinite, or far above the others of its pair: the outputs
+    are infinite with the sign of the down weight it meets (NaN at a zero one),
+    and where every weight it meets is 0 the others keep fp32's precision."""
+    hidden, aw, r0, c0 = 512, 256, 70, 33
+    w = {k: orc.gen_weights(O.Q8_0, s, r, c) for k, s, r, c in
+         (("o", 910, hidden, aw), ("g", 911, ffn, hidden), ("u", 912, ffn, hidden), ("d", 913, hidden, ffn))}
+
+    def code(k, cols, rows, col):
+        """The codes of a column, writable."""
+        b = w[k].reshape(-1, cols // 32, 34)
+        return b[rows, col // 32, 2 + col % 32:3 + col % 32]
+
+    # column c0 of the normalised vector is huge and reaches up's row r0 alone
+    code("g", hidden, slice(None), c0)[:] = code("u", hidden, slice(None), c0)[:] = 0
+    code("u", hidden, slice(r0, r0 + 1), c0)[:] = 100
+    w["u"].reshape(-1, hidden // 32, 34)[r0, c0 // 32, :2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
+    if np.isfinite(u0):
+        code("d", ffn, slice(None), r0)[:] = 0
+    x, nw, a = orc.gen_normal(914, hidden), orc.gen_normal(915, hidden), np.zeros(aw, np.float32)
+    x[c0] = 1.0
+    nw[c0] = 3e38 if np.isinf(u0) else u0 / 100
+    shapes = {"o": (hidden, aw), "g": (ffn, hidden), "u": (ffn, hidden), "d": (hidden, ffn)}
+    dev = {k: torch.zeros(zq.weight_bytes(O.Q8_0, r, c), dtype=torch.uint8, device=DEV) for k, (r, c) in shapes.items()}
+    for k in dev:
+        dev[k][: w[k].size] = torch.from_numpy(w[k]).to(DEV)
+    wsb = zq.ffn_residual_workspace_bytes(hidden, ffn)
+    ws, out = torch.empty(wsb, dtype=torch.uint8, device=DEV), torch.empty(hidden, device=DEV)
+    zq.ffn_residual_fused_dev(O.Q8_0, dev["o"], dev["g"], dev["u"], dev["d"], torch.from_numpy(nw).to(DEV),
+                              torch.from_numpy(x).to(DEV), torch.from_numpy(a).to(DEV), out, hidden, aw, ffn, 1e-5, ws, wsb)
+    W = {k: orc.dequantize(O.Q8_0, w[k], r * c).reshape(r, c).astype(np.float64) for k, (r, c) in shapes.items()}
+    h1 = x.astype(np.float64)
+    h2 = (h1 / np.sqrt((h1 * h1).mean() + 1e-5)).astype(np.float32) * nw  # fp32: up's sum overflows as there
+    with np.errstate(all="ignore"):
+        g, u = W["g"] @ h2, (W["u"] @ h2).astype(np.float32).astype(np.float64)
+        f = g / (1.0 + np.exp(-g)) * u
+        terms = W["d"] * f
+        want, mag = h1 + terms.sum(1), np.abs(h1) + np.abs(terms).sum(1)
+    got = out.double().cpu().numpy()
+    assert np.isinf(u[r0]) == np.isinf(u0) and np.isfinite(np.delete(u, r0)).all() and abs(u[r0]) > 1e8
+    if np.isinf(u0):
+        assert np.array_equal(got, want, equal_nan=True) and np.isinf(got).any()
+    else:  # the GEMV bar, as above
+        assert np.all(np.abs(got - want) <= 1e-4 + 1e-5 * mag)

@@ -1261,7 +1261,10 @@ __global__ __launch_bounds__(kThreads) void gemv_block_kernel(TaskTable tt, cons
 // fp32 reference's own rounding level.  Against the fp32-FMA kernel this
 // replaces ~2 VALU instructions per weight element by ~24 per 4096 elements,
 // so the decode tail after the last weight block shrinks.  Non-finite x makes
-// every output NaN.
+// every output NaN.  With RES (the FFN step's down projection, whose other
+// forms multiply in fp32) x that X does not carry is multiplied in fp32
+// instead: a non-finite one, or a pair a quarter of whose elements lie 2^20
+// below its largest.
 //
 // Work split: a wave owns a slice of 16 pairs (1024 columns) for the whole
 // kernel -- its digits stay in 16 VGPRs -- and each row block it streams
@@ -1285,6 +1288,21 @@ struct MfmaGeo {
     static constexpr int WBUF = ROWS * WROW;                // dwords per wave stash
     static constexpr int NU = (ROWS * UPR + 63) / 64;       // 16 B loads per lane per row block
 };
+
+// A lane's elements lane, lane + 64, ... of a row times x, in fp32.
+template <int FMT>
+__device__ __forceinline__ float lane_dot(const uint8_t* row, const float* x, uint32_t cols, uint32_t lane) {
+    float acc = 0.0f;
+    for (uint32_t k = lane; k < cols; k += 64) {
+        const uint8_t* b = row + size_t(k >> 5) * (FMT == kQ8_0 ? 34 : 18);
+        const uint32_t e = k & 31u;
+        int q;
+        if constexpr (FMT == kQ8_0) q = int8_t(b[2 + e]);
+        else q = int((b[2 + (e & 15u)] >> (e < 16 ? 0 : 4)) & 15u) - 8;
+        acc = fmaf(float(q) * half_bits_to_float(*reinterpret_cast<const uint16_t*>(b)), x[k], acc);
+    }
+    return acc;
+}
 
 template <int FMT, int XPT, int D, int XK, bool RES>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const float* __restrict__ x, uint32_t cols,
@@ -1416,6 +1434,16 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
         am = fmaxf(am, dpp_f<kDppHalfMirror>(am));
         am = fmaxf(am, dpp_f<kDppMirror>(am));
         bad |= !(am <= 3.402823466e38f);  // inf or NaN
+        if constexpr (RES) {
+            const float low = am * 0x1p-20f;
+            auto far = [&](float v) { return v != 0.0f && fabsf(v) < low ? 1.0f : 0.0f; };
+            float c = (far(t.x) + far(t.y)) + (far(t.z) + far(t.w));
+            c += dpp_f<kDppXor1>(c);
+            c += dpp_f<kDppXor2>(c);
+            c += dpp_f<kDppHalfMirror>(c);
+            c += dpp_f<kDppMirror>(c);
+            bad |= c >= 16.0f;
+        }
         const int s = 30 - (am > 0.0f && am <= 3.402823466e38f ? __builtin_amdgcn_frexp_expf(am) : 0);
         const uint32_t y0 = uint32_t(int(ldexpf(t.x, s))) + 0x80808080u;
         const uint32_t y1 = uint32_t(int(ldexpf(t.y, s))) + 0x80808080u;
@@ -1435,7 +1463,17 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
             if (e == 0) sexp[p] = s;
         }
     }
-    const bool nan_out = __syncthreads_or(bad) != 0;
+    const bool no_digits = __syncthreads_or(bad) != 0;
+    if constexpr (RES) {
+        if (no_digits) {  // the same in every workgroup: a wave per row
+            const GemvTask& t = tt.t[0];
+            for (uint32_t row = blockIdx.x * NW + wave; row < t.rows; row += gridDim.x * NW) {
+                const float v = wave_sum(lane_dot<FMT>(t.w + size_t(row) * rb, x, cols, lane));
+                if (lane == 0) t.y[row] = pro.res[row] + v;
+            }
+            return;
+        }
+    }
     // this lane's B operand: digit qi of pair p0 + qb (16 dwords, K order)
     int dig[16];
     {
@@ -1550,7 +1588,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
             for (uint32_t s2 = 0; s2 < 16; ++s2)
                 if (s2 < S) s += ((w[s2].x + w[s2].y) + w[s2].z) + w[s2].w;
             const GemvTask& t = tt.t[ti];
-            if (nan_out) s = __builtin_nanf("");
+            if (!RES && no_digits) s = __builtin_nanf("");
             if constexpr (RES && FMT != kQ8_0) rv = pro.res[min(row0 + lane, t.rows - 1)];
             if constexpr (RES) s = rv + s;
             if (row0 + lane < t.rows) t.y[row0 + lane] = s;
