@@ -2,6 +2,8 @@
 number of super-blocks and Q8_0 / Q4_0 of any number of blocks -- each remainder
 and count of slices, every start of a row within 16 bytes, one task and several,
 and Q6_K's paired gate|up form."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -54,6 +56,28 @@ def test_any_number_of_super_blocks(zq, orc, sb, rows):
 @pytest.mark.parametrize("fmt", (O.Q8_0, O.Q4_0))
 def test_any_number_of_blocks(zq, orc, fmt, blocks, rows):
     check(zq, orc, fmt, 32 * blocks, rows, 1100 + blocks)
+
+
+def streamed(zq, fmt, cols, rows):
+    """The library's own rule for which rows the streaming kernels take."""
+    f = zq.lib()._ZN2zq13gemv_streamedEijj
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32]
+    return f(fmt, cols, rows)
+
+
+# blocks (Q6_K: super-blocks) per row as above, with rows enough for the streaming
+# kernels: past the two-rows-per-step line with a last partial block of rows, 8
+# waves a workgroup, three tasks; and the few rows that long odd ones take
+@pytest.mark.parametrize("fmt,blocks,rows", [
+    *((O.Q6_K, b, r) for b in (2, 3, 4) for r in ((8190,), (4090,), (4000, 7, 4183))),
+    *((f, b, (8190,)) for f in (O.Q8_0, O.Q4_0) for b in (23, 29, 63, 90, 127, 129, 130, 253, 257, 345, 449, 510, 511)),
+    *((f, b, (4000, 7, 4183)) for f in (O.Q8_0, O.Q4_0) for b in (63, 90, 257)),
+    *((f, b, (2045,)) for f in (O.Q8_0, O.Q4_0) for b in (127, 130, 257)),
+    *((f, b, (67,)) for f in (O.Q8_0, O.Q4_0) for b in (225, 511))])
+def test_rows_that_are_streamed(zq, orc, fmt, blocks, rows):
+    cols = (256 if fmt == O.Q6_K else 32) * blocks
+    assert streamed(zq, fmt, cols, sum(rows))
+    check(zq, orc, fmt, cols, rows, 1200 + blocks)
 
 
 @pytest.mark.parametrize("sb", (1, 3, 20))

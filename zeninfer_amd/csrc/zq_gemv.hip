@@ -1963,6 +1963,43 @@ hipError_t launch_streamed(TaskTable& tt, const float* x, uint32_t c, uint32_t t
 }
 }  // namespace
 
+// Rows that a streaming launch of wgs workgroups does in the time of whole
+// rounds of one workgroup per CU: a last round that is partly empty costs as
+// much as a full one.
+static double streamed_rows(uint32_t rows, uint32_t rows_per_wg) {
+    const uint32_t wgs = (rows + rows_per_wg - 1) / rows_per_wg, cus = uint32_t(cu_count());
+    return double(rows) * wgs / (double(cus) * ((wgs + cus - 1) / cus));
+}
+// Where the streaming kernels beat the finer-grained ones (16-byte aligned
+// operands; `rows` of all tasks).  Measured over 1..100000 rows with weights
+// from HBM (first figures) and from L2 (second), other kernel -> streamed, us:
+// a streaming launch has the longer start and the coarser grid, and wins by its
+// rate.
+//  * Q6_K: rows of whole chunks and, from 1280 columns, all others (1 x 1280
+//    2.9 -> 2.8 / 3.3 -> 3.2; 20000 x 5120 97 -> 30).  From 512 columns where
+//    the grid is large and even (2048 x 1024 5.1 -> 3.8 / 4.1 -> 3.7; 8192 x 512
+//    11.4 -> 6.0 / 6.5 -> 6.6; but 6000 x 768 7.3 -> 6.0 / 4.5 -> 6.0).  Not one
+//    super-block (32000 x 256 15.9 -> 14.4 / 10.5 -> 15.5).
+//  * Q8_0 / Q4_0, rows that are not whole 16-byte units, from 704 columns (480
+//    columns at 20000 rows: 12.6 -> 13.9), by the work there is: an odd number
+//    of blocks goes lane by block otherwise (Q8_0 4096 x 1504 6.6 -> 5.9 / 1000 x
+//    4000 5.3 -> 4.5; 64 x 7200 6.2 -> 6.0; but 1000 x 1504 3.2 -> 4.3), an even
+//    one in dwords (Q8_0 8192 x 704 8.4 -> 7.4; 1000 x 2112 3.6 -> 4.4; Q4_0 12000
+//    x 704 10.5 -> 9.3; 4096 x 960 4.9 -> 5.2).
+bool gemv_streamed(int fmt, uint32_t cols, uint32_t rows) {
+    if (cols > 16384) return false;
+    if (fmt == kQ6_K) {
+        if (cols % 2048 == 0 || cols >= 1280) return true;
+        const uint32_t per = rows >= 4096 ? 16 : 8;
+        return cols >= 512 && rows >= 2048 && streamed_rows(rows, per) >= 0.9 * rows;
+    }
+    if (cols < 704) return false;
+    const uint32_t per = cols > 8192 ? 4 : cols > 4096 || rows <= 2048 ? 8 : 16;
+    const double work = streamed_rows(rows, per) * cols;
+    if (cols % 64 == 0) return work >= (fmt == kQ8_0 ? 5e6 : 7e6);
+    return work >= (cols >= 2048 ? 3e6 : 5e6) || (rows >= 64 && cols >= 7168);
+}
+
 hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x, size_t cols,
                        hipStream_t stream) {
     if (count < 1 || count > kMaxTasks || !x || !row_bytes(fmt, cols) || cols > (1u << 24))
@@ -2000,7 +2037,7 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
         if (reinterpret_cast<uintptr_t>(x) & 15u) return hipErrorInvalidValue;
         bool w16 = true;
         for (int i = 0; i < count; ++i) w16 = w16 && (reinterpret_cast<uintptr_t>(tasks[i].w) & 15u) == 0;
-        if (w16 && c <= 16384) {
+        if (w16 && gemv_streamed(fmt, c, total_rows)) {
             const hipError_t e = launch_q6k_stream_any(tt, x, c, stream, total_rows);
             if (e != hipErrorInvalidConfiguration) return e;
         }
@@ -2017,12 +2054,7 @@ hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x
         return fmt == kQ8_0 ? launch_streamed<kQ8_0, false>(tt, x, c, total_rows, XPrologue{}, stream)
                             : launch_streamed<kQ4_0, false>(tt, x, c, total_rows, XPrologue{}, stream);
     }
-    // From 704 columns the streaming form takes the rows that are not whole
-    // 16 B units.  At 20000 rows of Q8_0 against the kernels below: 480 columns
-    // 12.6 us there, 13.9 streamed; 736 14.9 / 14.0; 2080 31.9 / 15.4; 11040
-    // 140 / 59; 14400, whose pairs are dword-aligned, 84.9 / 58.6.  Under 704 a
-    // wave has little to do between the barriers of its workgroup.
-    if (w16 && x16 && c >= 704 && c <= 16384) {
+    if (w16 && x16 && gemv_streamed(fmt, c, total_rows)) {
         const int Rx = xreg_rows(total_rows);
         const hipError_t e = fmt == kQ8_0 ? launch_stream_any<kQ8_0, false, true>(Rx, tt, x, c, stream)
                                           : launch_stream_any<kQ4_0, false, true>(Rx, tt, x, c, stream);

@@ -24,6 +24,10 @@ size_t row_bytes(int fmt, size_t cols);
 hipError_t launch_gemv(int fmt, const GemvTask* tasks, int count, const float* x,
                        size_t cols, hipStream_t stream);
 
+// Whether launch_gemv streams such rows (Q6_K; Q8_0 / Q4_0 with cols % 256 != 0)
+// or gives them to the finer-grained kernels.
+bool gemv_streamed(int fmt, uint32_t cols, uint32_t rows);
+
 // The producer of a decode GEMV's input folded into the GEMV itself (every
 // workgroup recomputes it while staging x):
 //   kSiluMul   x = silu(a) * b, elementwise as launch_silu_mul
