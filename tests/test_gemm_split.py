@@ -171,6 +171,22 @@ def test_extreme_activations(zq, orc, fmt, m, n, k, split):
     check_extremes(orc, fmt, w, X, run_dev(zq, fmt, w, X, m, n, k, ws_bytes), m, n, k)
 
 
+# The matrix cores round the sums of 16-bit products down; a kernel that let this
+# add up would move every output the same way (measured: by 0.4 to 0.6 of the
+# errors' spread), which a model's later layers feel more than as much noise.
+# 33600 outputs or more: chance alone gives 0.01.
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,split", [(20, 1700, 4096, False), (48, 700, 4096, False)])
+@pytest.mark.parametrize("fmt", ALL)
+def test_errors_have_no_common_part(zq, orc, fmt, m, n, k, split):
+    w = orc.gen_weights(fmt, 540, n, k)
+    X = orc.gen_normal(541, m * k).reshape(m, k)
+    ws_bytes = zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32) if split else 0
+    assert takes_split(zq, fmt, m, n, k, ws_bytes) == split
+    e = run_dev(zq, fmt, w, X, m, n, k, ws_bytes) - orc.gemm_f64(fmt, w, X.reshape(-1), m, n, k)[0].reshape(m, n)
+    assert abs(e.mean()) < 0.1 * np.sqrt((e * e).mean())
+
+
 @pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))
 def test_generated_code(tmp_path, src):
     from zeninfer_amd.build import FLAGS, HIPCC, SRC

@@ -94,14 +94,17 @@ __device__ __forceinline__ bool needs_f32(f4_t x) {
     return fbits(top) - lo >= hi - lo && top != 0.0f;
 }
 
-// Eight signed code bytes as bf16 (|value| <= 128: exact).
-__device__ __forceinline__ b8_t codes8(uint32_t a, uint32_t b) {
+// Eight signed code bytes as bf16 (|value| <= 128: exact), the bits `flip` of
+// each pair changed.
+__device__ __forceinline__ b8_t codes8(uint32_t a, uint32_t b, uint32_t flip) {
     u4_t o;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         o[i] = hi_pair(sbyte(a, 2 * i), sbyte(a, 2 * i + 1));
         o[2 + i] = hi_pair(sbyte(b, 2 * i), sbyte(b, 2 * i + 1));
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] ^= flip;
     return __builtin_bit_cast(b8_t, o);
 }
 
@@ -151,22 +154,27 @@ __device__ __forceinline__ void load_group(const uint8_t* row, uint32_t b, uint3
         r.d = *reinterpret_cast<const uint16_t*>(p + 208);
     }
 }
-// The group's codes, its scale(s) -- per step for Q6_K --, its offset and the
-// min that the offset holds.
+// The group's codes, its scale(s) -- per step for Q6_K -- and, of its offset,
+// centre * scale and min.  flip (all bits of a uniform word, or none): codes and
+// scales with their signs changed.  The bf16 products' sums are rounded down, not
+// to nearest (measured: the mean of the errors of a long K is -0.4 of their
+// spread), which scales of one sign would carry to every output alike, and a
+// model's later layers feel that more than as much noise: with half of the
+// groups flipped it cancels.  Q6_K's sub-block scales have either sign already.
 template <int FMT>
-__device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, uint32_t h, b8_t (&w)[2], float (&s)[2],
-                                             float& off, float& min) {
+__device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, uint32_t h, uint32_t flip, b8_t (&w)[2],
+                                             float (&s)[2], float& cds, float& min) {
     const uint32_t g = b & 7u;
     uint32_t c[4];
-    off = min = 0.0f;
+    cds = min = 0.0f;
     if constexpr (FMT == kQ8_0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) c[i] = r.q[i];
-        s[0] = s[1] = half_bits_to_float(r.d);
+        s[0] = s[1] = bitsf(fbits(half_bits_to_float(r.d)) ^ (flip & 0x80000000u));
     } else if constexpr (FMT == kQ4_0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) c[i] = ((r.q[i] << (h ? 0 : 4)) & 0xF0F0F0F0u) ^ 0x80808080u;
-        s[0] = s[1] = half_bits_to_float(r.d) * 0.0625f;
+        s[0] = s[1] = bitsf(fbits(half_bits_to_float(r.d) * 0.0625f) ^ (flip & 0x80000000u));
     } else if constexpr (kOffset<FMT>) {
         const uint32_t sh = 8 * (g & 3u);
         const u4_t& hd = r.head[0];
@@ -174,13 +182,16 @@ __device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, ui
         const uint32_t mn = g < 4 ? (hd[2] >> sh) & 63u : ((hd[3] >> (sh + 4)) & 15u) | ((hd[2] >> (sh + 2)) & 0x30u);
         const float ds = half_bits_to_float(hd[0]) * float(sc);
         min = half_bits_to_float(hd[0] >> 16) * float(mn);  // exact
-        off = (FMT == kQ4_K ? 8.0f : 16.0f) * ds - min;
-        s[0] = s[1] = ds * (FMT == kQ4_K ? 0.0625f : 0.125f);
+        // flipped: the code's complement, which is centred one lower
+        constexpr uint32_t top = FMT == kQ4_K ? 0xF0F0F0F0u : 0xF8F8F8F8u;
+        const uint32_t sign = 0x80808080u ^ (flip & top);
+        cds = ((FMT == kQ4_K ? 8.0f : 16.0f) - (flip ? 1.0f : 0.0f)) * ds;
+        s[0] = s[1] = ds * (FMT == kQ4_K ? 0.0625f : 0.125f) * (flip ? -1.0f : 1.0f);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t n = (r.q[i] << (4 * (1 - (g & 1u)))) & 0xF0F0F0F0u;  // the code in the upper nibble
-            if constexpr (FMT == kQ4_K) c[i] = n ^ 0x80808080u;
-            else c[i] = ((n >> 1) | (((r.h[0][i] >> g) & 0x01010101u) << 7)) ^ 0x80808080u;
+            if constexpr (FMT == kQ4_K) c[i] = n ^ sign;
+            else c[i] = ((n >> 1) | (((r.h[0][i] >> g) & 0x01010101u) << 7)) ^ sign;
         }
     } else {
         const float d = half_bits_to_float(r.d) * 0.25f;
@@ -192,8 +203,8 @@ __device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, ui
             c[i] = ((n << 2) | (((r.h[0][i] >> (2 * (g & 3u))) & 0x03030303u) << 6)) ^ 0x80808080u;
         }
     }
-    w[0] = codes8(c[0], c[1]);
-    w[1] = codes8(c[2], c[3]);
+    w[0] = codes8(c[0], c[1], FMT == kQ8_0 || FMT == kQ4_0 ? flip & 0x80008000u : 0u);
+    w[1] = codes8(c[2], c[3], FMT == kQ8_0 || FMT == kQ4_0 ? flip & 0x80008000u : 0u);
 }
 
 template <int FMT, int MT>
@@ -213,6 +224,7 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t l32 = lane & 31, lh = lane >> 5;
     const uint32_t first = split * tasks.groups, end = min(K >> 5, first + tasks.groups);
+    const uint32_t flip = (first + wave) & 1u ? ~0u : 0u;  // by wave: a wave's groups are NW apart
     // loads cover whole lines: 8 lanes a row's 128 bytes (a lane reading its own
     // operand row touched 32 lines an instruction and bound the kernel)
     struct Source {
@@ -291,8 +303,8 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
     auto multiply = [&](uint32_t b, const Data& d) {
         stage_x(d, std::false_type{});
         b8_t w[2];
-        float sc[2], off, min;
-        decode_group<FMT>(d.w, b, lh, w, sc, off, min);
+        float sc[2], cds, min;
+        decode_group<FMT>(d.w, b, lh, flip, w, sc, cds, min);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             v16f p = zero;
@@ -313,7 +325,7 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
                     p = zero;
                 }
             }
-            if constexpr (kOffset<FMT>) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(sum, off, acc[i], 0, 0, 0);
+            if constexpr (kOffset<FMT>) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(sum, cds - min, acc[i], 0, 0, 0);
         }
     };
     if (first + wave < end) {
@@ -341,8 +353,8 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
             load(from, b, d);
             stage_x(d, std::true_type{});
             b8_t w[2];
-            float sc[2], off, min;
-            decode_group<FMT>(d.w, b, lh, w, sc, off, min);
+            float sc[2], cds, min;
+            decode_group<FMT>(d.w, b, lh, flip, w, sc, cds, min);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -352,7 +364,7 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
 #pragma unroll
                     for (int c = 0; c < 8; ++c) {
                         const float q = float(w[s][c]);
-                        const float wd = kOffset<FMT> ? fmaf(sc[s], q + 128.0f, -min) : sc[s] * q;
+                        const float wd = kOffset<FMT> ? fmaf(sc[s], q, cds) - min : sc[s] * q;  // one rounding
                         acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(e[c], wd, acc[i], 0, 0, 0);
                     }
                 }
