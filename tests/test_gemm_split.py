@@ -176,7 +176,7 @@ def test_extreme_activations(zq, orc, fmt, m, n, k, split):
 # errors' spread), which a model's later layers feel more than as much noise.
 # 33600 outputs or more: chance alone gives 0.01.
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k,split", [(20, 1700, 4096, False), (48, 700, 4096, False)])
+@pytest.mark.parametrize("m,n,k,split", [(20, 1700, 4096, False), (48, 700, 4096, False), (130, 1500, 4096, True)])
 @pytest.mark.parametrize("fmt", ALL)
 def test_errors_have_no_common_part(zq, orc, fmt, m, n, k, split):
     w = orc.gen_weights(fmt, 540, n, k)

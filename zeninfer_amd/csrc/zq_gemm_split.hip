@@ -126,12 +126,15 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
     asm volatile("" : "+v"(v));
     return v;
 }
-// Four code bytes u0..u3 (0..255) as binary16 u - off, two per dword: a byte
-// placed under 0x64 is the binary16 1024 + u.
+// Four code bytes u0..u3 (0..255) as binary16 u - off (NEG: off - u), two per
+// dword: a byte placed under 0x64 is the binary16 1024 + u.
+template <bool NEG = false>
 __device__ __forceinline__ void bytes_to_half(uint32_t u, _Float16 off, h2_t& a, h2_t& b) {
     const h2_t o = {off, off};
-    a = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - o;
-    b = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - o;
+    a = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u));
+    b = __builtin_bit_cast(h2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u));
+    a = NEG ? o - a : a - o;
+    b = NEG ? o - b : b - o;
 }
 
 // A thread's share of one 32-element block: half h holds elements 16h..16h+15.
@@ -154,16 +157,16 @@ __device__ __forceinline__ void load_raw(const uint8_t* base, uint32_t b, uint32
     r.q = *reinterpret_cast<const u4a2_t*>(p + opaque(co));
     r.d = *reinterpret_cast<const uint16_t*>(p + opaque(so));
 }
-// The 8 codes of step j.
-template <int FMT>
+// The 8 codes of step j, NEG: with their signs changed.
+template <int FMT, bool NEG = false>
 __device__ __forceinline__ h8_t decode_raw(const Raw<FMT>& r, uint32_t h, uint32_t j) {
     h8_t o;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const uint32_t q = r.q[2 * j + i];
         h2_t a, b;
-        if constexpr (FMT == kQ8_0) bytes_to_half(q ^ 0x80808080u, _Float16(1152.0f), a, b);
-        else bytes_to_half((q >> (4 * h)) & 0x0F0F0F0Fu, _Float16(1032.0f), a, b);
+        if constexpr (FMT == kQ8_0) bytes_to_half<NEG>(q ^ 0x80808080u, _Float16(1152.0f), a, b);
+        else bytes_to_half<NEG>((q >> (4 * h)) & 0x0F0F0F0Fu, _Float16(1032.0f), a, b);
         o[4 * i] = a[0];
         o[4 * i + 1] = a[1];
         o[4 * i + 2] = b[0];
@@ -316,11 +319,18 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
     auto store_a = [&](int buf, const Stage& r, int i) {
         *reinterpret_cast<u4_t*>(As + buf * G::A + i * (TH / 8) * 128 + a_dst) = r.a[i];
     };
-    auto store_w = [&](int buf, const Stage& r, uint32_t j) {  // step j's 8 codes
+    // Every other block is staged with the signs of its codes and scale changed
+    // (PAR): the f16 products' sums are rounded down, not to nearest, which scales
+    // of one sign would carry to every output alike (measured: the mean of the
+    // errors -0.4 to -0.6 of their spread); so it cancels.
+    auto store_w = [&](int buf, const Stage& r, uint32_t j, auto par_c) {  // step j's 8 codes
         *reinterpret_cast<h8_t*>(Bs + buf * G::W + w_row * 64 + (((2 * j + w_half) ^ w_swz) * 16)) =
-            decode_raw<FMT>(r.w, w_half, j);
+            decode_raw<FMT, decltype(par_c)::value == 1>(r.w, w_half, j);
     };
-    auto store_s = [&](int buf, const Stage& r) { Sw[buf * BN + w_row] = half_bits_to_float(r.w.d); };
+    auto store_s = [&](int buf, const Stage& r, auto par_c) {
+        const float d = half_bits_to_float(r.w.d);
+        Sw[buf * BN + w_row] = decltype(par_c)::value == 1 ? -d : d;
+    };
 
     v16f acc[2][2];
     v16f zero;
@@ -354,8 +364,8 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
     // a tile's 16 scaled additions follow in the next tile's four slots, and
     // the staging is spread over the slots, because a wave's VALU work runs
     // under its own MFMAs only where it is issued between them (measured: an
-    // MFMA and n VALU instructions take max(32, 8 + 4n) cycles).  PAR: the
-    // column order alternates so that the column read last is free first.
+    // MFMA and n VALU instructions take max(32, 8 + 4n) cycles).  PAR, the block's
+    // parity: the column order alternates so that the column read last is free first.
     v16f p[2];        // products of a tile; p[1] enters a stage with the previous stage's last tile
     float dc = 0.0f;  // ... its scale
     float dt = 0.0f;  // the scale of a stage's last but one tile (its column's is replaced early)
@@ -381,9 +391,9 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
             if (s == 2) read_a(BUF, 1, 1);
             if (s >= 3 && s < 3 + AU) store_a(WB, r, s - 3);
             if (s >= 4 && s < 4 + AU) load_a(far, r, s - 4);
-            if (s == 9) store_w(WB, r, 0);
-            if (s == 11) store_w(WB, r, 1);
-            if (s == 12) store_s(WB, r);
+            if (s == 9) store_w(WB, r, 0, par_c);  // block b + 2
+            if (s == 11) store_w(WB, r, 1, par_c);
+            if (s == 12) store_s(WB, r, par_c);
             if (s == 13) load_w(far, r);
             if (s == 8) read_a(NB, 0, 0);
             if (s == 10) read_a(NB, 0, 1);
@@ -393,18 +403,21 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
         lds_barrier();
     };
     if (b_begin >= b_end) return;
-    auto fill = [&](int buf, uint32_t b) {
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    auto fill = [&](int buf, uint32_t b, auto par_c) {
 #pragma unroll
         for (int i = 0; i < AU; ++i) load_a(b, r, i);
         load_w(b, r);
 #pragma unroll
         for (int i = 0; i < AU; ++i) store_a(buf, r, i);
-        store_w(buf, r, 0);
-        store_w(buf, r, 1);
-        store_s(buf, r);
+        store_w(buf, r, 0, par_c);
+        store_w(buf, r, 1, par_c);
+        store_s(buf, r, par_c);
     };
-    fill(0, b_begin);
-    fill(1, min(b_begin + 1, b_end - 1));
+    fill(0, b_begin, I0{});
+    fill(1, min(b_begin + 1, b_end - 1), I1{});
 #pragma unroll
     for (int i = 0; i < AU; ++i) load_a(min(b_begin + 2, b_end - 1), r, i);
     load_w(min(b_begin + 2, b_end - 1), r);
@@ -412,9 +425,6 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
     read_a(0, 0, 0);
     read_a(0, 0, 1);
     read_w(0, 0);
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
     int last = 0;  // the column order of the last stage
     for (uint32_t b = b_begin;;) {
         stage(I0{}, I0{}, b);
@@ -495,11 +505,12 @@ __device__ __forceinline__ uint32_t kq_min(const u4_t& w, uint32_t g) {
     const uint32_t sh = 8 * (g & 3u);
     return g < 4 ? (w[2] >> sh) & 63u : ((w[3] >> (sh + 4)) & 15u) | ((w[2] >> (sh + 2)) & 0x30u);
 }
-// The 8 scaled codes of step j (Q6_K: hi and lo).
+// The 8 scaled codes of step j (Q6_K: hi and lo), with their signs changed for
+// flip = 0x80008000 (uniform; else 0).
 template <int FMT>
-__device__ __forceinline__ void decode_rawk(const RawK<FMT>& r, uint32_t g, uint32_t j, h8_t (&o)[kPlanes<FMT>]) {
+__device__ __forceinline__ void decode_rawk(const RawK<FMT>& r, uint32_t g, uint32_t j, uint32_t flip, h8_t (&o)[kPlanes<FMT>]) {
     const _Float16 sc = kOffsets<FMT> ? _Float16(float(kq_scale(r.head[0], g))) : _Float16(float(int(int8_t(uint8_t(r.sc)))));
-    const h2_t s = {sc, sc};
+    const h2_t s = __builtin_bit_cast(h2_t, __builtin_bit_cast(uint32_t, h2_t{sc, sc}) ^ flip);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int e = 2 * j + i;
@@ -536,7 +547,7 @@ __device__ __forceinline__ void weights16k(const uint8_t* base, uint32_t off, ui
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
         h8_t o[kPlanes<FMT>];
-        decode_rawk<FMT>(r, g, j, o);
+        decode_rawk<FMT>(r, g, j, 0u, o);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             if constexpr (kOffsets<FMT>) {
@@ -613,29 +624,33 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
     auto store_a = [&](int buf, int i) {
         *reinterpret_cast<u4_t*>(As + buf * G::A + i * (TH / 8) * 128 + a_dst) = r.a[i];
     };
-    auto store_w = [&](int buf, uint32_t g, uint32_t j) {  // step j's 8 codes
+    // every other super-block with its signs changed, as in gemm_split_body
+    auto flip_of = [&](uint32_t b) { return (b >> 3) & 1u ? 0x80008000u : 0u; };
+    auto store_w = [&](int buf, uint32_t b, uint32_t j) {  // step j's 8 codes of block b
         h8_t o[P];
-        decode_rawk<FMT>(r.w, g, j, o);
+        decode_rawk<FMT>(r.w, b & 7u, j, flip_of(b), o);
 #pragma unroll
         for (int q = 0; q < P; ++q)
             *reinterpret_cast<h8_t*>(Bs + buf * G::W + q * BN * 64 + w_row * 64 + (((2 * j + w_half) ^ w_swz) * 16)) = o[q];
     };
     // the super-block's d and dmin and its offset factors (half 0: scales, 1: mins)
-    auto store_head = [&]() {
+    auto store_head = [&](uint32_t b) {
         int t = tid;  // opaque: the addresses below are not kept in registers around the loop
         asm volatile("" : "+v"(t));
         const uint32_t w_half = t & 1, w_row = t >> 1;
+        const float sign = flip_of(b) ? -1.0f : 1.0f;
         if constexpr (kOffsets<FMT>) {
+            const float f = sign * (w_half ? 32.0f : FMT == kQ4_K ? 256.0f : 512.0f);
             h8_t o;
 #pragma unroll
             for (uint32_t g = 0; g < 8; ++g) {
                 const uint32_t sc = kq_scale(r.w.head[0], g), mn = kq_min(r.w.head[0], g);
-                o[g] = _Float16(float(w_half ? 32u * mn : (FMT == kQ4_K ? 256u : 512u) * sc));
+                o[g] = _Float16(f * float(w_half ? mn : sc));
             }
             *reinterpret_cast<h8_t*>(Of + w_half * BN * 16 + w_row * 16) = o;
-            Ds[w_half * BN + w_row] = half_bits_to_float(w_half ? r.w.head[0][0] >> 16 : r.w.head[0][0]);
+            Ds[w_half * BN + w_row] = sign * half_bits_to_float(w_half ? r.w.head[0][0] >> 16 : r.w.head[0][0]);
         } else {
-            Ds[w_row] = half_bits_to_float(r.w.d);
+            Ds[w_row] = sign * half_bits_to_float(r.w.d);
         }
     };
 
@@ -713,14 +728,14 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
     };
     auto stage = [&](auto buf_c, uint32_t b) {
         constexpr int BUF = decltype(buf_c)::value, NB = (BUF + 1) % 3, WB = (BUF + 2) % 3;
-        const uint32_t g = b & 7u, far = min(b + 3, b_end - 1), ng = min(b + 2, b_end - 1) & 7u;
+        const uint32_t g = b & 7u, far = min(b + 3, b_end - 1), nb2 = min(b + 2, b_end - 1);
         if (g == 0) {
             if constexpr (kOffsets<FMT>) {  // row su / 2, hi or lo su % 2 (threads past the tile repeat)
                 const uint32_t su = sum_unit();
                 sums = *reinterpret_cast<const u4_t*>(SS + (size_t(min(m0 + (su >> 1), M - 1)) * (nb >> 3) + (b >> 3)) * 32 +
                                                       (su & 1) * 16);
             }
-            store_head();
+            store_head(b);
         }
         if constexpr (kOffsets<FMT>)
             if (g == 1) *reinterpret_cast<u4_t*>(Sa + sum_unit() * 16) = sums;
@@ -740,8 +755,8 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
                 if (f == 3 && s == 1) read_w(NB, 0, wn);
                 if (slot >= 2 && slot < 2 + AU) store_a(WB, slot - 2);
                 if (slot == 2 + AU) load_a(far);
-                if (slot == 6) store_w(WB, ng, 0);
-                if (slot == 9) store_w(WB, ng, 1);
+                if (slot == 6) store_w(WB, nb2, 0);
+                if (slot == 9) store_w(WB, nb2, 1);
                 if (slot == 10) load_w(far);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -752,16 +767,16 @@ __device__ __forceinline__ void gemm_split_kq_body(const uint8_t* W, const uint8
         lds_barrier();
     };
     if (b_begin >= b_end) return;
-    auto fill = [&](int buf, uint32_t b, uint32_t g) {
+    auto fill = [&](int buf, uint32_t b) {
         load_a(b);
         load_w(b);
 #pragma unroll
         for (int i = 0; i < AU; ++i) store_a(buf, i);
-        store_w(buf, g, 0);
-        store_w(buf, g, 1);
+        store_w(buf, b, 0);
+        store_w(buf, b, 1);
     };
-    fill(0, b_begin, 0);
-    fill(1, b_begin + 1, 1);
+    fill(0, b_begin);
+    fill(1, b_begin + 1);
     load_a(b_begin + 2);
     load_w(b_begin + 2);
     lds_barrier();
