@@ -106,7 +106,7 @@ def extremes(orc, fmt, w, m, n, k):
     X[7, [9, 33]] = np.inf, np.nan
     X[8] = np.where(np.arange(k) % 2, np.inf, -np.inf)
     X[9] *= np.float32(2.0 ** 120)
-    X[10] *= np.float32(2.0 ** -116)
+    X[10] *= np.float32(2.0 ** -100)
     X[11, 5] *= np.float32(2.0 ** 124)
     return X
 

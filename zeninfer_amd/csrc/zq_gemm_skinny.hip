@@ -15,9 +15,8 @@
 // v_mfma_f32_32x32x16_bf16 gives exact products in fp32 sums, three
 // instructions for each 16 k.  A group's sum is scaled by its fp32 scale into
 // the accumulator; the offset of Q4_K / Q5_K multiplies the group's sum of x on
-// the fp32 MFMA.  Activations for which that would not be exact (infinite, at
-// the ends of the fp32 range: needs_f32) are multiplied in fp32 by the dequantised
-// weights instead.
+// the fp32 MFMA.  Sums that are not finite are formed again in fp32 with the
+// dequantised weights (see the kernel).
 //
 // Bound: at a few tokens the launch and the chain of a wave's K groups (loads,
 // decoding, products; 16 and 8 waves sharing K measured the same), past ~100
@@ -28,7 +27,6 @@
 #include "zq_internal.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace zq {
 namespace {
@@ -62,8 +60,8 @@ __device__ __forceinline__ uint32_t hi_pair(float a, float b) {
     return __builtin_amdgcn_perm(fbits(b), fbits(a), 0x07060302u);
 }
 
-// x (8 elements) as bf16 planes: p0 + p1 + p2 == x exactly, for those that
-// needs_f32() does not take.  A NaN is one in p0 or p1.
+// x (8 elements) as bf16 planes: p0 + p1 + p2 == x exactly, down to 2^-110 (below,
+// to 2^-133 absolutely).  An infinity or a NaN gives a NaN in p1.
 __device__ __forceinline__ void split3(const float (&x)[8], b8_t& p0, b8_t& p1, b8_t& p2) {
     float r1[8], r2[8];
 #pragma unroll
@@ -80,18 +78,6 @@ __device__ __forceinline__ void split3(const float (&x)[8], b8_t& p0, b8_t& p1, 
     p0 = __builtin_bit_cast(b8_t, a);
     p1 = __builtin_bit_cast(b8_t, b);
     p2 = __builtin_bit_cast(b8_t, c);
-}
-
-// Whether four activations need fp32 products: the largest is infinite (an
-// infinity times a centred code and times the group's offset can have opposite
-// signs where the weight's own sign decides), so large that a code times it
-// could overflow where the weight times it does not (from 2^112: 32 products
-// by codes below 2^7 stay under 2^124), or so small that its third part falls
-// below the smallest bf16 (under 2^-108, but not all 0).
-__device__ __forceinline__ bool needs_f32(f4_t x) {
-    const float top = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-    constexpr uint32_t lo = (127u - 108u) << 23, hi = (127u + 112u) << 23;
-    return fbits(top) - lo >= hi - lo && top != 0.0f;
 }
 
 // Eight signed code bytes as bf16 (|value| <= 128: exact), the bits `flip` of
@@ -264,32 +250,12 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
 #pragma unroll
             for (int q = 0; q < 4; ++q) d.x[i][q] = *reinterpret_cast<const f4_t*>(from.x[i][q] + 32 * b);
     };
-    // Those that need fp32 products are staged as 0, and multiplied after the
-    // loop; REST: those alone.
-    bool rest = false;
-    auto stage_x = [&](const Data& d, auto rest_c) {
-        constexpr bool REST = decltype(rest_c)::value;
-        bool f[MT][4], any = false;
+    auto stage_x = [&](const Data& d) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) any |= f[i][q] = needs_f32(d.x[i][q]);
-        auto put = [&](int i, int q, f4_t v) {  // row 8q + lane / 8 of the tile, unit lane % 8
-            *reinterpret_cast<f4_t*>(stage + i * 1024 + q * 256 + (st_w ^ (q & 1 ? 16u : 0u))) = v;
-        };
-        const f4_t none = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (REST || __any(any)) {
-            rest = true;
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) put(i, q, f[i][q] == REST ? d.x[i][q] : none);
-        } else {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) put(i, q, d.x[i][q]);
-        }
+            for (int q = 0; q < 4; ++q)  // row 8q + lane / 8 of the tile, unit lane % 8
+                *reinterpret_cast<f4_t*>(stage + i * 1024 + q * 256 + (st_w ^ (q & 1 ? 16u : 0u))) = d.x[i][q];
     };
     auto read_x = [&](int i, int s, float (&e)[8]) {
 #pragma unroll
@@ -301,7 +267,7 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
         }
     };
     auto multiply = [&](uint32_t b, const Data& d) {
-        stage_x(d, std::false_type{});
+        stage_x(d);
         b8_t w[2];
         float sc[2], cds, min;
         decode_group<FMT>(d.w, b, lh, flip, w, sc, cds, min);
@@ -343,15 +309,26 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
             if ((b += NW) >= end) break;
         }
     }
-    // the products left out above, in fp32 with the dequantised weights
-    if (rest) {
+    // Sums that are not finite again, in fp32 with the dequantised weights: an
+    // infinite activation is to give an infinity of the sign of the weight it meets
+    // (a centred code and the group's offset can have opposite ones), and a code
+    // times a huge one may have overflowed where the weight times it does not.
+    float odd = 0.0f;  // NaN if one is not
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) odd = fmaf(acc[i][v], 0.0f, odd);
+    if (__any(odd != 0.0f)) {
         uint32_t l = lane;  // opaque: the addresses are formed here again, not kept through the loop above
         asm volatile("" : "+v"(l));
         const Source from = source(l);
+        v16f t[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) t[i] = zero;
         for (uint32_t b = first + wave; b < end; b += NW) {
             Data d;
             load(from, b, d);
-            stage_x(d, std::true_type{});
+            stage_x(d);
             b8_t w[2];
             float sc[2], cds, min;
             decode_group<FMT>(d.w, b, lh, flip, w, sc, cds, min);
@@ -365,10 +342,15 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
                     for (int c = 0; c < 8; ++c) {
                         const float q = float(w[s][c]);
                         const float wd = kOffset<FMT> ? fmaf(sc[s], q, cds) - min : sc[s] * q;  // one rounding
-                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(e[c], wd, acc[i], 0, 0, 0);
+                        t[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(e[c], wd, t[i], 0, 0, 0);
                     }
                 }
         }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (!(fabsf(acc[i][v]) < __builtin_inff())) acc[i][v] = t[i][v];
     }
     // the waves' sums, added in wave order (a wave's own region: no wait before)
     float* Y = split ? tasks.partial + size_t(split - 1) * M * N : tasks.y[t];
