@@ -1,8 +1,8 @@
 """The fp32-activation GEMMs (zq_gemm_split.hip on split f16 activations,
-zq_gemm_skinny.hip for few tokens): edges of their tiles and K splits, rows of very different magnitude, and
-non-finite activations; and, on the CPU, that its kernels neither spill nor
-use packed fp32 arithmetic."""
-import ctypes
+zq_gemm_skinny.hip for few tokens): edges of their tiles and K splits, a
+workspace for some of the tokens, rows of very different magnitude, non-finite
+and extreme activations, the rounding's common part; and, on the CPU, that the
+kernels neither spill nor use packed fp32 arithmetic."""
 import os
 import re
 import subprocess
@@ -13,6 +13,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from oracle import oracle as O
+from tests.plans import launch_split, split_bytes, split_plan, takes_split
 from tests.tolerance import assert_close
 
 ALL = (O.Q8_0, O.Q4_0, O.Q6_K, O.Q4_K, O.Q5_K)
@@ -25,10 +26,10 @@ def small(zq):
     zq.set_min_elements(old)
 
 
-# Tiles are 128 tokens by 128 or 256 rows (32 or 64 by 32 for few tokens),
-# stages 32 k (three in flight), super-blocks 256: one of each, one less and one
-# more, an odd count of stages, one stage, fewer groups than waves, and K long
-# enough to split.
+# Whichever kernel the dispatch takes (mostly the few-token one: 32 or 64 tokens
+# by 32 rows): one tile, one less and one more, an odd count of groups, fewer
+# groups than waves, and K long enough to split.  The split kernels' own edges
+# are below.
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ALL)
 @pytest.mark.parametrize("m,n,blocks", [(1, 1, 8), (2, 129, 8), (127, 255, 8), (128, 256, 16), (129, 257, 24), (257, 130, 8),
@@ -57,13 +58,13 @@ def test_any_number_of_blocks(zq, orc, small, fmt, m, blocks):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(140, 700, 2048), (20, 70, 512)])  # split activations; few tokens
+@pytest.mark.parametrize("m,n,k,split", [(140, 700, 2048, False), (20, 70, 512, False), (140, 700, 4096, True)])
 @pytest.mark.parametrize("fmt", ALL)
-def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k):
+def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k, split):
     """Each row has its own power of two, so a row's result does not depend on
-    its scale; an infinite or NaN activation stays in its row, and with codes
-    of one plane and no offset gives what the product of the dequantised
-    weights gives."""
+    its scale; an infinite or NaN activation stays in its row, and an infinite
+    one gives what the products of the dequantised weights give."""
+    assert takes_split(zq, fmt, m, n, k) == split
     w = orc.gen_weights(fmt, 520, n, k)
     X = orc.gen_normal(521, m * k).reshape(m, k)
     base = zq.gemm(fmt, w, X, m, n, k, zq.ACT_F32).reshape(m, n)
@@ -79,14 +80,66 @@ def test_row_magnitudes_and_non_finite(zq, orc, small, fmt, m, n, k):
     assert np.array_equal(got[3], base[3] * np.float32(2.0 ** -100)) and np.array_equal(got[4], base[4] * np.float32(2.0 ** 90))
     assert np.all(got[5] == 0) and np.all(np.isfinite(got[6]))
     assert np.all(np.isnan(got[9]))
-    assert not np.isfinite(got[7:9]).any()
-    if fmt in (O.Q8_0, O.Q4_0):
-        W = orc.dequantize(fmt, w, n * k).reshape(n, k)
-        with np.errstate(invalid="ignore"):
-            for r, c in ((7, 17), (8, 300)):
-                want = Z[r, c] * W[:, c]  # the finite terms do not matter beside it
-                assert np.array_equal(got[r], want, equal_nan=True)
+    W = orc.dequantize(fmt, w, n * k).reshape(n, k)
+    with np.errstate(invalid="ignore"):
+        for r, c in ((7, 17), (8, 300)):
+            want = Z[r, c] * W[:, c]  # the finite terms do not matter beside it
+            assert np.array_equal(got[r], want, equal_nan=True)
     zq.release(w)
+
+
+# The split kernels, called directly: tiles are 128 tokens by 128 or 256 rows,
+# stages 32 k with three in flight, super-blocks 256.  (tokens, rows, tile
+# columns): one tile, one less and one more of each, and grids of two rounds of
+# 128-column tiles, which take the 256-column form.  Q8_0 / Q4_0 take any count
+# of blocks (the main loop is six stages long, and one or two are fewer than it
+# has in flight); the others whole super-blocks.
+def split_case(zq, orc, fmt, m, n, blocks, planes, room=None):
+    """Result and launches against the float64 product (the GEMM bar; the fp32
+    oracle's own rounding takes up to 0.96 of it at long K)."""
+    k = 32 * blocks
+    w = orc.gen_weights(fmt, 550 + n, n, k)
+    X = orc.gen_normal(551 + m, m * k)
+    dw = torch.full((zq.weight_bytes(fmt, n, k),), 255, dtype=torch.uint8, device="cuda:0")
+    dw[: w.size] = torch.from_numpy(w).to("cuda:0")
+    Y = torch.full((m * n + 64,), 7.0, device="cuda:0")
+    ws_bytes = split_bytes(zq, fmt, room or m, k) + planes * m * n * 4
+    ws = torch.full((ws_bytes + 256,), 255, dtype=torch.uint8, device="cuda:0")
+    launches = launch_split(zq, fmt, dw, torch.from_numpy(X).to("cuda:0"), Y, ws, ws_bytes, m, n, k)
+    W = orc.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
+    want = X.reshape(m, k).astype(np.float64) @ W.T
+    assert bool((Y[m * n:] == 7.0).all()) and bool((ws[ws_bytes:] == 255).all())
+    assert_close(Y[: m * n].cpu().numpy(), want.reshape(-1), f"fmt={fmt} {m}x{n}x{k}")
+    return launches
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ALL)
+@pytest.mark.parametrize("m,n,cols", [(1, 1, 128), (127, 129, 128), (128, 128, 128), (129, 255, 128), (257, 270, 128),
+                                      (255, 16639, 256), (257, 11009, 256), (129, 16641, 256), (256, 16640, 256)])
+def test_split_tiles(zq, orc, fmt, m, n, cols):
+    counts = (1, 2, 3, 5, 7, 31, 67) if fmt in (O.Q8_0, O.Q4_0) else (8, 16, 24, 72)
+    for blocks in counts[:3] if cols == 256 else counts:
+        assert split_plan(zq, fmt, m, n, 32 * blocks, 0) == (cols, 1)
+        assert split_case(zq, orc, fmt, m, n, blocks, 0) == 2
+
+
+# K splits: even, with a last one that is shorter, and the most
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ALL)
+@pytest.mark.parametrize("m,n,blocks,planes", [(130, 40, 264, 3), (130, 1500, 128, 5), (1, 33, 448, 31)])
+def test_split_k(zq, orc, fmt, m, n, blocks, planes):
+    assert split_plan(zq, fmt, m, n, 32 * blocks, planes)[1] > 1
+    assert split_case(zq, orc, fmt, m, n, blocks, planes) == 3
+
+
+# room for the split activations of `room` tokens: the others follow, on the
+# few-token kernel (one launch) or on the split one again (two)
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ALL)
+@pytest.mark.parametrize("m,n,room,launches", [(300, 700, 256, 3), (129, 33, 128, 3), (500, 9000, 256, 4)])
+def test_room_for_some_tokens(zq, orc, fmt, m, n, room, launches):
+    assert split_case(zq, orc, fmt, m, n, 16, 0, room) == launches
 
 
 def extremes(orc, fmt, w, m, n, k):
@@ -132,21 +185,6 @@ def check_extremes(orc, fmt, w, X, got, m, n, k):
             mag = (np.abs(X[r].astype(np.float64)) * top).sum(1)[finite]
             err = np.abs(got[r][finite].astype(np.float64) - want[finite])
             assert np.all(err <= (8 + k ** 0.5) * 2.0 ** -24 * mag), f"row {r}: {np.nanmax(err / mag) * 2.0 ** 24} roundings"
-
-
-class SkinnyPlan(ctypes.Structure):
-    _fields_ = [("ks", ctypes.c_uint32), ("us", ctypes.c_double)]
-
-
-def takes_split(zq, fmt, m, n, k, ws_bytes):
-    """Whether the library's planners send this call to the split kernels (else
-    to the few-token kernel): the comparison launch_gemm_f32_batch makes."""
-    L, z = zq.lib(), ctypes.c_size_t
-    skinny, split = L._ZN2zq20plan_gemm_skinny_f32Eimmmm, L._ZN2zq13gemm_split_usEimmmPKvm
-    skinny.restype, skinny.argtypes = SkinnyPlan, [ctypes.c_int, z, z, z, z]
-    split.restype, split.argtypes = ctypes.c_double, [ctypes.c_int, z, z, z, ctypes.c_void_p, z]
-    use = min(ws_bytes, zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32))
-    return skinny(fmt, m, n, k, use // (m * n * 4)).us > split(fmt, m, n, k, 256 if use else None, use)
 
 
 def run_dev(zq, fmt, w, X, m, n, k, ws_bytes):

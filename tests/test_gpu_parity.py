@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
+from tests.plans import takes_split
 from tests.tolerance import assert_close
 
 pytestmark = pytest.mark.gpu
@@ -368,14 +369,14 @@ def test_gemm_f32(zq, orc, fmt, m, n, k):
     zq.release(w)
 
 
+@pytest.mark.parametrize("m,n,k,split", [(37, 70, 2048, False), (140, 700, 4096, True)])
 @pytest.mark.parametrize("fmt", [O.Q6_K, O.Q4_K, O.Q5_K])
-def test_superblock_gemm_mixed_scales(zq, orc, fmt):
+def test_superblock_gemm_mixed_scales(zq, orc, fmt, m, n, k, split):
     """Super-blocks of one weight row whose d (and dmin) lie 1 to 1e5 times below
-    the row's largest, and an all-zero row, through the f16-MFMA GEMM (explicit
-    workspace): it scales each weight row by one power of two taken from its
-    largest super-block, so the small super-blocks carry fewer bits in their low
-    halves and must still meet the fp32 bar against the reference arithmetic."""
-    m, n, k = 37, 70, 2048
+    the row's largest, and an all-zero row, on the few-token kernel (d and dmin in
+    each group's scale and offset) and on the split one (d and dmin applied where a
+    super-block is closed): the small super-blocks must still meet the fp32 bar
+    against the reference arithmetic."""
     w = orc.gen_weights(fmt, 4242, n, k).copy()
     bb = {O.Q6_K: 210, O.Q4_K: 144, O.Q5_K: 176}[fmt]
     doff = 208 if fmt == O.Q6_K else 0
@@ -393,6 +394,7 @@ def test_superblock_gemm_mixed_scales(zq, orc, fmt):
     X = orc.gen_normal(4243, m * k)
     Y = torch.empty(m * n, device=DEV)
     wsb = zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32)
+    assert takes_split(zq, fmt, m, n, k, wsb) == split
     ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device=DEV)
     zq.gemm_dev(fmt, dev_weights(zq, fmt, w, n, k), to_dev(X), Y, m, n, k, zq.ACT_F32, ws, wsb)
     got = Y.cpu().numpy()
@@ -402,8 +404,9 @@ def test_superblock_gemm_mixed_scales(zq, orc, fmt):
 
 # The BASELINE configs' own GEMM workloads at full size: config 2 (Q8_0, int8
 # activations, M = 32 / 128 / 512 / 2048 on both FFN shapes) and config 3
-# (Q4_0 int8 and Q6_K fp32 at M = 512), plus the Q4_K / Q5_K fp32 path at
-# M = 512.  Every M of the sweep runs on both shapes (M = 32 takes the skinny
+# (Q4_0 int8 and Q6_K fp32 at M = 512), plus the fp32 path of the other formats
+# at M = 512 and, with 1000 tokens of Q8_0, of a workspace that holds the split
+# activations of some of them only.  Every M of the sweep runs on both shapes (M = 32 takes the skinny
 # kernel, 448 row tiles at 14336 rows; M = 2048 at K = 14336 the 128-token
 # tile over 448 K blocks).  Rows and tokens are independent, so
 # sampled (token, row) outputs are checked against the oracle.
@@ -413,7 +416,8 @@ _FULL_GEMM = [(O.Q8_0, 1, 2048, 14336, 4096), (O.Q8_0, 1, 2048, 4096, 14336),
               (O.Q8_0, 1, 512, 14336, 4096), (O.Q8_0, 1, 512, 4096, 14336),
               (O.Q4_0, 1, 512, 14336, 4096), (O.Q4_0, 1, 512, 4096, 14336),
               (O.Q6_K, 2, 512, 14336, 4096), (O.Q6_K, 2, 512, 4096, 14336),
-              (O.Q4_K, 2, 512, 14336, 4096), (O.Q4_K, 2, 512, 4096, 14336), (O.Q5_K, 2, 512, 4096, 14336)]
+              (O.Q4_K, 2, 512, 14336, 4096), (O.Q4_K, 2, 512, 4096, 14336), (O.Q5_K, 2, 512, 4096, 14336),
+              (O.Q8_0, 2, 512, 14336, 4096), (O.Q4_0, 2, 512, 4096, 14336), (O.Q8_0, 2, 1000, 4096, 14336)]
 
 
 @pytest.mark.parametrize("fmt,act,m,n,k", _FULL_GEMM)
@@ -423,6 +427,7 @@ def test_gemm_full_size_sampled(zq, orc, fmt, act, m, n, k):
     X = orc.gen_normal(82 + m, m * k)
     Y = torch.empty(m * n, device=DEV)
     ws_bytes = zq.gemm_workspace_bytes(fmt, m, n, k, act)
+    assert act == zq.ACT_INT8 or takes_split(zq, fmt, m, n, k, ws_bytes)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=DEV)
     zq.gemm_dev(fmt, wd, to_dev(X), Y, m, n, k, act, ws, ws_bytes)
     Yh = Y.cpu().numpy().reshape(m, n)

@@ -11,7 +11,7 @@
 // Bound: the matrix cores at the chip's power limit.  With random data the clock
 // falls to ~1.5 GHz, and a loop of these MFMAs with the stage's LDS reads and
 // VALU work reaches 1.3-1.4 PF of f16 products; the kernels run at 0.8-0.9 PF.
-// A tile of 128 x 256 (128 x 128 for small grids, see plan_split) because the
+// A tile of 128 x 256 (128 x 128 for small grids, see plan_gemm_split) because the
 // next operand reads, the staging and the scale FMAs of a stage then just fit
 // between its MFMAs.  Measured, fp32-MFMA or three-product f16 kernel -> here:
 //   Q8_0  512 x 14336 x 4096   555 -> 151 us (108 -> 398 TFLOP/s of the GEMM)
@@ -817,16 +817,11 @@ static double split_cost(bool super, int wn, uint32_t tiles, uint32_t ks, uint32
     const double t = rounds * blocks * (wn == 4 ? (super ? 1.4 : 1.17) : (super ? 1.02 : 0.60));
     return ks > 1 ? t + 3.0 + double(ks - 1) * double(M) * double(N) * 8.0 / 4.0e6 : t;
 }
-struct SplitPlan {
-    int wn = 4;           // waves per tile row: 4 (256 columns) or 2 (128)
-    uint32_t ks = 1;      // K splits
-    uint32_t blocks = 0;  // blocks per split
-    double us = 1e300;    // estimated kernel time
-};
 // The cheapest tile width and split with at most `planes` planes beside Y;
 // splits are whole super-blocks where the format has them, and at least 8
 // blocks.
-static SplitPlan plan_split(bool super, size_t M, size_t N, size_t K, size_t planes) {
+SplitPlan plan_gemm_split(int fmt, size_t M, size_t N, size_t K, size_t planes) {
+    const bool super = fmt != kQ8_0 && fmt != kQ4_0;
     const uint32_t unit = super ? 8 : 1, units = uint32_t(K / 32) / unit;
     const uint32_t most = uint32_t(std::min<size_t>({planes + 1, 32, std::max(1u, units * unit / 8)}));
     SplitPlan best;
@@ -912,7 +907,7 @@ double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size
     }
     // beside the GEMM: two launches and the activations read and written once
     return 8.0 + double(M) * double(K) * 8.0 / 4.0e6 +
-           plan_split(fmt != kQ8_0 && fmt != kQ4_0, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float))).us;
+           plan_gemm_split(fmt, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float))).us;
 }
 
 hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
@@ -940,7 +935,7 @@ hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y
     int* ex = reinterpret_cast<int*>(ss + (sums ? M * (K / 256) * 32 : 0));
     const SplitArgs a{w, xs, ss, ex, X, Y, reinterpret_cast<float*>(xs + sb), uint32_t(M), uint32_t(N), uint32_t(K), stream};
     const SplitPlan plan =
-        plan_split(fmt != kQ8_0 && fmt != kQ4_0, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float)));
+        plan_gemm_split(fmt, M, N, K, (ws_bytes - sb) / (M * N * sizeof(float)));
     if (sums)
         hipLaunchKernelGGL(split_acts_kernel<true>, dim3(a.m), dim3(kThreads), 0, stream, X,
                            reinterpret_cast<_Float16*>(xs), ex, reinterpret_cast<_Float16*>(ss), a.k);

@@ -134,10 +134,18 @@ hipError_t launch_gemm_f32_batch(int fmt, const uint8_t* const* w, float* const*
 
 // The fp32-activation GEMM on the f16 matrix cores over split activations
 // (zq_gemm_split.hip); hipErrorInvalidConfiguration when the format, shape or
-// workspace is not covered.  gemm_split_us: its estimated time (infinite when
-// not covered).
+// workspace is not covered.  plan_gemm_split: the tile and K splits for at most
+// `planes` planes beside Y; gemm_split_us: the call's estimated time (infinite
+// when not covered).
 bool gemm_split_supported(int fmt, size_t K);
 size_t gemm_split_bytes(int fmt, size_t M, size_t K);
+struct SplitPlan {
+    int wn = 4;           // waves per tile row: 4 (256 columns) or 2 (128)
+    uint32_t ks = 1;      // K splits
+    uint32_t blocks = 0;  // blocks per split
+    double us = 1e300;    // estimated kernel time
+};
+SplitPlan plan_gemm_split(int fmt, size_t M, size_t N, size_t K, size_t planes);
 double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size_t ws_bytes);
 hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y, void* ws, size_t ws_bytes, size_t M,
                              size_t N, size_t K, hipStream_t stream, uint32_t* launches = nullptr);
