@@ -62,11 +62,12 @@ def test_down_stores_the_residual_sum(zq, orc, fmt, hidden, ffn):
 
 
 @pytest.mark.parametrize("ffn", (4096, 4352, 14336))  # down on the fp32 and the MFMA streaming kernel
-@pytest.mark.parametrize("u0", (np.inf, 3e11))
+@pytest.mark.parametrize("u0", (np.inf, 3e11, np.nan))
 def test_a_huge_activation_in_front_of_down(zq, orc, ffn, u0):
-    """One SiLU * up is infinite, or far above the others of its pair: the outputs
-    are infinite with the sign of the down weight it meets (NaN at a zero one),
-    and where every weight it meets is 0 the others keep fp32's precision."""
+    """One SiLU * up is infinite, far above the others of its pair, or NaN (an
+    infinite up and a gate of -inf): the outputs are infinite with the sign of the
+    down weight it meets (NaN at a zero one), keep fp32's precision for the others
+    where every weight it meets is 0, or are all NaN."""
     hidden, aw, r0, c0 = 512, 256, 70, 33
     w = {k: orc.gen_weights(O.Q8_0, s, r, c) for k, s, r, c in
          (("o", 910, hidden, aw), ("g", 911, ffn, hidden), ("u", 912, ffn, hidden), ("d", 913, hidden, ffn))}
@@ -82,9 +83,12 @@ def test_a_huge_activation_in_front_of_down(zq, orc, ffn, u0):
     w["u"].reshape(-1, hidden // 32, 34)[r0, c0 // 32, :2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
     if np.isfinite(u0):
         code("d", ffn, slice(None), r0)[:] = 0
+    if np.isnan(u0):
+        code("g", hidden, slice(r0, r0 + 1), c0)[:] = -100 & 255
+        w["g"].reshape(-1, hidden // 32, 34)[r0, c0 // 32, :2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
     x, nw, a = orc.gen_normal(914, hidden), orc.gen_normal(915, hidden), np.zeros(aw, np.float32)
     x[c0] = 1.0
-    nw[c0] = 3e38 if np.isinf(u0) else u0 / 100
+    nw[c0] = u0 / 100 if np.isfinite(u0) else 3e38
     shapes = {"o": (hidden, aw), "g": (ffn, hidden), "u": (ffn, hidden), "d": (hidden, ffn)}
     dev = {k: torch.zeros(zq.weight_bytes(O.Q8_0, r, c), dtype=torch.uint8, device=DEV) for k, (r, c) in shapes.items()}
     for k in dev:
@@ -97,13 +101,15 @@ def test_a_huge_activation_in_front_of_down(zq, orc, ffn, u0):
     h1 = x.astype(np.float64)
     h2 = (h1 / np.sqrt((h1 * h1).mean() + 1e-5)).astype(np.float32) * nw  # fp32: up's sum overflows as there
     with np.errstate(all="ignore"):
-        g, u = W["g"] @ h2, (W["u"] @ h2).astype(np.float32).astype(np.float64)
+        g, u = ((W[p] @ h2).astype(np.float32).astype(np.float64) for p in "gu")
         f = g / (1.0 + np.exp(-g)) * u
         terms = W["d"] * f
         want, mag = h1 + terms.sum(1), np.abs(h1) + np.abs(terms).sum(1)
     got = out.double().cpu().numpy()
-    assert np.isinf(u[r0]) == np.isinf(u0) and np.isfinite(np.delete(u, r0)).all() and abs(u[r0]) > 1e8
-    if np.isinf(u0):
+    assert np.isfinite(np.delete(f, r0)).all() and abs(u[r0]) > 1e8 and np.isfinite(u[r0]) == np.isfinite(u0)
+    if np.isnan(u0):
+        assert np.isnan(f[r0]) and np.isnan(got).all()
+    elif np.isinf(u0):
         assert np.array_equal(got, want, equal_nan=True) and np.isinf(got).any()
     else:  # the GEMV bar, as above
         assert np.all(np.abs(got - want) <= 1e-4 + 1e-5 * mag)

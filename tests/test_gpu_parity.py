@@ -202,6 +202,18 @@ print('ok')
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout + r.stderr
 
 
+# the MFMA and the fp32 streaming kernels, rows that are not whole 16-byte units
+@pytest.mark.parametrize("rows,cols", [(40, 4352), (9000, 1280), (40, 1280), (4099, 5120 + 32)])
+@pytest.mark.parametrize("fmt", [O.Q8_0, O.Q4_0])
+def test_gemv_one_nan_reaches_every_row(zq, orc, fmt, rows, cols):
+    w = orc.gen_weights(fmt, 7, rows, cols)
+    x = orc.gen_normal(8, cols)
+    x[1000] = np.nan
+    y = torch.zeros(rows, device=DEV)
+    zq.gemv_dev(fmt, dev_weights(zq, fmt, w, rows, cols), to_dev(x), y, rows, cols)
+    assert torch.isnan(y).all()
+
+
 def test_residency_budget_eviction_within_a_call(zq, orc):
     """Calls that read several host weights resolve all of them before any
     launch.  With the residency budget lowered to about 2.7 weights: a batch

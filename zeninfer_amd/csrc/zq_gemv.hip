@@ -1433,7 +1433,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
         am = fmaxf(am, dpp_f<kDppXor2>(am));
         am = fmaxf(am, dpp_f<kDppHalfMirror>(am));
         am = fmaxf(am, dpp_f<kDppMirror>(am));
-        bad |= !(am <= 3.402823466e38f);  // inf or NaN
+        // an infinity; a NaN, which the maxima pass over
+        bad |= !(am <= 3.402823466e38f) || __builtin_isunordered(t.x, t.y) || __builtin_isunordered(t.z, t.w);
         if constexpr (RES) {
             const float low = am * 0x1p-20f;
             auto far = [&](float v) { return v != 0.0f && fabsf(v) < low ? 1.0f : 0.0f; };
