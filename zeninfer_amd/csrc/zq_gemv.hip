@@ -1437,13 +1437,15 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
         bad |= !(am <= 3.402823466e38f) || __builtin_isunordered(t.x, t.y) || __builtin_isunordered(t.z, t.w);
         if constexpr (RES) {
             const float low = am * 0x1p-20f;
-            auto far = [&](float v) { return v != 0.0f && fabsf(v) < low ? 1.0f : 0.0f; };
-            float c = (far(t.x) + far(t.y)) + (far(t.z) + far(t.w));
-            c += dpp_f<kDppXor1>(c);
-            c += dpp_f<kDppXor2>(c);
-            c += dpp_f<kDppHalfMirror>(c);
-            c += dpp_f<kDppMirror>(c);
-            bad |= c >= 16.0f;
+            if (__any(fminf(fminf(fabsf(t.x), fabsf(t.y)), fminf(fabsf(t.z), fabsf(t.w))) < low)) {  // seldom: count
+                auto far = [&](float v) { return v != 0.0f && fabsf(v) < low ? 1.0f : 0.0f; };
+                float c = (far(t.x) + far(t.y)) + (far(t.z) + far(t.w));
+                c += dpp_f<kDppXor1>(c);
+                c += dpp_f<kDppXor2>(c);
+                c += dpp_f<kDppHalfMirror>(c);
+                c += dpp_f<kDppMirror>(c);
+                bad |= c >= 16.0f;
+            }
         }
         const int s = 30 - (am > 0.0f && am <= 3.402823466e38f ? __builtin_amdgcn_frexp_expf(am) : 0);
         const uint32_t y0 = uint32_t(int(ldexpf(t.x, s))) + 0x80808080u;
