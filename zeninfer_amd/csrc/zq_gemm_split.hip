@@ -94,8 +94,17 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
             split(f[k], a, b);
             h[k] = a;
             l[k] = b;
-            const float t = fabsf(f[k]);
-            wide += t == __builtin_inff() ? 1e9f : t == 0.0f ? 0.0f : t < 0x1p-6f ? 3.0f : -1.0f;
+        }
+        const float least = fminf(fminf(fabsf(f[0]), fabsf(f[1])), fminf(fabsf(f[2]), fabsf(f[3])));
+        const float most = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
+        if (__any(least < 0x1p-6f || most == __builtin_inff())) {  // seldom: one by one
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float t = fabsf(f[k]);
+                wide += t == __builtin_inff() ? 1e9f : t == 0.0f ? 0.0f : t < 0x1p-6f ? 3.0f : -1.0f;
+            }
+        } else {
+            wide -= 4.0f;
         }
         _Float16* d = o + size_t(i >> 3) * 64 + (i & 7u) * 4;
         *reinterpret_cast<h4_t*>(d) = h;
@@ -223,29 +232,37 @@ __device__ __forceinline__ void store_tile(v16f (&acc)[2][2], const int* __restr
     uint32_t lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));  // opaque: nothing below is formed before the main loop
     const uint32_t l32 = lane & 31, lh = lane >> 5;
+    // the exponents of rows l32 and 32 + l32, passed between lanes: one wait for them
+    int er[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) er[i] = ex[min(m0 + i * 32 + l32, M - 1)];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const uint32_t r = min(m0 + i * 32 + l32, M - 1);
-        if (__any(ex[r] == kExactRow)) {
-            const float* x = X + size_t(r) * K + 16 * lh;
+        int ev[16];
+#pragma unroll
+        for (uint32_t v = 0; v < 16; ++v) ev[v] = __shfl(er[i], 8 * (v >> 2) + 4 * lh + (v & 3));
+        if (__any(er[i] == kExactRow)) {
+            const float* x = X + size_t(min(m0 + i * 32 + l32, M - 1)) * K + 16 * lh;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const uint32_t n = min(n0 + j * 32 + l32, N - 1);
                 const v16f t = exact_tile(x, b_begin, b_end, [&](uint32_t b, float (&w)[16]) { load(n, lh, b, w); });
 #pragma unroll
                 for (int v = 0; v < 16; ++v)
-                    if (ex[min(m0 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3), M - 1)] == kExactRow) acc[i][j][v] = t[v];
+                    if (ev[v] == kExactRow) acc[i][j][v] = t[v];
             }
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (ev[v] == kExactRow) ev[v] = 0;
         }
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const uint32_t m = m0 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
             if (m >= M) continue;
-            const int e = ex[m] == kExactRow ? 0 : -ex[m];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const uint32_t n = n0 + j * 32 + l32;
-                if (n < N) Y[size_t(m) * N + n] = ldexpf(acc[i][j][v], e);
+                if (n < N) Y[size_t(m) * N + n] = ldexpf(acc[i][j][v], -ev[v]);
             }
         }
     }
