@@ -414,7 +414,13 @@ def _task_table(types, task, flat):
     """ctypes array of {address, address, count} tasks from their flat values (taken modulo 2^64, as ctypes does)."""
     n = len(flat) // 3
     t = types[n] if n < len(types) else task * n
-    return t.from_buffer_copy(struct.pack("=%dQ" % len(flat), *[v & _U64 for v in flat])) if n else t()
+    if not n:
+        return t()
+    try:
+        raw = struct.pack("=%dQ" % len(flat), *flat)
+    except struct.error:  # a value past either end
+        raw = struct.pack("=%dQ" % len(flat), *[v & _U64 for v in flat])
+    return t.from_buffer_copy(raw)
 
 
 def gemv_dev(fmt, w, x, y, rows, cols, stream=None):
