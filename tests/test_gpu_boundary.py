@@ -282,3 +282,53 @@ def test_device_calls_under_graph_capture(zq, orc):
             assert torch.isfinite(ref[key]).all(), key
             assert torch.equal(cap[key], ref[key]), f"graph replay {rep} differs from eager: {key}"
     assert torch.equal(cap["noalloc"], cap["gemm"])
+
+
+def test_host_gemm_without_memory_for_the_faster_workspace(zq, tmp_path):
+    """A host GEMM with fp32 activations runs where the device has memory for the
+    workspace that a device-pointer caller is asked for, but not for the larger one
+    of the faster kernels.  A stand-in for hipMalloc refuses the larger size, in a
+    process of its own (loaded before the library, its symbol is found first)."""
+    import os, subprocess, sys
+    src, shim = tmp_path / "limit.c", tmp_path / "liblimit.so"
+    src.write_text("""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+size_t limit = (size_t)-1, refused = 0;
+int hipMalloc(void** p, size_t n) {
+    static int (*real)(void**, size_t);
+    if (n > limit) { refused = n; return 2; }
+    if (!real) real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so", RTLD_NOW | RTLD_NOLOAD), "hipMalloc");
+    return real(p, n);
+}
+""")
+    hip = [l.split()[2] for l in subprocess.run(["ldd", os.environ.get("ZQ_HIP_LIB", zq.LIB)], capture_output=True, text=True,
+                                                check=True).stdout.splitlines() if "libamdhip64" in l][0]
+    src.write_text(src.read_text().replace('"libamdhip64.so"', f'"{os.path.realpath(hip)}"'))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(shim), str(src), "-ldl"], check=True)
+    code = f"""
+import ctypes, sys, numpy as np
+sys.path.insert(0, {os.getcwd()!r})
+shim = ctypes.CDLL({str(shim)!r}, ctypes.RTLD_GLOBAL)
+limit, refused = (ctypes.c_size_t.in_dll(shim, n) for n in ('limit', 'refused'))
+from oracle import oracle as O
+from zeninfer_amd import zq
+from tests.tolerance import assert_close
+o = O.Oracle(); zq.init(); zq.set_min_elements(0)
+for fmt, m, n, k in ((O.Q8_0, 1100, 2048, 1024), (O.Q4_K, 1100, 2048, 1024)):
+    w = o.gen_weights(fmt, 3, n, k); X = o.gen_normal(4, m * k)
+    zq.gemm(fmt, w, X[:k], 1, n, k, zq.ACT_F32)  # the weights are on the device
+    asked = zq.gemm_workspace_bytes(fmt, m, n, k, zq.ACT_F32)
+    limit.value, refused.value = 4 * m * (n + k) + asked + 512, 0
+    Y = zq.gemm(fmt, w, X, m, n, k, zq.ACT_F32)
+    assert refused.value > limit.value
+    W = o.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
+    assert_close(Y, (X.reshape(m, k).astype(np.float64) @ W.T).reshape(-1), str(fmt))
+    limit.value = 2 ** 64 - 1
+    assert_close(zq.gemm(fmt, w, X, m, n, k, zq.ACT_F32), Y.astype(np.float64), str(fmt))
+    zq.release(w); zq.shutdown()
+print('ok')
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and "ok" in r.stdout, r.stdout + r.stderr

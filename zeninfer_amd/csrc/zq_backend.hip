@@ -698,10 +698,20 @@ int gemm_batch_locked(Backend& b, int fmt, const float* X, const zq_gemm_task* t
         ybytes += align_up(tokens * rows[i] * sizeof(float), 256);
         ymax = std::max(ymax, tokens * rows[i] * sizeof(float));
     }
-    size_t wsbytes = batch_workspace_bytes(fmt, rows, count, tokens, cols, act);
+    // the faster kernels' workspace where there is memory for it, else what a
+    // caller with device pointers is asked for
+    const size_t asked = batch_workspace_bytes(fmt, rows, count, tokens, cols, act);
+    size_t wsbytes = asked;
     if (act != ZQ_ACT_INT8)
         for (size_t i = 0; i < count; ++i) wsbytes = std::max(wsbytes, zq::gemm_f32_best_bytes(fmt, tokens, rows[i], cols));
     st = ensure_scratch(b, xbytes + ybytes + wsbytes, std::max(xbytes, ymax));
+    bool best = true;
+    if (st == ZQ_ERR_OOM && wsbytes > asked) {
+        (void)hipGetLastError();  // the failed allocation's, which a launch's check would find
+        best = false;
+        wsbytes = asked;
+        st = ensure_scratch(b, xbytes + ybytes + wsbytes, std::max(xbytes, ymax));
+    }
     if (st != ZQ_OK) return st;
     uint8_t* base = static_cast<uint8_t*>(b.dev_scratch);
     float* dx = reinterpret_cast<float*>(base);
@@ -716,7 +726,7 @@ int gemm_batch_locked(Backend& b, int fmt, const float* X, const zq_gemm_task* t
     if ((st = c.put(dx, X, tokens * cols * sizeof(float))) != ZQ_OK) return st;
     c.begin();
     uint64_t n = 0;
-    st = enqueue_gemm_batch(fmt, dw, dy, rows, count, dx, tokens, cols, act, ws, wsbytes, b.stream, &n, true);
+    st = enqueue_gemm_batch(fmt, dw, dy, rows, count, dx, tokens, cols, act, ws, wsbytes, b.stream, &n, best);
     if (st != ZQ_OK) {
         ++b.stats.errors;
         return st;
