@@ -19,10 +19,11 @@
 // dequantised weights (see the kernel).
 //
 // Bound: at a few tokens the launch and the chain of a wave's K groups (loads,
-// decoding, products; 16 and 8 waves sharing K measured the same), past ~100
-// tokens the VALU work of decoding each weight again for every 64 tokens, which
-// is where the estimates in plan_gemm_skinny_f32 and plan_split cross.  Q4_K,
-// 19 tokens, 4096 + 1024 + 1024 rows x 4096: 94 us in nine launches -> 17.3 in one.
+// decoding, products; 16 and 8 waves sharing K measured the same), at many the
+// VALU work of decoding each weight again for every 64 tokens.  Where the split
+// kernels are faster depends on rows, K and workspace as well as tokens: the
+// estimates of plan_gemm_skinny_f32 and plan_gemm_split.  Q4_K, 19 tokens, 4096 +
+// 1024 + 1024 rows x 4096: 94 us in nine launches -> 16.9 in one.
 #include "zq_device.hpp"
 #include "zq_internal.hpp"
 

@@ -8,16 +8,20 @@
 //  * the GEMM multiplies codes by hi and lo on v_mfma_f32_32x32x16_f16 (exact
 //    products, fp32 sums: two instructions where one fp32 MFMA of the same
 //    size would take sixteen) and applies the group scales in fp32.
-// Bound: the matrix cores at the chip's power limit.  With random data the clock
-// falls to ~1.5 GHz, and a loop of these MFMAs with the stage's LDS reads and
-// VALU work reaches 1.3-1.4 PF of f16 products; the kernels run at 0.8-0.9 PF.
+// Bound: the issue of what runs beside the MFMAs.  By the counters the matrix
+// cores are busy 42 % of the chip's cycles with Q8_0 512 x 14336 x 4096 (0.88 PF
+// of f16 products; 224 workgroups on 256 CUs), 54 % with Q6_K 1000 x 4096 x 14336
+// (1.05 PF), at 1.9-2.0 GHz; a loop of these MFMAs alone reaches 1.6 PF on random
+// data, where power takes the clock to 1.6 GHz, and 1.2 PF with 8 FMAs to each.
 // A tile of 128 x 256 (128 x 128 for small grids, see plan_gemm_split) because the
 // next operand reads, the staging and the scale FMAs of a stage then just fit
 // between its MFMAs.  Measured, fp32-MFMA or three-product f16 kernel -> here:
-//   Q8_0  512 x 14336 x 4096   555 -> 151 us (108 -> 398 TFLOP/s of the GEMM)
-//   Q6_K 1000 x 14336 x 4096   534 -> 379 us; 512 tokens 0.32-0.37 -> 0.22 ms
+//   Q8_0  512 x 14336 x 4096   555 -> 144-150 us (108 -> 400-417 TFLOP/s of the GEMM)
+//   Q6_K 1000 x 4096 x 14336   534 -> 370-380 us; 512 tokens 0.32-0.37 -> 0.22 ms
 //   Q4_K / Q5_K 512 x 14336 x 4096   0.29-0.32 -> 0.18 / 0.30-0.34 -> 0.19 ms
-// and an error against 64 bits that is no larger in any format.
+// and an error against 64 bits that is no larger in any format, of a single
+// product (Q8_0 4e-7..1.2e-6 -> 1.1e-7..3.5e-7, Q4_K 2.0e-7..2.2e-7 ->
+// 1.3e-7..2.1e-7) and of a decoder's logits.
 #include "zq_device.hpp"
 #include "zq_gemm_common.hpp"
 #include "zq_internal.hpp"
@@ -381,8 +385,8 @@ __device__ __forceinline__ void gemm_split_body(const uint8_t* W, const uint8_t*
     // a tile's 16 scaled additions follow in the next tile's four slots, and
     // the staging is spread over the slots, because a wave's VALU work runs
     // under its own MFMAs only where it is issued between them (measured: an
-    // MFMA and n VALU instructions take max(32, 8 + 4n) cycles).  PAR, the block's
-    // parity: the column order alternates so that the column read last is free first.
+    // MFMA with 4, 8, 16 FMAs behind it takes 38, 53, 89 cycles of a SIMD's one
+    // wave, 33, 43, 66 with two).  PAR, the block's parity: the column order alternates so that the column read last is free first.
     v16f p[2];        // products of a tile; p[1] enters a stage with the previous stage's last tile
     float dc = 0.0f;  // ... its scale
     float dt = 0.0f;  // the scale of a stage's last but one tile (its column's is replaced early)
