@@ -113,3 +113,32 @@ def test_a_huge_activation_in_front_of_down(zq, orc, ffn, u0):
         assert np.array_equal(got, want, equal_nan=True) and np.isinf(got).any()
     else:  # the GEMV bar, as above
         assert np.all(np.abs(got - want) <= 1e-4 + 1e-5 * mag)
+
+
+@pytest.mark.parametrize("ffn", (4352, 14336))
+def test_saturated_gates_stay_on_the_digits(zq, orc, ffn):
+    """Half of the gates are far below zero, so that nearly half of every pair's
+    SiLU * up is next to nothing beside the rest: the down projection is the MFMA
+    GEMV's as for any other x (launch_gemv's sums, bit for bit), not the fp32 form
+    of values that the digits do not carry, which is several times slower."""
+    hidden, aw = 512, 256
+    w = {k: orc.gen_weights(O.Q8_0, s, r, c) for k, s, r, c in
+         (("o", 920, hidden, aw), ("g", 921, ffn, hidden), ("u", 922, ffn, hidden), ("d", 923, hidden, ffn))}
+    dev = {}
+    for k, (r, c) in {"o": (hidden, aw), "g": (ffn, hidden), "u": (ffn, hidden), "d": (hidden, ffn)}.items():
+        dev[k] = torch.zeros(zq.weight_bytes(O.Q8_0, r, c), dtype=torch.uint8, device=DEV)
+        dev[k][: w[k].size] = torch.from_numpy(w[k]).to(DEV)
+    x = torch.from_numpy(orc.gen_normal(924, hidden)).to(DEV)
+    W = torch.from_numpy(orc.dequantize(O.Q8_0, w["g"], ffn * hidden).reshape(ffn, hidden))
+    nw = torch.full((hidden,), float(60.0 / (W @ x.cpu()).std()), device=DEV)  # gates of +-60
+    wsb = zq.ffn_residual_workspace_bytes(hidden, ffn)
+    ws, out = torch.empty(wsb, dtype=torch.uint8, device=DEV), torch.empty(hidden, device=DEV)
+    zq.ffn_residual_fused_dev(O.Q8_0, dev["o"], dev["g"], dev["u"], dev["d"], nw, x, torch.zeros(aw, device=DEV), out, hidden, aw,
+                              ffn, 1e-5, ws, wsb)
+    f = ws.view(torch.float32)[3 * hidden: 3 * hidden + ffn].clone()  # behind three hidden vectors: SiLU * up
+    pairs = f.abs().reshape(-1, 64)
+    far = ((pairs != 0) & (pairs < pairs.max(1, keepdim=True).values * 2.0 ** -20)).sum(1)
+    assert bool((far >= 16).any())
+    d = torch.empty(hidden, device=DEV)
+    zq.gemv_dev(O.Q8_0, dev["d"], f, d, hidden, ffn)
+    assert torch.equal(out, x + d)

@@ -1263,8 +1263,8 @@ __global__ __launch_bounds__(kThreads) void gemv_block_kernel(TaskTable tt, cons
 // so the decode tail after the last weight block shrinks.  Non-finite x makes
 // every output NaN.  With RES (the FFN step's down projection, whose other
 // forms multiply in fp32) x that X does not carry is multiplied in fp32
-// instead: a non-finite one, or a pair a quarter of whose elements lie 2^20
-// below its largest.
+// instead: a non-finite one, or a pair far above all others a quarter of whose
+// elements lie 2^20 below its largest.
 //
 // Work split: a wave owns a slice of 16 pairs (1024 columns) for the whole
 // kernel -- its digits stay in 16 VGPRs -- and each row block it streams
@@ -1423,7 +1423,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
     // their max comes from a 16-lane DPP reduction.  Digit j of the pair's
     // float4 e lands at dword p*68 + 4e + j (one 16 B write per float4; the
     // 68-dword pair stride makes the B reads below conflict-free).
-    int bad = 0;
+    int bad = 0, wide = 0;
 #pragma unroll
     for (int k = 0; k < XPT; ++k) {
         const uint32_t idx = threadIdx.x + uint32_t(k) * NT;
@@ -1444,10 +1444,11 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
                 c += dpp_f<kDppXor2>(c);
                 c += dpp_f<kDppHalfMirror>(c);
                 c += dpp_f<kDppMirror>(c);
-                bad |= c >= 16.0f;
+                wide |= c >= 16.0f;
             }
         }
-        const int s = 30 - (am > 0.0f && am <= 3.402823466e38f ? __builtin_amdgcn_frexp_expf(am) : 0);
+        // (a pair of zeros: an exponent below all others)
+        const int s = 30 - (am > 0.0f && am <= 3.402823466e38f ? __builtin_amdgcn_frexp_expf(am) : RES && am == 0.0f ? -200 : 0);
         const uint32_t y0 = uint32_t(int(ldexpf(t.x, s))) + 0x80808080u;
         const uint32_t y1 = uint32_t(int(ldexpf(t.y, s))) + 0x80808080u;
         const uint32_t y2 = uint32_t(int(ldexpf(t.z, s))) + 0x80808080u;
@@ -1466,9 +1467,23 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(TaskTable tt, const flo
             if (e == 0) sexp[p] = s;
         }
     }
-    const bool no_digits = __syncthreads_or(bad) != 0;
+    bool no_digits = __syncthreads_or(bad | wide) != 0;
     if constexpr (RES) {
-        if (no_digits) {  // the same in every workgroup: a wave per row
+        // A wide pair matters if what its digits drop, 2^-27 of its largest element,
+        // shows beside the rest of x: if the other pairs' largest elements together
+        // (root of the sum of squares, in powers of two) are below an eighth of it.
+        // Without this a few saturated gates, whose SiLU is next to nothing, sent
+        // ordinary steps the slow way (4096 / 13824: 47 -> 187 us).
+        if (no_digits) {  // the same in every wave and workgroup
+            int top = -1000;
+            for (uint32_t p = lane; p < pairs; p += 64) top = max(top, -sexp[p]);
+            top = int(wave_max(float(top)));
+            float q = 0.0f;
+            for (uint32_t p = lane; p < pairs; p += 64) q += ldexpf(1.0f, 2 * (-sexp[p] - top));
+            q = wave_sum(q);
+            no_digits = __syncthreads_or(bad) != 0 || q < 1.0f + 1.0f / 64;
+        }
+        if (no_digits) {  // a wave per row
             const GemvTask& t = tt.t[0];
             for (uint32_t row = blockIdx.x * NW + wave; row < t.rows; row += gridDim.x * NW) {
                 const float v = wave_sum(lane_dot<FMT>(t.w + size_t(row) * rb, x, cols, lane));
