@@ -13,10 +13,11 @@ DEV = "cuda:0"
 
 
 # (hidden, ffn): pair + fp32 store with 8 / 16 waves; pair + MFMA store at one
-# and four row blocks per workgroup and at its longest rows; pair + separate add
-# (ffn not whole 256); SiLU * up in front (hidden past 4096) with one, two and
+# and four row blocks per workgroup and at its most slices; gate|up on the MFMA
+# kernel (Q8_0; Q4_0 as before, at the longest rows); pair + separate add (ffn not
+# whole 256); SiLU * up in front (hidden past 4096) with one, two and
 # four slices per row; nothing fused (hidden not whole 256)
-@pytest.mark.parametrize("hidden,ffn", [(256, 256), (2304, 1024), (512, 4352), (4096, 8192), (768, 16384), (512, 2880),
+@pytest.mark.parametrize("hidden,ffn", [(256, 256), (2304, 1024), (512, 4352), (4096, 8192), (512, 16128), (768, 16384), (512, 2880),
                                         (4352, 512), (4352, 4352), (4352, 8448), (288, 512)])
 @pytest.mark.parametrize("fmt", (O.Q8_0, O.Q4_0))
 def test_down_stores_the_residual_sum(zq, orc, fmt, hidden, ffn):

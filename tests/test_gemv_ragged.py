@@ -92,7 +92,7 @@ def test_an_infinity_reaches_every_row(zq, orc, sb):
     assert not np.isfinite(y.cpu().numpy()).any()
 
 
-@pytest.mark.parametrize("hidden,ffn", [(256, 768), (2304, 2816), (5120, 1280)])
+@pytest.mark.parametrize("hidden,ffn", [(256, 768), (256, 8192), (2304, 2816), (5120, 1280)])
 def test_paired_gate_up(zq, orc, hidden, ffn):
     """ffn_residual_fused against separate calls (as for the other formats: the
     SiLU's expf and orders of addition, within the GEMV bar)."""

@@ -52,6 +52,9 @@ constexpr int kXPlain = 0, kSiluMul = 1, kAddNorm = 2;
 // kernels instead.
 hipError_t launch_gemv_prologue(int fmt, const GemvTask* tasks, int count, const XPrologue& pro, size_t cols,
                                 hipStream_t stream);
+// Whether launch_gemv_prologue takes `rows` (of all tasks) behind kAddNorm with
+// the MFMA kernel, where the operands are aligned.
+bool gemv_norm_on_mfma(int fmt, size_t cols, size_t rows);
 // y = res + W . x: the streaming kernel launch_gemv takes for the shape, so
 // the sums are its sums, with the add in its store.  Coverage as
 // launch_gemv_prologue's.
