@@ -225,6 +225,44 @@ def test_errors_have_no_common_part(zq, orc, fmt, m, n, k, split):
     assert abs(e.mean()) < 0.1 * np.sqrt((e * e).mean())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ALL)
+def test_rows_marked_for_fp32(zq, orc, fmt):
+    """Only rows that f16 hi + lo under one power of two do not carry are marked (the
+    rows' exponents follow the split activations in the workspace): not those with
+    many elements next to nothing, as SiLU leaves, or one 2^13 above the others, as
+    some models' activations have."""
+    m, n, k = 128, 40, 2048
+    w = orc.gen_weights(fmt, 560, n, k)
+    X = orc.gen_normal(561, m * k).reshape(m, k)
+    X[1, 7] = np.inf
+    X[2, 9] = 1e8
+    X[3, [9, 700, 701]] = 1e8, -1e8, 3e7
+    X[4, 9] = 1e5
+    X[5, ::2] *= 1e-12
+    X[6, :1900] *= 1e-12
+    X[7, 9] = 8000.0
+    X[8] = 0.0
+    X[9, 9] = np.nan
+    X[10] = np.exp2(-np.arange(k) % 60).astype(np.float32)  # evenly over 60 powers of two
+    X[11, 1:] = 0.0
+    marked = {1, 2, 3}
+    dw = torch.zeros(zq.weight_bytes(fmt, n, k), dtype=torch.uint8, device="cuda:0")
+    dw[: w.size] = torch.from_numpy(w).to("cuda:0")
+    nbytes = split_bytes(zq, fmt, m, k)
+    ws, Y = torch.zeros(nbytes, dtype=torch.uint8, device="cuda:0"), torch.empty(m * n, device="cuda:0")
+    launch_split(zq, fmt, dw, torch.from_numpy(X).to("cuda:0"), Y, ws, nbytes, m, n, k)
+    at = m * k * 4 + (m * (k // 256) * 32 if fmt in (O.Q4_K, O.Q5_K) else 0)
+    ex = ws[at: at + 4 * m].view(torch.int32).cpu().numpy()
+    assert set(np.flatnonzero(ex == 1 << 20)) == marked
+    rows = np.array([r for r in range(m) if r not in (1, 9)])  # the two are test_extreme_activations'
+    W = orc.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
+    Xr = X[rows].astype(np.float64)
+    mag = np.abs(Xr) @ np.abs(W).T + (fmt in (O.Q4_K, O.Q5_K)) * (np.abs(Xr).sum(1)[:, None] * np.abs(W).max())
+    err = np.abs(Y.cpu().numpy().reshape(m, n)[rows] - Xr @ W.T)
+    assert np.all(err <= (8 + k ** 0.5) * 2.0 ** -24 * mag)
+
+
 @pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))
 def test_generated_code(tmp_path, src):
     from zeninfer_amd.build import FLAGS, HIPCC, SRC

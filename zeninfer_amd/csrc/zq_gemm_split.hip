@@ -52,9 +52,12 @@ typedef uint32_t u4a4_t __attribute__((ext_vector_type(4), aligned(4)));
 // subnormal).  A NaN reaches every output of its row.  A row with an infinity
 // (whose products with a weight's parts can have opposite signs where the
 // weight's own sign decides), or with so large a span that 2^-40 of its maximum
-// shows (a quarter of its elements 2^20 below it: a huge one that meets a zero
-// code would leave the others with less than fp32's precision), is marked
-// instead: ex[r] = kExactRow, and exact_tile() multiplies it in fp32.
+// shows where its largest elements meet zero codes, is marked instead: ex[r] =
+// kExactRow, and exact_tile() multiplies it in fp32.  That is: the elements more
+// than 2^20 below the maximum, `lost` of them, lose up to 2^-25 each (scaled), and
+// this is set against fp32's rounding of the sum of those more than 2^8 below it
+// (the others may meet zeros): marked if the sum of their squares is under lost /
+// 16.  A row whose small elements are few, or that has others between, is not.
 constexpr int kExactRow = 1 << 20;
 __device__ __forceinline__ float finite_abs(float v) {
     const float a = fabsf(v);
@@ -81,7 +84,7 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, red[w]);
     const int e = m > 0.0f ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
-    float wide = 0.0f;  // > 0 for a row to mark
+    float lost = 0.0f;  // non-zero elements more than 2^20 below the maximum, 1e9 for an infinity
     _Float16* o = out + size_t(blockIdx.x) * K * 2;
     auto split = [](float f, _Float16& h, _Float16& l) {
         h = _Float16(f);
@@ -101,14 +104,12 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
         }
         const float least = fminf(fminf(fabsf(f[0]), fabsf(f[1])), fminf(fabsf(f[2]), fabsf(f[3])));
         const float most = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
-        if (__any(least < 0x1p-6f || most == __builtin_inff())) {  // seldom: one by one
+        if (__any(least < 0x1p-6f || most == __builtin_inff())) {  // seldom
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 const float t = fabsf(f[k]);
-                wide += t == __builtin_inff() ? 1e9f : t == 0.0f ? 0.0f : t < 0x1p-6f ? 3.0f : -1.0f;
+                lost += t == __builtin_inff() ? 1e9f : t != 0.0f && t < 0x1p-6f ? 1.0f : 0.0f;
             }
-        } else {
-            wide -= 4.0f;
         }
         _Float16* d = o + size_t(i >> 3) * 64 + (i & 7u) * 4;
         *reinterpret_cast<h4_t*>(d) = h;
@@ -124,11 +125,26 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
             }
         }
     }
-    wide = wave_sum(wide);  // whole numbers below 2^24, or past 2^28
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wide;
-    __syncthreads();
-    if (threadIdx.x == 0) ex[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]) > 0.0f ? kExactRow : e;
+    auto block_sum = [&](float v) {
+        v = wave_sum(v);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        return (red[0] + red[1]) + (red[2] + red[3]);
+    };
+    lost = block_sum(lost);  // whole numbers below 2^24, or past 2^28
+    bool exact = lost >= 1e9f;
+    if (lost > 0.0f && !exact) {
+        float low = 0.0f;
+        for (uint32_t i = threadIdx.x; i < K4; i += kThreads) {
+            const float4 v = r[i];
+            const float f[4] = {ldexpf(v.x, e), ldexpf(v.y, e), ldexpf(v.z, e), ldexpf(v.w, e)};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) low = fabsf(f[k]) < 0x1p6f ? fmaf(f[k], f[k], low) : low;
+        }
+        exact = block_sum(low) < 0.0625f * lost;
+    }
+    if (threadIdx.x == 0) ex[blockIdx.x] = exact ? kExactRow : e;
 }
 
 // ------------------------------------------------------------- decoders ---
