@@ -7,7 +7,7 @@ _Z = ctypes.c_size_t
 
 
 class SkinnyPlan(ctypes.Structure):
-    _fields_ = [("ks", ctypes.c_uint32), ("us", ctypes.c_double)]
+    _fields_ = [("ks", ctypes.c_uint32), ("nw", ctypes.c_uint32), ("us", ctypes.c_double)]
 
 
 class SplitPlan(ctypes.Structure):
@@ -31,6 +31,11 @@ def takes_split(zq, fmt, m, n, k, ws_bytes=None):
     skinny = _function(zq, "_ZN2zq20plan_gemm_skinny_f32Eimmmm", SkinnyPlan, ctypes.c_int, _Z, _Z, _Z, _Z)
     split = _function(zq, "_ZN2zq13gemm_split_usEimmmPKvm", ctypes.c_double, ctypes.c_int, _Z, _Z, _Z, ctypes.c_void_p, _Z)
     return skinny(fmt, m, n, k, use // (m * n * 4)).us > split(fmt, m, n, k, 256 if use else None, use)
+
+
+def skinny_waves(zq, fmt, m, n, k):
+    """Waves of the few-token kernel's workgroups, without a workspace (m > 32)."""
+    return _function(zq, "_ZN2zq20plan_gemm_skinny_f32Eimmmm", SkinnyPlan, ctypes.c_int, _Z, _Z, _Z, _Z)(fmt, m, n, k, 0).nw
 
 
 def split_bytes(zq, fmt, m, k):

@@ -13,7 +13,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from oracle import oracle as O
-from tests.plans import launch_split, split_bytes, split_plan, takes_split
+from tests.plans import launch_split, skinny_waves, split_bytes, split_plan, takes_split
 from tests.tolerance import assert_close
 
 ALL = (O.Q8_0, O.Q4_0, O.Q6_K, O.Q4_K, O.Q5_K)
@@ -261,6 +261,32 @@ def test_rows_marked_for_fp32(zq, orc, fmt):
     mag = np.abs(Xr) @ np.abs(W).T + (fmt in (O.Q4_K, O.Q5_K)) * (np.abs(Xr).sum(1)[:, None] * np.abs(W).max())
     err = np.abs(Y.cpu().numpy().reshape(m, n)[rows] - Xr @ W.T)
     assert np.all(err <= (8 + k ** 0.5) * 2.0 ** -24 * mag)
+
+
+# Short K and a large grid: workgroups of four and two waves, without a workspace;
+# and a batch with a small matrix that takes eight, whose bits are those of single
+# calls.
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,nw", [(1000, 4096, 256, 2), (130, 14300, 256, 4), (577, 4096, 1024, 4), (70, 14336, 512, 2)])
+@pytest.mark.parametrize("fmt", ALL)
+def test_fewer_waves(zq, orc, fmt, m, n, k, nw):
+    assert skinny_waves(zq, fmt, m, n, k) == nw and skinny_waves(zq, fmt, m, 33, k) == 8
+    rows = (33, n)
+    ws = [orc.gen_weights(fmt, 570 + i, r, k) for i, r in enumerate(rows)]
+    X = orc.gen_normal(571, m * k).reshape(m, k)
+    W = orc.dequantize(fmt, ws[1], n * k).reshape(n, k).astype(np.float64)
+    got = run_dev(zq, fmt, ws[1], X, m, n, k, 0)
+    assert_close(got.reshape(-1), (X.astype(np.float64) @ W.T).reshape(-1), f"fmt={fmt} {m}x{n}x{k}")
+    single = [run_dev(zq, fmt, w, X, m, r, k, zq.gemm_workspace_bytes(fmt, m, r, k, zq.ACT_F32)) for w, r in zip(ws, rows)]
+    ds = [torch.zeros(zq.weight_bytes(fmt, r, k), dtype=torch.uint8, device="cuda:0") for r in rows]
+    for d, w in zip(ds, ws):
+        d[: w.size] = torch.from_numpy(w).to("cuda:0")
+    Ys = [torch.empty(m * r, device="cuda:0") for r in rows]
+    need = zq.gemm_batch_workspace_bytes(fmt, rows, m, k, zq.ACT_F32)
+    buf = torch.empty(need + 16, dtype=torch.uint8, device="cuda:0")
+    zq.gemm_batch_dev(fmt, torch.from_numpy(X).to("cuda:0"), list(zip(ds, Ys, rows)), m, k, zq.ACT_F32, buf, need)
+    for Y, one in zip(Ys, single):
+        assert np.array_equal(Y.cpu().numpy(), one.reshape(-1))
 
 
 @pytest.mark.parametrize("src", ("zq_gemm_split.hip", "zq_gemm_skinny.hip"))

@@ -435,7 +435,7 @@ int enqueue_ffn_residual(int fmt, const uint8_t* wo, const uint8_t* wg, const ui
     // hidden 5120 / 13824: 61.9 -> 59.7 us.
     // Below that, with gate and up rows enough for the MFMA GEMV, whose form this
     // is not, they go there and SiLU * up in front of down: hidden 512 / ffn 16384
-    // 32.6 -> 20.6 us a call, 2048 / 16384 37.1 -> 31.6 (3072 43.4 -> 42.5).
+    // 31.8 -> 19.9 us a call, 2048 / 16384 36.5 -> 31.3, 3072 42.0 -> 41.5.
     bool paired = hidden >= 4096 || !zq::gemv_norm_on_mfma(fmt, hidden, 2 * ffn_rows);  // g holds silu(gate) * up
     hipError_t e = paired ? zq::launch_gemv_prologue_silu_pair(fmt, gu[0], gu[1], norm, hidden, s) : hipErrorInvalidConfiguration;
     if (e == hipErrorInvalidConfiguration) {

@@ -1140,11 +1140,11 @@ hipError_t launch_gemm_f32_batch(int fmt, const uint8_t* const* w, float* const*
             return hipErrorInvalidValue;
     // Each matrix's kernel and split depend on its own shape and workspace
     // alone, so a batch gives the bits of its single calls; those that the
-    // few-token kernel takes unsplit share one launch.
+    // few-token kernel takes unsplit, with the same waves, share one launch.
     const uint8_t* sw[kMaxTasks];
     float* sy[kMaxTasks];
     size_t sn[kMaxTasks], shared = 0;
-    uint32_t total = 0;
+    uint32_t snw[kMaxTasks], total = 0;
     for (size_t i = 0; i < count; ++i) {
         const size_t N = rows[i];
         // a workspace larger than the shape asks for changes nothing
@@ -1158,17 +1158,21 @@ hipError_t launch_gemm_f32_batch(int fmt, const uint8_t* const* w, float* const*
             total += n;
         } else if (sk.ks > 1) {
             if (const hipError_t e = launch_gemm_skinny_f32(fmt, &w[i], &Y[i], &rows[i], 1, X, static_cast<float*>(ws), sk.ks,
-                                                            M, K, stream);
+                                                            sk.nw, M, K, stream);
                 e != hipSuccess)
                 return e;
             total += 2;
         } else {
-            sw[shared] = w[i], sy[shared] = Y[i], sn[shared] = N;
-            ++shared;
+            size_t at = shared++;  // in the order of their workgroups' waves
+            for (; at && snw[at - 1] < sk.nw; --at)
+                sw[at] = sw[at - 1], sy[at] = sy[at - 1], sn[at] = sn[at - 1], snw[at] = snw[at - 1];
+            sw[at] = w[i], sy[at] = Y[i], sn[at] = N, snw[at] = sk.nw;
         }
     }
-    if (shared) {
-        if (const hipError_t e = launch_gemm_skinny_f32(fmt, sw, sy, sn, shared, X, nullptr, 1, M, K, stream); e != hipSuccess)
+    for (size_t i = 0, n; i < shared; i += n) {
+        for (n = 1; i + n < shared && snw[i + n] == snw[i];) ++n;
+        if (const hipError_t e = launch_gemm_skinny_f32(fmt, sw + i, sy + i, sn + i, n, X, nullptr, 1, snw[i], M, K, stream);
+            e != hipSuccess)
             return e;
         ++total;
     }

@@ -39,9 +39,9 @@ typedef uint32_t u4a2_t __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u4a4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef __bf16 b8_t __attribute__((ext_vector_type(8)));
 
-// Waves of a workgroup: 16 for one token tile, 8 for two (their registers)
-template <int MT>
-constexpr int kWaves = MT == 1 ? 16 : 8;
+// Waves of a workgroup: 16 for one token tile; for two (their registers) 8, or 4
+// or 2 where K is short and the grid large, so that a CU has 2 or 4 workgroups
+// and their starts and ends overlap (see plan_gemm_skinny_f32).
 
 // The weight matrices of one launch: task i's 32-row tiles start at tile[i].
 struct SkinnyTasks {
@@ -194,10 +194,9 @@ __device__ __forceinline__ void decode_group(const Group<FMT>& r, uint32_t b, ui
     w[1] = codes8(c[2], c[3], FMT == kQ8_0 || FMT == kQ4_0 ? flip & 0x80008000u : 0u);
 }
 
-template <int FMT, int MT>
-__global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_f32_kernel(SkinnyTasks tasks, const float* X, uint32_t M,
-                                                                           uint32_t K) {
-    constexpr int NW = kWaves<MT>;
+template <int FMT, int MT, int NW>
+__global__ __launch_bounds__(64 * NW, MT == 1 ? 4 : 2) void gemm_skinny_f32_kernel(SkinnyTasks tasks, const float* X, uint32_t M,
+                                                                                    uint32_t K) {
     // each wave's activations of one group, [MT * 32 rows][128 B], 16-byte units
     // XOR-swizzled by the row; the waves' sums at the end
     __shared__ __align__(16) float lds[NW][MT][16 * 64];
@@ -374,13 +373,13 @@ __global__ __launch_bounds__(64 * kWaves<MT>, MT == 1 ? 4 : 2) void gemm_skinny_
 }
 
 template <int FMT>
-hipError_t launch_skinny_fmt(const SkinnyTasks& t, const float* X, uint32_t ks, uint32_t M, uint32_t K, hipStream_t stream) {
-    const uint32_t grid = t.tile[t.count] * ks;
-    if (M <= 32)
-        hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 1>), dim3(grid), dim3(64 * kWaves<1>), 0, stream, t, X, M, K);
-    else
-        hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 2>), dim3(grid * ((M + 63) / 64)), dim3(64 * kWaves<2>), 0, stream, t,
-                           X, M, K);
+hipError_t launch_skinny_fmt(const SkinnyTasks& t, const float* X, uint32_t ks, uint32_t nw, uint32_t M, uint32_t K,
+                             hipStream_t stream) {
+    const dim3 grid(t.tile[t.count] * ks * (M <= 32 ? 1 : (M + 63) / 64));
+    if (M <= 32) hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 1, 16>), grid, dim3(1024), 0, stream, t, X, M, K);
+    else if (nw == 2) hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 2, 2>), grid, dim3(128), 0, stream, t, X, M, K);
+    else if (nw == 4) hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 2, 4>), grid, dim3(256), 0, stream, t, X, M, K);
+    else hipLaunchKernelGGL((gemm_skinny_f32_kernel<FMT, 2, 8>), grid, dim3(512), 0, stream, t, X, M, K);
     return hipGetLastError();
 }
 
@@ -403,14 +402,29 @@ SkinnyPlan plan_gemm_skinny_f32(int fmt, size_t M, size_t N, size_t K, size_t pl
     uint32_t ks = std::max(1u, std::min(most, (nb + 127) / 128));
     const uint32_t per = (nb + ks - 1) / ks;
     ks = (nb + per - 1) / per;  // no empty splits
-    const double rounds = double((wgs * ks + cus - 1) / cus);
-    double us = 3.0 + rounds * (per * group_us + 2.0);  // 2 us: a workgroup's start and its waves' sum
+    auto rounds = [&](uint32_t slots) { return double((wgs * ks + slots - 1) / slots); };
+    double us = 3.0 + rounds(cus) * (per * group_us + 2.0);  // 2 us: a workgroup's start and its waves' sum
+    // Fewer waves: two or four workgroups on a CU share its time, 15 % better, and
+    // one start and end (which 3 us describes better here).  1000 x 14336 x 256 of
+    // Q6_K 150 us with 8 waves, 81 with 4, 73 with 2; 1000 x 4096 x 1024 of Q8_0
+    // 71, 55, 63; a grid of one round loses: 64 x 4096 x 1024 11.7, 12.8, 18.8.
+    // Up to 32 groups, where the 128 x 128 tiles on the fp32 MFMA before this
+    // kernel had been up to 1.7x faster than 8 waves.
+    uint32_t nw = 8;
+    double best = 3.0 + rounds(cus) * (per * group_us + 3.0);
+    for (uint32_t n : {4u, 2u}) {
+        const uint32_t share = 8 / n;
+        const double t = 3.0 + rounds(cus * share) * (0.85 * share * per * group_us + 2.0);
+        if (wide && per <= 32 && t < best) best = t, nw = n;
+    }
+    if (nw < 8) us = std::min(us, best);
     if (ks > 1) us += 3.0 + double(ks - 1) * double(M) * double(N) * 8.0 / 4.0e6;
-    return SkinnyPlan{ks, us};
+    return SkinnyPlan{ks, nw, us};
 }
 
 hipError_t launch_gemm_skinny_f32(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
-                                  const float* X, float* partial, uint32_t ks, size_t M, size_t K, hipStream_t stream) {
+                                  const float* X, float* partial, uint32_t ks, uint32_t nw, size_t M, size_t K,
+                                  hipStream_t stream) {
     SkinnyTasks t{};
     t.count = int(count);
     for (size_t i = 0; i < count; ++i) {
@@ -424,11 +438,11 @@ hipError_t launch_gemm_skinny_f32(int fmt, const uint8_t* const* w, float* const
     t.groups = (nb + ks - 1) / ks;
     hipError_t e = hipErrorInvalidValue;
     switch (fmt) {
-    case kQ8_0: e = launch_skinny_fmt<kQ8_0>(t, X, ks, m, k, stream); break;
-    case kQ4_0: e = launch_skinny_fmt<kQ4_0>(t, X, ks, m, k, stream); break;
-    case kQ4_K: e = launch_skinny_fmt<kQ4_K>(t, X, ks, m, k, stream); break;
-    case kQ5_K: e = launch_skinny_fmt<kQ5_K>(t, X, ks, m, k, stream); break;
-    case kQ6_K: e = launch_skinny_fmt<kQ6_K>(t, X, ks, m, k, stream); break;
+    case kQ8_0: e = launch_skinny_fmt<kQ8_0>(t, X, ks, nw, m, k, stream); break;
+    case kQ4_0: e = launch_skinny_fmt<kQ4_0>(t, X, ks, nw, m, k, stream); break;
+    case kQ4_K: e = launch_skinny_fmt<kQ4_K>(t, X, ks, nw, m, k, stream); break;
+    case kQ5_K: e = launch_skinny_fmt<kQ5_K>(t, X, ks, nw, m, k, stream); break;
+    case kQ6_K: e = launch_skinny_fmt<kQ6_K>(t, X, ks, nw, m, k, stream); break;
     default: break;
     }
     return e != hipSuccess || ks <= 1 ? e : launch_splitk_add(partial, Y[0], M, rows[0], ks - 1, stream);

@@ -925,10 +925,12 @@ static size_t tokens_that_fit(int fmt, size_t M, size_t K, size_t ws_bytes) {
     return t;
 }
 // The rest of the tokens after such a part: by the cheaper kernel, unsplit.
-static bool rest_on_skinny(int fmt, size_t rest, size_t N, size_t K, const void* ws, size_t ws_bytes, double& us) {
-    const double a = plan_gemm_skinny_f32(fmt, rest, N, K, 0).us, b = gemm_split_us(fmt, rest, N, K, ws, ws_bytes);
-    us = std::min(a, b);
-    return a <= b;
+static bool rest_on_skinny(int fmt, size_t rest, size_t N, size_t K, const void* ws, size_t ws_bytes, SkinnyPlan& p) {
+    p = plan_gemm_skinny_f32(fmt, rest, N, K, 0);
+    const double us = gemm_split_us(fmt, rest, N, K, ws, ws_bytes);
+    if (p.us <= us) return true;
+    p.us = us;
+    return false;
 }
 
 double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size_t ws_bytes) {
@@ -938,9 +940,9 @@ double gemm_split_us(int fmt, size_t M, size_t N, size_t K, const void* ws, size
         // (Q4_K / Q5_K at the asked-for size, which has no room for the group
         // sums: 97 of 100 tokens fit; less than half is not worth it)
         if (fit < (M + 1) / 2) return 1e300;
-        double rest;
+        SkinnyPlan rest;
         (void)rest_on_skinny(fmt, M - fit, N, K, ws, ws_bytes, rest);
-        return gemm_split_us(fmt, fit, N, K, ws, ws_bytes) + rest;
+        return gemm_split_us(fmt, fit, N, K, ws, ws_bytes) + rest.us;
     }
     // beside the GEMM: two launches and the activations read and written once
     return 8.0 + double(M) * double(K) * 8.0 / 4.0e6 +
@@ -958,10 +960,10 @@ hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y
         if (const hipError_t e = launch_gemm_split(fmt, w, X, Y, ws, ws_bytes, fit, N, K, stream, &n); e != hipSuccess) return e;
         const float* rx = X + fit * K;
         float* ry = Y + fit * N;
-        double us;
+        SkinnyPlan p;
         const hipError_t e =
-            rest_on_skinny(fmt, M - fit, N, K, ws, ws_bytes, us)
-                ? launch_gemm_skinny_f32(fmt, &w, &ry, &N, 1, rx, nullptr, 1, M - fit, K, stream)
+            rest_on_skinny(fmt, M - fit, N, K, ws, ws_bytes, p)
+                ? launch_gemm_skinny_f32(fmt, &w, &ry, &N, 1, rx, nullptr, 1, p.nw, M - fit, K, stream)
                 : launch_gemm_split(fmt, w, rx, ry, ws, ws_bytes, M - fit, N, K, stream, &rest_n);
         if (launches) *launches = n + rest_n;
         return e;

@@ -159,11 +159,13 @@ hipError_t launch_gemm_split(int fmt, const uint8_t* w, const float* X, float* Y
 // one matrix, its partial planes, and a second launch that adds them).
 struct SkinnyPlan {
     uint32_t ks;
+    uint32_t nw;  // waves of a workgroup that takes 64 tokens: 8, 4 or 2
     double us;
 };
 SkinnyPlan plan_gemm_skinny_f32(int fmt, size_t M, size_t N, size_t K, size_t planes);
 hipError_t launch_gemm_skinny_f32(int fmt, const uint8_t* const* w, float* const* Y, const size_t* rows, size_t count,
-                                  const float* X, float* partial, uint32_t ks, size_t M, size_t K, hipStream_t stream);
+                                  const float* X, float* partial, uint32_t ks, uint32_t nw, size_t M, size_t K,
+                                  hipStream_t stream);
 
 // Bit-exact tier helpers.
 hipError_t launch_dequantize(int fmt, const uint8_t* w, float* out, size_t rows, size_t cols,
