@@ -85,6 +85,8 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
     for (int w = 1; w < kThreads / 64; ++w) m = fmaxf(m, red[w]);
     const int e = m > 0.0f ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
     float lost = 0.0f;  // non-zero elements more than 2^20 below the maximum, 1e9 for an infinity
+    float low = 0.0f;   // squares of those more than 2^8 below it, as far as looked at
+    auto add_low = [&](float f) { low = fabsf(f) < 0x1p6f ? fmaf(f, f, low) : low; };
     _Float16* o = out + size_t(blockIdx.x) * K * 2;
     auto split = [](float f, _Float16& h, _Float16& l) {
         h = _Float16(f);
@@ -109,6 +111,7 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
             for (int k = 0; k < 4; ++k) {
                 const float t = fabsf(f[k]);
                 lost += t == __builtin_inff() ? 1e9f : t != 0.0f && t < 0x1p-6f ? 1.0f : 0.0f;
+                add_low(f[k]);
             }
         }
         _Float16* d = o + size_t(i >> 3) * 64 + (i & 7u) * 4;
@@ -134,13 +137,15 @@ __global__ __launch_bounds__(kThreads) void split_acts_kernel(const float* __res
     };
     lost = block_sum(lost);  // whole numbers below 2^24, or past 2^28
     bool exact = lost >= 1e9f;
-    if (lost > 0.0f && !exact) {
-        float low = 0.0f;
+    // the neighbours of the few lost elements of an ordinary row are enough
+    if (lost > 0.0f && !exact && block_sum(low) < 0.0625f * lost) {
+        low = 0.0f;
         for (uint32_t i = threadIdx.x; i < K4; i += kThreads) {
             const float4 v = r[i];
-            const float f[4] = {ldexpf(v.x, e), ldexpf(v.y, e), ldexpf(v.z, e), ldexpf(v.w, e)};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) low = fabsf(f[k]) < 0x1p6f ? fmaf(f[k], f[k], low) : low;
+            add_low(ldexpf(v.x, e));
+            add_low(ldexpf(v.y, e));
+            add_low(ldexpf(v.z, e));
+            add_low(ldexpf(v.w, e));
         }
         exact = block_sum(low) < 0.0625f * lost;
     }
