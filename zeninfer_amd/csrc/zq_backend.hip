@@ -430,7 +430,7 @@ int enqueue_ffn_residual(int fmt, const uint8_t* wo, const uint8_t* wg, const ui
     // epilogue where both fit (Q8_0 / Q4_0 up to 4096 columns), so that the down
     // GEMV is a plain one and not one whose every workgroup recomputes SiLU * up.
     // With the residual add in the down GEMV's store, Q8_0 with hidden 4096: ffn
-    // 14336 45.2 -> 42.2 us a call, ffn 4096 23.5 -> 21.7; 512 / 1024, bound by
+    // 14336 45.2 -> 42.6 us a call, ffn 4096 23.5 -> 21.7; 512 / 1024, bound by
     // its launches, 22.2 -> 14.0 (three instead of four).  The add alone, with
     // hidden 5120 / 13824: 61.9 -> 59.7 us.
     // Below that, with gate and up rows enough for the MFMA GEMV, whose form this
